@@ -32,7 +32,10 @@
 // are one coalesced 256-byte row.  Per-stream tables (histogram, code table,
 // decode table) live in LDS as [symbol][lane] so every lane works in its own
 // column without bank conflicts or barriers.
+#include <algorithm>
+#include <mutex>
 #include <type_traits>
+#include <vector>
 #include "common.h"
 #include "cachegen_decode.h"
 #include "cachegen_gw.h"
@@ -107,6 +110,27 @@ __device__ __forceinline__ void unpack_row(const int16_t *row, int nb,
   }
 }
 
+// Inclusive prefix sum over the 64 lanes of a wave with DPP moves: shifts
+// by 1, 2, 4 and 8 within each row of 16 lanes, then the last lane of row
+// 0 (row_bcast:15) and of row 1 (row_bcast:31) added to the rows after it.
+__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
+  int x = static_cast<int>(v);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, true);  // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, true);  // row_shr:2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, true);  // row_shr:4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, true);  // row_shr:8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false); // row_bcast:15 to rows 1, 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false); // row_bcast:31 to rows 2, 3
+  return static_cast<uint32_t>(x);
+}
+
+// Address of stream s's symbol of token 0 (streams are numbered over the
+// layers, channels fastest; a layer's symbols are [T, C]).
+__device__ __forceinline__ const uint8_t *stream_column(const uint8_t *in, int64_t s, int T, int C) {
+  const int64_t l = s / C;
+  return in + l * T * C + (s - l * C);
+}
+
 // calculate_cdf: 64 streams per block, four waves.  The block's symbols are
 // staged into LDS 256 tokens at a time ([tokens][64] u8, 16-byte loads); wave
 // q counts the q-th quarter of each staged piece into per-stream LDS
@@ -125,7 +149,12 @@ __device__ __forceinline__ void unpack_row(const int16_t *row, int nb,
 // makes the serial aligned assignment of the other streams (the width of
 // each interval capped by the lowest set bit of the running base, after the
 // Kraft repair).  The block's 64 rows, contiguous in the output, leave as
-// coalesced dword stores.
+// coalesced dword stores.  Blocks take 64 consecutive streams whatever their
+// layer, so no block is partly filled but the last.  With `lens` the streams'
+// lengths in bytes under these rows are written too (the sum of count times
+// code length, from the counts already in registers), and per block the sum
+// of the lengths cut to `cap`, so a caller knows every stream's place before
+// anything has been encoded.
 constexpr int kCdfWaves = 4;
 constexpr int kCdfThreads = 64 * kCdfWaves;
 constexpr int kCdfPiece = 256;  // tokens staged at a time
@@ -234,7 +263,8 @@ __device__ __forceinline__ void gw_lengths(uint32_t *hist, uint32_t *lists, uint
 template <int kBins, bool kExact>
 __global__ void __launch_bounds__(kCdfThreads)
     cdf_tile_kernel(const uint8_t *__restrict__ in, int T, int C, int nb,
-                    int16_t *__restrict__ out, int tiles, int vec_tile) {
+                    int16_t *__restrict__ out, int64_t n_streams, int vec_tile,
+                    int32_t *__restrict__ lens, int64_t *__restrict__ sums, int64_t cap) {
   // Wave priority: 1, and 0 for a wave making the one-lane Garsia-Wachs
   // steps.  A step wave issues VALU almost every cycle and the SIMD arbiter
   // prefers the oldest wave among equals: with every wave at one priority,
@@ -254,9 +284,14 @@ __global__ void __launch_bounds__(kCdfThreads)
   // symbol share, the wave that runs the one-lane steps) is then uniform.
   const int q = __builtin_amdgcn_readfirstlane(tid / 64);
   const int lane = tid % 64;
-  const int l = blockIdx.x / tiles;
-  const int c0 = (blockIdx.x % tiles) * 64;
-  const int cnt = C - c0 < 64 ? C - c0 : 64;
+  const int64_t s0 = static_cast<int64_t>(blockIdx.x) * 64;
+  const int cnt = n_streams - s0 < 64 ? static_cast<int>(n_streams - s0) : 64;
+  // The stream column this thread stages: its 16-byte piece of every token
+  // row (vec_tile), or its lane's byte.  A piece lies in one layer (C % 16
+  // == 0 with vec_tile).
+  const int col = vec_tile ? 16 * (tid & 3) : lane;
+  const bool col_on = col < cnt;
+  const uint8_t *col_src = stream_column(in, s0 + (col_on ? col : 0), T, C);
   uint8_t *tile = reinterpret_cast<uint8_t *>(lds);
   uint32_t *hist = lds + cdf_stage_words(T, nb);
   uint32_t *psum = hist + nb * 64;          // [wave][stream]: partial interval sums
@@ -269,25 +304,23 @@ __global__ void __launch_bounds__(kCdfThreads)
   for (int t0 = 0; t0 < T; t0 += kCdfPiece) {
     const int tc = T - t0 < kCdfPiece ? T - t0 : kCdfPiece;
     if (t0 > 0) __syncthreads();  // the previous piece has been counted
-    const uint8_t *src = in + (static_cast<int64_t>(l) * T + t0) * C + c0;
-    const int pieces = tc * 4;
-    if (vec_tile && cnt == 64) {
+    const uint8_t *src = col_src + static_cast<int64_t>(t0) * C;
+    if (vec_tile) {
       typedef unsigned int w4 __attribute__((ext_vector_type(4)));
-      w4 v[4];
-      int pi[4];
+      if (col_on) {
+        w4 v[4];
+        int t[4];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const int i = k * kCdfThreads + tid;
-        pi[k] = i < pieces ? i : pieces - 1;
-        v[k] = gload(reinterpret_cast<const w4 *>(src + static_cast<int64_t>(pi[k] >> 2) * C + (pi[k] & 3) * 16));
-      }
+        for (int k = 0; k < 4; ++k) {
+          t[k] = k * (kCdfThreads / 4) + (tid >> 2);
+          t[k] = t[k] < tc ? t[k] : tc - 1;
+          v[k] = gload(reinterpret_cast<const w4 *>(src + static_cast<int64_t>(t[k]) * C));
+        }
 #pragma unroll
-      for (int k = 0; k < 4; ++k) reinterpret_cast<w4 *>(tile)[pi[k]] = v[k];
-    } else {
-      for (int i = tid; i < tc * 64; i += kCdfThreads) {
-        const int c = i % 64;
-        tile[i] = c < cnt ? src[static_cast<int64_t>(i / 64) * C + c] : 0xFFu;
+        for (int k = 0; k < 4; ++k) reinterpret_cast<w4 *>(tile)[t[k] * 4 + (tid & 3)] = v[k];
       }
+    } else if (col_on) {
+      for (int t = q; t < tc; t += kCdfWaves) tile[t * 64 + lane] = src[static_cast<int64_t>(t) * C];
     }
     __syncthreads();
     const int Tq = (tc + kCdfWaves - 1) / kCdfWaves;
@@ -435,6 +468,15 @@ __global__ void __launch_bounds__(kCdfThreads)
       if (in_range) hist[s * 64 + lane] = (xl << kLenShift) | cs;
     }
     psum[q * 64 + lane] = own;
+    // The wave's share of the stream's length in bits, in list rows that
+    // hold no depths (16 on): the lists are dead.
+    if (lens != nullptr) {
+      uint32_t nbits = 0;
+#pragma unroll
+      for (int k = 0; k < kS; ++k)
+        if (kExact || (k < share && j0 + k < j1)) nbits += len[k] * cv[k];
+      lds[(16 + q) * 64 + lane] = nbits;
+    }
     __syncthreads();
     int16_t *row = rows + lane * (nb + 1);
     if (gw) {
@@ -491,6 +533,7 @@ __global__ void __launch_bounds__(kCdfThreads)
     // taken is min(2^(16 - length), that bit), and the length follows from
     // it.  The chain from one symbol to the next is four operations.
     uint32_t r = 1u << kPrec;
+    uint32_t nbits = 0;
 #pragma unroll
     for (int s = 0; s < kBins; ++s) {
       if (s < nb) {
@@ -500,12 +543,32 @@ __global__ void __launch_bounds__(kCdfThreads)
         const uint32_t x = x0 ? static_cast<uint32_t>(__builtin_clz(w)) - (31u - kPrec) : 0u;
         row[s] = static_cast<int16_t>(static_cast<uint16_t>((r | x) & 0xFFFFu));
         r += w;
+        if (lens != nullptr) nbits += x * (wcol[s * 64] & kCountMask);
       }
+    }
+    // In place of the waves' shares.
+    if (lens != nullptr) {
+#pragma unroll
+      for (int w = 0; w < kCdfWaves; ++w) lds[(16 + w) * 64 + lane] = w == 0 ? nbits : 0u;
     }
   }
   __syncthreads();
+  // Stream lengths in bytes, and the block's bytes once every stream is cut
+  // to cap.
+  if (lens != nullptr && q == 0) {
+    uint32_t nbits = 0;
+#pragma unroll
+    for (int w = 0; w < kCdfWaves; ++w) nbits += lds[(16 + w) * 64 + lane];
+    const uint32_t nbytes = lane < cnt ? (nbits + 7) >> 3 : 0u;
+    if (lane < cnt) lens[s0 + lane] = static_cast<int32_t>(nbytes);
+    const uint32_t kept = static_cast<int64_t>(nbytes) < cap ? nbytes : static_cast<uint32_t>(cap);
+    // A stream has at most 2^26 codes of 12 bits, so the sum of 64 fits only
+    // 64 bits: two scans, of the low and high halves.
+    const uint32_t lo = wave_incl_scan(kept & 0xFFFFu), hi = wave_incl_scan(kept >> 16);
+    if (lane == 63) sums[blockIdx.x] = (static_cast<int64_t>(hi) << 16) + lo;
+  }
   // The block's rows are contiguous in the output.
-  int16_t *dst = out + (static_cast<int64_t>(l) * C + c0) * (nb + 1);
+  int16_t *dst = out + s0 * (nb + 1);
   const int total = cnt * (nb + 1);
   if ((reinterpret_cast<uintptr_t>(dst) & 3) == 0) {
     for (int i = tid; i < total / 2; i += kCdfThreads)
@@ -627,20 +690,6 @@ __device__ __forceinline__ void put_word(uint8_t *row, int64_t chunk, uint32_t i
     cg_st(reinterpret_cast<uint32_t *>(row + at), __builtin_bswap32(word));
   else
     put_bytes(row, chunk, at, word, n);
-}
-
-// Inclusive prefix sum over the 64 lanes of a wave with DPP moves: shifts
-// by 1, 2, 4 and 8 within each row of 16 lanes, then the last lane of row
-// 0 (row_bcast:15) and of row 1 (row_bcast:31) added to the rows after it.
-__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
-  int x = static_cast<int>(v);
-  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, true);  // row_shr:1
-  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, true);  // row_shr:2
-  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, true);  // row_shr:4
-  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, true);  // row_shr:8
-  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false); // row_bcast:15 to rows 1, 3
-  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false); // row_bcast:31 to rows 2, 3
-  return static_cast<uint32_t>(x);
 }
 
 // Encode staging: the block's CDF rows (contiguous in memory) into `stage`
@@ -1696,6 +1745,197 @@ __global__ void __launch_bounds__(kDecLanes)
   decode_one_wave<Tab>(lds, cdf, bytes, nbytes, prefix, T, C, nb, out, tiles, lane);
 }
 
+// Exclusive prefix sums of the blocks' byte counts, in one workgroup: off[b]
+// for block b, off[n] and *total the sum.  `sums` and `off` may not overlap.
+// One workgroup: 1024 blocks (65536 streams) take 4.1 us, of which most is
+// the launch, under which nothing else has to wait but the encoder.
+constexpr int kOffThreads = 1024;
+__global__ void __launch_bounds__(kOffThreads)
+    stream_offsets_kernel(const int64_t *__restrict__ sums, int64_t n, int64_t *__restrict__ off,
+                          int64_t *total) {
+  __shared__ int64_t wave_sum[kOffThreads / 64];
+  const int lane = static_cast<int>(threadIdx.x) & 63;
+  const int wave = static_cast<int>(threadIdx.x) >> 6;
+  int64_t carry = 0;
+  for (int64_t i0 = 0; i0 < n; i0 += kOffThreads) {
+    const int64_t i = i0 + threadIdx.x;
+    const int64_t own = i < n ? sums[i] : 0;
+    int64_t incl = own;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int64_t v = __shfl_up(incl, d, 64);
+      incl += lane >= d ? v : 0;
+    }
+    if (lane == 63) wave_sum[wave] = incl;
+    __syncthreads();
+    int64_t before = 0, all = 0;
+#pragma unroll
+    for (int w = 0; w < kOffThreads / 64; ++w) {
+      before += w < wave ? wave_sum[w] : 0;
+      all += wave_sum[w];
+    }
+    if (i < n) off[i] = carry + before + incl - own;
+    carry += all;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    off[n] = carry;
+    *total = carry;
+  }
+}
+
+// Concatenates the used bytes of the streams' rows ([n_streams, cap], stream
+// s using min(lens[s], cap)): 64 streams per block, whose bytes start at
+// off[block] of `out`.  Half a wave copies a stream, kPackU of its
+// destination dwords in flight per lane; a destination dword inside the
+// stream takes two source dwords of the row and one align, and the bytes of
+// the dwords shared with the streams before and after are stored one by one.
+// Every source dword read holds a byte of the stream's own row.  Measured on
+// MI355X (64 planes x 256 tokens x 1024 channels, 7.3 MB of streams): 11.5 us,
+// in place of about 330 us for a boolean mask over the rows and a masked
+// select (a mask, its count, a partition and an index pass over every byte of
+// the rows' capacity); the whole chunk 408 -> 54 us.
+constexpr int kPackThreads = 512;
+constexpr int kPackHalves = kPackThreads / 32;
+constexpr int kPackU = 64 / kPackHalves;  // streams per half wave
+__global__ void __launch_bounds__(kPackThreads)
+    pack_streams_kernel(const uint8_t *__restrict__ rows, int64_t cap, const int32_t *__restrict__ lens,
+                        int64_t n_streams, const int64_t *__restrict__ off, uint8_t *__restrict__ out) {
+  __shared__ int64_t start[64];
+  __shared__ uint32_t size[64];
+  const int tid = static_cast<int>(threadIdx.x);
+  const int64_t s0 = static_cast<int64_t>(blockIdx.x) * 64;
+  if (tid < 64) {
+    const int64_t len = s0 + tid < n_streams ? lens[s0 + tid] : 0;
+    const uint32_t kept = static_cast<uint32_t>(len < cap ? len : cap);
+    const uint32_t lo = wave_incl_scan(kept & 0xFFFFu), hi = wave_incl_scan(kept >> 16);
+    start[tid] = off[blockIdx.x] + (static_cast<int64_t>(hi) << 16) + lo - kept;
+    size[tid] = kept;
+  }
+  __syncthreads();
+  const int half = tid >> 5, hl = tid & 31;
+  const uint8_t *src[kPackU];
+  uint8_t *dst[kPackU];
+  uint32_t n[kPackU], longest = 0;
+#pragma unroll
+  for (int u = 0; u < kPackU; ++u) {
+    const int st = u * kPackHalves + half;
+    src[u] = rows + (s0 + st) * cap;
+    dst[u] = out + start[st];
+    n[u] = size[st];
+    longest = max(longest, n[u]);
+  }
+  // Dword k of a stream is the aligned destination dword at dst - lead + 4k.
+  for (uint32_t k0 = 0; 4 * k0 < longest + 3; k0 += 32) {
+    uint32_t w[kPackU];
+    int64_t at[kPackU];  // stream byte at the dword's first byte
+#pragma unroll
+    for (int u = 0; u < kPackU; ++u) {
+      at[u] = static_cast<int64_t>(4) * (k0 + hl) - static_cast<int64_t>(reinterpret_cast<uintptr_t>(dst[u]) & 3);
+      const int64_t end = n[u];
+      w[u] = 0;
+      if (at[u] < end && n[u] != 0) {
+        // The aligned source dwords holding bytes at .. at + 3, each read
+        // only if it holds a byte of [0, n).
+        const uint8_t *p = src[u] + at[u];
+        const uint32_t sh = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(p) & 3);
+        const uint32_t *a = reinterpret_cast<const uint32_t *>(p - sh);
+        const int64_t lo_at = at[u] - sh;  // stream byte at a[0]
+        const uint32_t x = lo_at + 4 > 0 ? gload(a) : 0u;
+        const uint32_t y = sh != 0 && lo_at + 4 < end ? gload(a + 1) : 0u;
+        w[u] = __builtin_amdgcn_alignbyte(y, x, sh);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kPackU; ++u) {
+      const int64_t end = n[u];
+      if (at[u] >= 0 && at[u] + 4 <= end) {
+        gstore(reinterpret_cast<uint32_t *>(dst[u] + at[u]), w[u]);
+      } else if (at[u] < end) {
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+          if (at[u] + b >= 0 && at[u] + b < end) dst[u][at[u] + b] = static_cast<uint8_t>(w[u] >> (8 * b));
+      }
+    }
+  }
+}
+
+// What a call that waits for a device value needs: an event and a word of
+// pinned host memory.  Taken from a pool per call and given back once the
+// event has completed; the pool keeps at most kKept of them.
+class HostWord {
+public:
+  explicit HostWord(int device) {
+    {
+      std::lock_guard<std::mutex> g(mu());
+      auto &p = pool();
+      for (size_t i = 0; i < p.size(); ++i)
+        if (p[i].device == device) {
+          s_ = p[i];
+          p.erase(p.begin() + static_cast<std::ptrdiff_t>(i));
+          return;
+        }
+    }
+    s_.device = device;
+    hip_check(hipEventCreateWithFlags(&s_.event, hipEventDisableTiming), "hipEventCreate");
+    const hipError_t e = hipHostMalloc(reinterpret_cast<void **>(&s_.word), sizeof(int64_t),
+                                       hipHostMallocMapped | hipHostMallocPortable);
+    if (e != hipSuccess) {
+      (void)hipEventDestroy(s_.event);
+      hip_check(e, "hipHostMalloc");
+    }
+  }
+  HostWord(const HostWord &) = delete;
+  HostWord &operator=(const HostWord &) = delete;
+  // The kernel that writes the word has to be over before it is given back:
+  // wait() sees to that, and a call that fails after its launch waits for
+  // the stream here.
+  ~HostWord() {
+    if (pending_) (void)hipStreamSynchronize(stream_);
+    {
+      std::lock_guard<std::mutex> g(mu());
+      if (pool().size() < kKept) {
+        pool().push_back(s_);
+        return;
+      }
+    }
+    (void)hipEventDestroy(s_.event);
+    (void)hipHostFree(s_.word);
+  }
+  int64_t *word() const { return s_.word; }
+  // Call before the launch of the kernel that writes the word, then record()
+  // after it.
+  void launching(hipStream_t stream) {
+    stream_ = stream;
+    pending_ = true;
+  }
+  void record() { hip_check(hipEventRecord(s_.event, stream_), "hipEventRecord"); }
+  int64_t wait() {
+    hip_check(hipEventSynchronize(s_.event), "hipEventSynchronize");
+    pending_ = false;
+    return *static_cast<volatile int64_t *>(s_.word);
+  }
+
+private:
+  struct Slot {
+    int device = 0;
+    hipEvent_t event = nullptr;
+    int64_t *word = nullptr;
+  };
+  static constexpr size_t kKept = 16;
+  static std::mutex &mu() {
+    static std::mutex m;
+    return m;
+  }
+  static std::vector<Slot> &pool() {
+    static std::vector<Slot> *p = new std::vector<Slot>();  // outlives the runtime's own teardown
+    return *p;
+  }
+  Slot s_;
+  hipStream_t stream_ = nullptr;
+  bool pending_ = false;
+};
+
 // Row-major contiguity; a tensor without elements has no layout to check.
 bool contiguous(const lmc_tensor &t) {
   if (numel(t) == 0) return true;
@@ -1712,6 +1952,121 @@ void need_device(const lmc_tensor &t, const char *what) {
   check(contiguous(t), std::string(what) + " must be contiguous");
 }
 
+// calculate_cdf (csrc/cachegen_kernels.cpp:119-155), with the streams'
+// lengths and the 64-stream blocks' bytes when `lens` is given (see
+// cdf_tile_kernel).
+void make_cdf(const lmc_tensor &in, int32_t n_bins, const lmc_tensor &o, int32_t *lens, int64_t *sums, int64_t cap,
+              hipStream_t stream) {
+  need_device(in, "input");
+  need_device(o, "output");
+  check(in.ndim == 3, "input must be [layers, tokens, channels]");
+  check(in.dtype == LMC_U8 || in.dtype == LMC_I8, "input must be uint8/int8");
+  check(o.dtype == LMC_I16, "output must be int16");
+  check(n_bins >= 1 && n_bins <= kMaxBins,
+        "n_bins must be in [1, " + std::to_string(kMaxBins) + "]");
+  const int64_t L = in.sizes[0], T = in.sizes[1], C = in.sizes[2];
+  check(o.ndim == 3 && o.sizes[0] == L && o.sizes[1] == C &&
+            o.sizes[2] == n_bins + 1,
+        "output must be [layers, channels, n_bins + 1]");
+  check(T < (int64_t(1) << 26) && C < (int64_t(1) << 30), "input too large");
+  if (L == 0 || C == 0) return;
+  DeviceGuard guard(in.device);
+  const int64_t n_streams = L * C;
+  const int64_t blocks = (n_streams + 63) / 64;
+  check(blocks < (int64_t(1) << 31), "too many streams");
+  const size_t lds = static_cast<size_t>(cdf_lds_bytes(static_cast<int>(T), n_bins));
+  const int vec_tile = (C % 16 == 0 && (reinterpret_cast<uintptr_t>(in.data) & 15) == 0) ? 1 : 0;
+  const auto kern = n_bins == 32         ? cdf_tile_kernel<32, true>
+                    : n_bins < 32        ? cdf_tile_kernel<32, false>
+                    : n_bins == kMaxBins ? cdf_tile_kernel<kMaxBins, true>
+                                         : cdf_tile_kernel<kMaxBins, false>;
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(kCdfThreads), lds, stream,
+                     static_cast<const uint8_t *>(in.data), (int)T, (int)C, n_bins,
+                     static_cast<int16_t *>(o.data), n_streams, vec_tile, lens, sums, cap);
+  hip_check(hipGetLastError(), "cdf_tile_kernel launch");
+}
+
+// encode_fast_new (csrc/cachegen_kernels.cpp:17-58).
+void encode_rows(const lmc_tensor &cdf, const lmc_tensor &in, const lmc_tensor &ob, const lmc_tensor &ol,
+                 hipStream_t stream) {
+  need_device(cdf, "cdf");
+  need_device(in, "input_sym");
+  need_device(ob, "output_buffer");
+  need_device(ol, "output_lengths");
+  check(in.ndim == 3 && cdf.ndim == 3 && ob.ndim == 3,
+        "cdf, input_sym and output_buffer must be 3-D");
+  const int64_t L = in.sizes[0], T = in.sizes[1], C = in.sizes[2];
+  const int64_t nb = cdf.sizes[2] - 1;
+  const int64_t chunk = ob.sizes[2];
+  // csrc/cachegen_kernels.cpp:33-35
+  check(C <= (1 << 15),
+        "encode takes at most 32768 channels per layer");
+  check(in.dtype == LMC_U8 || in.dtype == LMC_I8, "input_sym must be int8/uint8");
+  check(cdf.dtype == LMC_I16, "cdf must be int16");
+  check(ob.dtype == LMC_U8 || ob.dtype == LMC_I8, "output_buffer must be uint8");
+  check(ol.dtype == LMC_I32 && numel(ol) == L * C, "output_lengths must be int32 [L, C]");
+  check(nb >= 1 && nb <= kMaxBins, "number of bins must be in [1, 64]");
+  check(cdf.sizes[0] == L && cdf.sizes[1] == C, "cdf must be [L, C, nbins + 1]");
+  check(ob.sizes[0] == L && ob.sizes[1] == C, "output_buffer must be [L, C, chunk]");
+  if (L == 0 || C == 0) return;
+  DeviceGuard guard(in.device);
+  const int tiles = static_cast<int>((C + kEncLanes - 1) / kEncLanes);
+  const int word_stores =
+      (chunk % 4 == 0 && (reinterpret_cast<uintptr_t>(ob.data) & 3) == 0) ? 1 : 0;
+  const int vec_in = (C % 16 == 0 && (reinterpret_cast<uintptr_t>(in.data) & 15) == 0) ? 1 : 0;
+  const bool rows_dw = (reinterpret_cast<uintptr_t>(cdf.data) & 3) == 0;
+  if (LMC_ENC_SPLIT && T > 0 && T <= kEncTileMaxT && nb <= kEncLanes && C % kEncLanes == 0 && vec_in &&
+      rows_dw) {
+    // Split encoder: bit rows of 2T bytes plus one word (codes are at
+    // most 16 bits), an odd number of words so that the lanes' rows start
+    // in different banks.
+    const int row_words = (static_cast<int>(T + 1) / 2 + 1) | 1;
+    const int rows_words = static_cast<int>(((nb + 1) * kEncLanes * 2 + 15) / 16 * 4);
+    const int phase1 = rows_words + kEncTileMaxT * kEncLanes / 4 + static_cast<int>(nb + 1) * kEncLanes;
+    const int stage_words = std::max(phase1, kEncLanes * row_words);
+    const size_t lds = 4 * (static_cast<size_t>((stage_words + kEncPieces * kEncLanes + 2) & ~1) + 2 * kEncLanes);
+    check(lds <= 65536, "encode: LDS budget exceeded");
+    hipLaunchKernelGGL(encode_split_kernel<kEncPieces>, dim3(L * tiles), dim3(64 * kEncPieces), lds,
+                       stream,
+                       static_cast<const int16_t *>(cdf.data),
+                       static_cast<const uint8_t *>(in.data), (int)T, (int)C,
+                       (int)nb, static_cast<uint8_t *>(ob.data), chunk,
+                       static_cast<int32_t *>(ol.data), tiles, word_stores, row_words, stage_words);
+    hip_check(hipGetLastError(), "encode_split_kernel launch");
+    return;
+  }
+  if (T > 0 && T <= kEncTileMaxT && nb <= kEncLanes) {
+    // Bits past min(chunk, 2 bytes per symbol) are never written (codes
+    // are at most 16 bits), so a wave's bit buffer holds that many bytes.
+    const int64_t cap_bytes = std::min<int64_t>(chunk, 2 * T);
+    const int cap_words = static_cast<int>((cap_bytes + 3) / 4);
+    const int sym_stride = (((T + 3) / 4) + 1) | 1;
+    const size_t lds = 4 * ((static_cast<size_t>(nb + 1) * kEncLanes * 2 + 15) / 16 * 4 +
+                            static_cast<size_t>(kEncLanes) * sym_stride +
+                            static_cast<size_t>(2 * kEncWaves) * cap_words);
+    const int vec_tile = vec_in;
+    check(lds <= 65536, "encode: LDS budget exceeded");
+    hipLaunchKernelGGL(encode_wave_kernel, dim3(L * tiles), dim3(kEncTileThreads), lds,
+                       stream,
+                       static_cast<const int16_t *>(cdf.data),
+                       static_cast<const uint8_t *>(in.data), (int)T, (int)C,
+                       (int)nb, static_cast<uint8_t *>(ob.data), chunk,
+                       static_cast<int32_t *>(ol.data), tiles, word_stores, vec_tile, sym_stride,
+                       cap_words);
+    hip_check(hipGetLastError(), "encode_wave_kernel launch");
+    return;
+  }
+  const size_t lds = static_cast<size_t>(nb) * kEncLanes * 4 +
+                     static_cast<size_t>(nb + 1) * kEncLanes * 2;
+  hipLaunchKernelGGL(encode_kernel, dim3(L * tiles), dim3(kEncLanes), lds,
+                     stream,
+                     static_cast<const int16_t *>(cdf.data),
+                     static_cast<const uint8_t *>(in.data), (int)T, (int)C,
+                     (int)nb, static_cast<uint8_t *>(ob.data), chunk,
+                     static_cast<int32_t *>(ol.data), tiles, word_stores);
+  hip_check(hipGetLastError(), "encode_kernel launch");
+}
+
 } // namespace
 
 } // namespace lmc
@@ -1723,33 +2078,8 @@ extern "C" {
 int lmc_calculate_cdf(const lmc_tensor *input, int32_t n_bins,
                       const lmc_tensor *output, void *stream) {
   return guarded([&] {
-    const lmc_tensor &in = deref(input, "input");
-    const lmc_tensor &o = deref(output, "output");
-    need_device(in, "input");
-    need_device(o, "output");
-    check(in.ndim == 3, "input must be [layers, tokens, channels]");
-    check(in.dtype == LMC_U8 || in.dtype == LMC_I8, "input must be uint8/int8");
-    check(o.dtype == LMC_I16, "output must be int16");
-    check(n_bins >= 1 && n_bins <= kMaxBins,
-          "n_bins must be in [1, " + std::to_string(kMaxBins) + "]");
-    const int64_t L = in.sizes[0], T = in.sizes[1], C = in.sizes[2];
-    check(o.ndim == 3 && o.sizes[0] == L && o.sizes[1] == C &&
-              o.sizes[2] == n_bins + 1,
-          "output must be [layers, channels, n_bins + 1]");
-    check(T < (int64_t(1) << 26) && C < (int64_t(1) << 30), "input too large");
-    if (L == 0 || C == 0) return;
-    DeviceGuard guard(in.device);
-    const int tiles64 = static_cast<int>((C + 63) / 64);
-    const size_t lds = static_cast<size_t>(cdf_lds_bytes(static_cast<int>(T), n_bins));
-    const int vec_tile = (C % 16 == 0 && (reinterpret_cast<uintptr_t>(in.data) & 15) == 0) ? 1 : 0;
-    const auto kern = n_bins == 32         ? cdf_tile_kernel<32, true>
-                      : n_bins < 32          ? cdf_tile_kernel<32, false>
-                      : n_bins == kMaxBins   ? cdf_tile_kernel<kMaxBins, true>
-                                             : cdf_tile_kernel<kMaxBins, false>;
-    hipLaunchKernelGGL(kern, dim3(L * tiles64), dim3(kCdfThreads), lds, static_cast<hipStream_t>(stream),
-                       static_cast<const uint8_t *>(in.data), (int)T, (int)C, n_bins,
-                       static_cast<int16_t *>(o.data), tiles64, vec_tile);
-    hip_check(hipGetLastError(), "cdf_tile_kernel launch");
+    make_cdf(deref(input, "input"), n_bins, deref(output, "output"), nullptr, nullptr, 0,
+             static_cast<hipStream_t>(stream));
   });
 }
 
@@ -1757,86 +2087,82 @@ int lmc_encode_fast_new(const lmc_tensor *cdf_t, const lmc_tensor *input_sym,
                         const lmc_tensor *output_buffer,
                         const lmc_tensor *output_lengths, void *stream) {
   return guarded([&] {
+    encode_rows(deref(cdf_t, "cdf"), deref(input_sym, "input_sym"), deref(output_buffer, "output_buffer"),
+                deref(output_lengths, "output_lengths"), static_cast<hipStream_t>(stream));
+  });
+}
+
+int lmc_cachegen_encode_rows(const lmc_tensor *input, int32_t n_bins, const lmc_tensor *cdf_t,
+                             const lmc_tensor *rows_t, const lmc_tensor *lengths_t,
+                             const lmc_tensor *offsets_t, int64_t *total, void *stream_p) {
+  return guarded([&] {
+    const lmc_tensor &in = deref(input, "input");
     const lmc_tensor &cdf = deref(cdf_t, "cdf");
-    const lmc_tensor &in = deref(input_sym, "input_sym");
-    const lmc_tensor &ob = deref(output_buffer, "output_buffer");
-    const lmc_tensor &ol = deref(output_lengths, "output_lengths");
-    need_device(cdf, "cdf");
-    need_device(in, "input_sym");
-    need_device(ob, "output_buffer");
-    need_device(ol, "output_lengths");
-    check(in.ndim == 3 && cdf.ndim == 3 && ob.ndim == 3,
-          "cdf, input_sym and output_buffer must be 3-D");
-    const int64_t L = in.sizes[0], T = in.sizes[1], C = in.sizes[2];
-    const int64_t nb = cdf.sizes[2] - 1;
-    const int64_t chunk = ob.sizes[2];
-    // csrc/cachegen_kernels.cpp:33-35
-    check(C <= (1 << 15),
-          "encode takes at most 32768 channels per layer");
-    check(in.dtype == LMC_U8 || in.dtype == LMC_I8, "input_sym must be int8/uint8");
-    check(cdf.dtype == LMC_I16, "cdf must be int16");
-    check(ob.dtype == LMC_U8 || ob.dtype == LMC_I8, "output_buffer must be uint8");
-    check(ol.dtype == LMC_I32 && numel(ol) == L * C, "output_lengths must be int32 [L, C]");
-    check(nb >= 1 && nb <= kMaxBins, "number of bins must be in [1, 64]");
-    check(cdf.sizes[0] == L && cdf.sizes[1] == C, "cdf must be [L, C, nbins + 1]");
-    check(ob.sizes[0] == L && ob.sizes[1] == C, "output_buffer must be [L, C, chunk]");
-    if (L == 0 || C == 0) return;
+    const lmc_tensor &rows = deref(rows_t, "rows");
+    const lmc_tensor &lens = deref(lengths_t, "lengths");
+    const lmc_tensor &off = deref(offsets_t, "offsets");
+    check_value(total != nullptr, "total is null");
+    need_device(in, "input");
+    need_device(rows, "rows");
+    need_device(lens, "lengths");
+    need_device(off, "offsets");
+    check(in.ndim == 3 && rows.ndim == 3, "input and rows must be 3-D");
+    check(lens.dtype == LMC_I32 && numel(lens) == in.sizes[0] * in.sizes[2], "lengths must be int32 [L, C]");
+    const int64_t n_streams = in.sizes[0] * in.sizes[2];
+    const int64_t blocks = (n_streams + 63) / 64;
+    check(off.dtype == LMC_I64 && numel(off) == 2 * blocks + 1,
+          "offsets must be int64 with one entry per block of 64 streams, one more, and one per block of scratch");
+    *total = 0;
+    hipStream_t stream = static_cast<hipStream_t>(stream_p);
+    if (n_streams == 0) {
+      make_cdf(in, n_bins, cdf, nullptr, nullptr, 0, stream);
+      return;
+    }
     DeviceGuard guard(in.device);
-    const int tiles = static_cast<int>((C + kEncLanes - 1) / kEncLanes);
-    const int word_stores =
-        (chunk % 4 == 0 && (reinterpret_cast<uintptr_t>(ob.data) & 3) == 0) ? 1 : 0;
-    const int vec_in = (C % 16 == 0 && (reinterpret_cast<uintptr_t>(in.data) & 15) == 0) ? 1 : 0;
-    const bool rows_dw = (reinterpret_cast<uintptr_t>(cdf.data) & 3) == 0;
-    if (LMC_ENC_SPLIT && T > 0 && T <= kEncTileMaxT && nb <= kEncLanes && C % kEncLanes == 0 && vec_in &&
-        rows_dw) {
-      // Split encoder: bit rows of 2T bytes plus one word (codes are at
-      // most 16 bits), an odd number of words so that the lanes' rows start
-      // in different banks.
-      const int row_words = (static_cast<int>(T + 1) / 2 + 1) | 1;
-      const int rows_words = static_cast<int>(((nb + 1) * kEncLanes * 2 + 15) / 16 * 4);
-      const int phase1 = rows_words + kEncTileMaxT * kEncLanes / 4 + static_cast<int>(nb + 1) * kEncLanes;
-      const int stage_words = std::max(phase1, kEncLanes * row_words);
-      const size_t lds = 4 * (static_cast<size_t>((stage_words + kEncPieces * kEncLanes + 2) & ~1) + 2 * kEncLanes);
-      check(lds <= 65536, "encode: LDS budget exceeded");
-      hipLaunchKernelGGL(encode_split_kernel<kEncPieces>, dim3(L * tiles), dim3(64 * kEncPieces), lds,
-                         static_cast<hipStream_t>(stream),
-                         static_cast<const int16_t *>(cdf.data),
-                         static_cast<const uint8_t *>(in.data), (int)T, (int)C,
-                         (int)nb, static_cast<uint8_t *>(ob.data), chunk,
-                         static_cast<int32_t *>(ol.data), tiles, word_stores, row_words, stage_words);
-      hip_check(hipGetLastError(), "encode_split_kernel launch");
-      return;
-    }
-    if (T > 0 && T <= kEncTileMaxT && nb <= kEncLanes) {
-      // Bits past min(chunk, 2 bytes per symbol) are never written (codes
-      // are at most 16 bits), so a wave's bit buffer holds that many bytes.
-      const int64_t cap_bytes = std::min<int64_t>(chunk, 2 * T);
-      const int cap_words = static_cast<int>((cap_bytes + 3) / 4);
-      const int sym_stride = (((T + 3) / 4) + 1) | 1;
-      const size_t lds = 4 * ((static_cast<size_t>(nb + 1) * kEncLanes * 2 + 15) / 16 * 4 +
-                              static_cast<size_t>(kEncLanes) * sym_stride +
-                              static_cast<size_t>(2 * kEncWaves) * cap_words);
-      const int vec_tile = vec_in;
-      check(lds <= 65536, "encode: LDS budget exceeded");
-      hipLaunchKernelGGL(encode_wave_kernel, dim3(L * tiles), dim3(kEncTileThreads), lds,
-                         static_cast<hipStream_t>(stream),
-                         static_cast<const int16_t *>(cdf.data),
-                         static_cast<const uint8_t *>(in.data), (int)T, (int)C,
-                         (int)nb, static_cast<uint8_t *>(ob.data), chunk,
-                         static_cast<int32_t *>(ol.data), tiles, word_stores, vec_tile, sym_stride,
-                         cap_words);
-      hip_check(hipGetLastError(), "encode_wave_kernel launch");
-      return;
-    }
-    const size_t lds = static_cast<size_t>(nb) * kEncLanes * 4 +
-                       static_cast<size_t>(nb + 1) * kEncLanes * 2;
-    hipLaunchKernelGGL(encode_kernel, dim3(L * tiles), dim3(kEncLanes), lds,
-                       static_cast<hipStream_t>(stream),
-                       static_cast<const int16_t *>(cdf.data),
-                       static_cast<const uint8_t *>(in.data), (int)T, (int)C,
-                       (int)nb, static_cast<uint8_t *>(ob.data), chunk,
-                       static_cast<int32_t *>(ol.data), tiles, word_stores);
-    hip_check(hipGetLastError(), "encode_kernel launch");
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    hip_check(hipStreamIsCapturing(stream, &cap), "hipStreamIsCapturing");
+    check(cap == hipStreamCaptureStatusNone,
+          "a chunk's size is read on the host: its encoding cannot be captured into a graph");
+    int64_t *offsets = static_cast<int64_t *>(off.data);
+    int64_t *sums = offsets + blocks + 1;
+    make_cdf(in, n_bins, cdf, static_cast<int32_t *>(lens.data), sums, rows.sizes[2], stream);
+    // The sizes follow from the histograms, so the host learns the total
+    // while the rows are still being encoded.
+    HostWord word(in.device);
+    word.launching(stream);
+    hipLaunchKernelGGL(stream_offsets_kernel, dim3(1), dim3(kOffThreads), 0, stream, sums, blocks, offsets,
+                       word.word());
+    hip_check(hipGetLastError(), "stream_offsets_kernel launch");
+    word.record();
+    encode_rows(cdf, in, rows, lens, stream);
+    *total = word.wait();
+  });
+}
+
+int lmc_cachegen_pack_rows(const lmc_tensor *rows_t, const lmc_tensor *lengths_t, const lmc_tensor *offsets_t,
+                           const lmc_tensor *streams_t, void *stream) {
+  return guarded([&] {
+    const lmc_tensor &rows = deref(rows_t, "rows");
+    const lmc_tensor &lens = deref(lengths_t, "lengths");
+    const lmc_tensor &off = deref(offsets_t, "offsets");
+    const lmc_tensor &o = deref(streams_t, "streams");
+    need_device(rows, "rows");
+    need_device(lens, "lengths");
+    need_device(off, "offsets");
+    need_device(o, "streams");
+    check(rows.ndim == 3 && rows.dtype == LMC_U8 && o.dtype == LMC_U8, "rows and streams must be uint8");
+    const int64_t n_streams = rows.sizes[0] * rows.sizes[1];
+    const int64_t blocks = (n_streams + 63) / 64;
+    check(lens.dtype == LMC_I32 && numel(lens) == n_streams, "lengths must be int32 [L, C]");
+    check(off.dtype == LMC_I64 && numel(off) == 2 * blocks + 1, "offsets do not match the rows");
+    if (n_streams == 0 || numel(o) == 0) return;
+    check(blocks < (int64_t(1) << 31), "too many streams");
+    DeviceGuard guard(rows.device);
+    hipLaunchKernelGGL(pack_streams_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kPackThreads), 0,
+                       static_cast<hipStream_t>(stream), static_cast<const uint8_t *>(rows.data), rows.sizes[2],
+                       static_cast<const int32_t *>(lens.data), n_streams, static_cast<const int64_t *>(off.data),
+                       static_cast<uint8_t *>(o.data));
+    hip_check(hipGetLastError(), "pack_streams_kernel launch");
   });
 }
 

@@ -36,6 +36,8 @@ using BlendFn = int (*)(const lmc_tensor *, int32_t, const int64_t *, const lmc_
                         int64_t, int32_t, int32_t, int32_t, void *);
 using CdfFn = int (*)(const lmc_tensor *, int32_t, const lmc_tensor *, void *);
 using Codec4Fn = int (*)(const lmc_tensor *, const lmc_tensor *, const lmc_tensor *, const lmc_tensor *, void *);
+using EncodeRowsFn = int (*)(const lmc_tensor *, int32_t, const lmc_tensor *, const lmc_tensor *, const lmc_tensor *,
+                             const lmc_tensor *, int64_t *, void *);
 using ErrFn = const char *(*)();
 
 struct Table {
@@ -48,6 +50,8 @@ struct Table {
   CdfFn cdf = nullptr;
   Codec4Fn encode = nullptr;
   Codec4Fn decode = nullptr;
+  EncodeRowsFn encode_rows = nullptr;
+  Codec4Fn pack_rows = nullptr;
   ErrFn last_error = nullptr;
 } g;
 
@@ -228,9 +232,38 @@ void codec4(Codec4Fn fn, const at::Tensor &t0, const at::Tensor &t1, const at::T
   raise_for(fn(&a, &b, &c, &d, stream_of(dev)));
 }
 
+// A chunk's CDF, stream lengths and concatenated streams (formats.py).  The
+// rows and offsets are scratch of this call; the streams are allocated once
+// the device has written their size, which the rows' encoding overlaps.
+std::tuple<at::Tensor, at::Tensor, at::Tensor> cachegen_encode_chunk(const at::Tensor &symbols, int64_t n_bins,
+                                                                     int64_t cap) {
+  check_bound();
+  if (!symbols.is_cuda()) throw std::runtime_error("cachegen_encode_chunk: symbols must be a GPU tensor");
+  if (symbols.dim() != 3) throw std::runtime_error("input must be [layers, tokens, channels]");
+  const int64_t L = symbols.size(0), C = symbols.size(2);
+  const at::TensorOptions opt = symbols.options();
+  at::Tensor cdf = at::empty({L, C, n_bins + 1}, opt.dtype(at::kShort));
+  at::Tensor rows = at::empty({L, C, cap}, opt.dtype(at::kByte));
+  at::Tensor lengths = at::empty({L, C}, opt.dtype(at::kInt));
+  at::Tensor offsets = at::empty({2 * ((L * C + 63) / 64) + 1}, opt.dtype(at::kLong));
+  const lmc_tensor i = desc(symbols), c = desc(cdf), r = desc(rows), n = desc(lengths), o = desc(offsets);
+  void *stream = stream_of(symbols.get_device());
+  int64_t total = 0;
+  int status;
+  {
+    py::gil_scoped_release nogil;  // the call waits for the device
+    status = g.encode_rows(&i, static_cast<int32_t>(n_bins), &c, &r, &n, &o, &total, stream);
+  }
+  raise_for(status);
+  at::Tensor streams = at::empty({total}, opt.dtype(at::kByte));
+  const lmc_tensor s = desc(streams);
+  raise_for(g.pack_rows(&r, &n, &o, &s, stream));
+  return {cdf, lengths, streams};
+}
+
 void bind(uintptr_t multi, uintptr_t single, uintptr_t load_flash, uintptr_t reshape_flash,
           uintptr_t rope, uintptr_t blend, uintptr_t cdf, uintptr_t encode, uintptr_t decode,
-          uintptr_t last_error) {
+          uintptr_t encode_rows, uintptr_t pack_rows, uintptr_t last_error) {
   g.multi = reinterpret_cast<MultiFn>(multi);
   g.single = reinterpret_cast<SingleFn>(single);
   g.load_flash = reinterpret_cast<FlashFn>(load_flash);
@@ -240,6 +273,8 @@ void bind(uintptr_t multi, uintptr_t single, uintptr_t load_flash, uintptr_t res
   g.cdf = reinterpret_cast<CdfFn>(cdf);
   g.encode = reinterpret_cast<Codec4Fn>(encode);
   g.decode = reinterpret_cast<Codec4Fn>(decode);
+  g.encode_rows = reinterpret_cast<EncodeRowsFn>(encode_rows);
+  g.pack_rows = reinterpret_cast<Codec4Fn>(pack_rows);
   g.last_error = reinterpret_cast<ErrFn>(last_error);
 }
 
@@ -264,6 +299,7 @@ PYBIND11_MODULE(_c_ops_ext, m) {
   m.def("rotary_embedding_k_fused", &rotary_embedding_k_fused);
   m.def("blend_layer_to_paged", &blend_layer_to_paged);
   m.def("calculate_cdf", &calculate_cdf);
+  m.def("cachegen_encode_chunk", &cachegen_encode_chunk);
   m.def("encode_fast_new", [](const at::Tensor &cdf, const at::Tensor &sym, at::Tensor &out, at::Tensor &lens) {
     codec4(g.encode, cdf, sym, out, lens, sym);
   });

@@ -47,6 +47,8 @@ try:
         _addr("lmc_calculate_cdf"),
         _addr("lmc_encode_fast_new"),
         _addr("lmc_decode_fast_prefsum"),
+        _addr("lmc_cachegen_encode_rows"),
+        _addr("lmc_cachegen_pack_rows"),
         _addr("lmc_last_error"),
     )
 except ImportError:
@@ -399,6 +401,29 @@ def encode_fast_new(cdf, input_sym, output_buffer, output_lengths) -> None:
     dev = _device_index(input_sym)
     c, i, o, n = _desc(cdf), _desc(input_sym), _desc(output_buffer), _desc(output_lengths)
     _run(_L.lmc_encode_fast_new(_ref(c), _ref(i), _ref(o), _ref(n), _stream(dev)))
+
+
+def cachegen_encode_chunk(symbols, n_bins: int, cap: int):
+    """CDF int16 [L, C, n_bins + 1], stream lengths int32 [L, C] and the
+    concatenated streams of uint8 symbols [L, T, C]: calculate_cdf and
+    encode_fast_new into rows of `cap` bytes, then the rows' used bytes
+    one after the other.  Waits for the streams' total size."""
+    if _ext is not None:
+        return _ext.cachegen_encode_chunk(symbols, int(n_bins), int(cap))
+    L, _, C = symbols.shape
+    dev = symbols.device
+    cdf = torch.empty((L, C, int(n_bins) + 1), dtype=torch.int16, device=dev)
+    rows = torch.empty((L, C, int(cap)), dtype=torch.uint8, device=dev)
+    lengths = torch.empty((L, C), dtype=torch.int32, device=dev)
+    offsets = torch.empty(2 * ((L * C + 63) // 64) + 1, dtype=torch.int64, device=dev)
+    total = ctypes.c_int64(0)
+    i, c, r, n, o = _desc(symbols), _desc(cdf), _desc(rows), _desc(lengths), _desc(offsets)
+    _run(_L.lmc_cachegen_encode_rows(_ref(i), int(n_bins), _ref(c), _ref(r), _ref(n), _ref(o), ctypes.byref(total),
+                                     _stream(dev.index)))
+    streams = torch.empty(total.value, dtype=torch.uint8, device=dev)
+    s = _desc(streams)
+    _run(_L.lmc_cachegen_pack_rows(_ref(r), _ref(n), _ref(o), _ref(s), _stream(dev.index)))
+    return cdf, lengths, streams
 
 
 def decode_fast_new(cdf, bytestreams, lengths, output) -> None:

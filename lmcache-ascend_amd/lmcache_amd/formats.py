@@ -198,17 +198,14 @@ def encode_chunk(symbols: torch.Tensor, n_bins: int, max_stream_bytes: int = 0) 
     """Encodes uint8 symbols [L, T, C] (values below n_bins) on the GPU:
     calculate_cdf, encode_fast_new into per-stream rows of
     `max_stream_bytes` (default: enough for 16 bits per symbol), then the
-    rows' used bytes concatenated in (layer, channel) order."""
+    rows' used bytes concatenated in (layer, channel) order.  The streams'
+    size is read on the host before the call returns."""
     if not symbols.is_cuda or symbols.dtype != torch.uint8 or symbols.dim() != 3:
         raise ValueError("encode_chunk takes uint8 GPU symbols [L, T, C]")
     L, T, C = symbols.shape
     cap = int(max_stream_bytes) or 2 * T
-    cdf = c_ops.calculate_cdf(symbols, int(n_bins))
-    rows = torch.zeros((L, C, cap), dtype=torch.uint8, device=symbols.device)
-    lengths = torch.zeros((L, C), dtype=torch.int32, device=symbols.device)
-    c_ops.encode_fast_new(cdf, symbols, rows, lengths)
-    used = torch.arange(cap, device=symbols.device).view(1, 1, cap) < lengths.unsqueeze(-1)
-    return CacheGenChunk(cdf, lengths, rows[used], int(T))
+    cdf, lengths, streams = c_ops.cachegen_encode_chunk(symbols, int(n_bins), cap)
+    return CacheGenChunk(cdf, lengths, streams, int(T))
 
 
 def decode_chunk(chunk: CacheGenChunk) -> torch.Tensor:

@@ -1,0 +1,59 @@
+"""GPU tests of the chunk codec's own paths (formats.encode_chunk and
+decode_chunk) against the CPU oracle, at the sizes where their kernels can go
+wrong: blocks of 64 streams that span layers or are partly filled, rows that
+do not start on a dword, streams cut to a row's capacity, and chunks longer
+than one 256-token piece."""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import cachegen as oc
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def F():
+    from lmcache_amd import formats
+
+    return formats
+
+
+def _symbols(L, T, C, nb, seed, kind="normal"):
+    rng = np.random.default_rng(seed)
+    if kind == "normal":
+        return oc.quantize(rng.normal(0, 2, size=(L, T, C)).astype(np.float32), nb)
+    if kind == "constant":  # one present symbol per stream: 1-bit codes
+        return np.broadcast_to(rng.integers(0, nb, size=(L, 1, C), dtype=np.uint8), (L, T, C)).copy()
+    # Skewed counts (the longest codes), with symbols past nb that are not coded.
+    p = 0.5 ** np.minimum(np.arange(nb + 1), 14)
+    return rng.choice(nb + 1, size=(L, T, C), p=p / p.sum()).astype(np.uint8)
+
+
+# Streams end inside a block (L * C % 64 != 0), blocks span layers (C = 96,
+# 32, 17), rows start at odd addresses (cap odd), and caps cut streams.
+@pytest.mark.parametrize("kind", ["normal", "constant", "skewed"])
+@pytest.mark.parametrize("L,T,C,nb,cap", [
+    (1, 1, 32, 16, 0), (2, 256, 96, 32, 0), (3, 37, 17, 16, 0), (5, 255, 48, 32, 511), (3, 64, 96, 33, 7),
+    (2, 257, 64, 32, 0), (1, 1000, 160, 32, 0), (2, 600, 33, 16, 301), (3, 300, 96, 64, 0), (1, 9, 1, 2, 0),
+])
+def test_encode_chunk_vs_oracle(F, L, T, C, nb, cap, kind):
+    sym = _symbols(L, T, C, nb, L * T + C + nb, kind)
+    chunk = F.encode_chunk(torch.from_numpy(sym).to(DEV), nb, cap)
+    cdf = oc.calculate_cdf(sym, nb)
+    rows, lens = oc.encode(cdf, sym, cap or 2 * T)
+    kept = np.minimum(lens, rows.shape[2])
+    want = np.concatenate([rows[l, c, :kept[l, c]] for l in range(L) for c in range(C)])
+    assert np.array_equal(chunk.cdf.cpu().numpy(), cdf)
+    assert np.array_equal(chunk.lengths.cpu().numpy(), lens)
+    assert np.array_equal(chunk.streams.cpu().numpy(), want)
+
+
+def test_encode_chunk_without_tokens_or_streams(F):
+    for shape in [(2, 0, 64), (0, 5, 64), (2, 5, 0)]:
+        chunk = F.encode_chunk(torch.zeros(shape, dtype=torch.uint8, device=DEV), 16)
+        assert chunk.streams.numel() == 0
+        assert chunk.lengths.shape == (shape[0], shape[2]) and int(chunk.lengths.sum()) == 0
