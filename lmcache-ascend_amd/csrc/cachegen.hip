@@ -1324,7 +1324,7 @@ template <class Tab>
 __device__ __forceinline__ void decode_block_fast(const Tab &tb, int T, int C,
                                                   const uint32_t *win, uint32_t win_last,
                                                   uint32_t lo, uint32_t hi, uint8_t *obuf,
-                                                  uint8_t *__restrict__ out_blk) {
+                                                  uint32_t *__restrict__ odst) {
   const int lane = static_cast<int>(threadIdx.x);
   uint32_t q = lo & ~3u;
   uint64_t buf = static_cast<uint64_t>(clip_word(win[q >> 2], q, hi)) << 32;
@@ -1346,8 +1346,7 @@ __device__ __forceinline__ void decode_block_fast(const Tab &tb, int T, int C,
     have -= len;
     return s;
   };
-  // Lane j stores token (t0 + j / 16), channels 4 * (j % 16) .. + 3.
-  uint32_t *odst = reinterpret_cast<uint32_t *>(out_blk + static_cast<int64_t>(lane >> 4) * C) + (lane & 15);
+  // odst: DecBlock::quad, a full block.
   const int64_t step4 = static_cast<int64_t>(C);  // in dwords: 4 tokens of C bytes
   int t = 0;
   for (; t + 4 <= T; t += 4) {
@@ -1373,13 +1372,12 @@ __device__ __forceinline__ void decode_block_fast(const Tab &tb, int T, int C,
 __device__ __forceinline__ void decode_block_bytes(const cgdec::ByteTables &tb, int T, int C,
                                                    const uint32_t *win, uint32_t win_last,
                                                    uint32_t lo, uint32_t hi, uint8_t *obuf,
-                                                   uint8_t *__restrict__ out_blk) {
+                                                   uint32_t *__restrict__ odst) {
   const int lane = static_cast<int>(threadIdx.x);
   cgdec::BitCursor cur;
   cur.start(win, win_last, 8 * lo, hi);
   auto step = [&]() -> uint32_t { return tb.step(cur) >> 3; };
-  // Lane j stores token (t0 + j / 16), channels 4 * (j % 16) .. + 3.
-  uint32_t *odst = reinterpret_cast<uint32_t *>(out_blk + static_cast<int64_t>(lane >> 4) * C) + (lane & 15);
+  // odst: DecBlock::quad, a full block.
   const int64_t step4 = static_cast<int64_t>(C);  // in dwords: 4 tokens of C bytes
   int t = 0;
   for (; t + 4 <= T; t += 4) {
@@ -1402,20 +1400,20 @@ __device__ __forceinline__ void decode_block_bytes(const cgdec::ByteTables &tb, 
 // with the escape branch.
 __device__ __forceinline__ void decode_fast(const cgdec::ByteTables &tb, int T, int C,
                                             const uint32_t *win, uint32_t win_last, uint32_t lo,
-                                            uint32_t hi, uint8_t *obuf, uint8_t *__restrict__ out_blk) {
+                                            uint32_t hi, uint8_t *obuf, uint32_t *__restrict__ odst) {
   if (__any(tb.escapes)) {
     cgdec::ByteTables t = tb;
     t.finish();
-    decode_block_fast(t, T, C, win, win_last, lo, hi, obuf, out_blk);
+    decode_block_fast(t, T, C, win, win_last, lo, hi, obuf, odst);
   } else {
-    decode_block_bytes(tb, T, C, win, win_last, lo, hi, obuf, out_blk);
+    decode_block_bytes(tb, T, C, win, win_last, lo, hi, obuf, odst);
   }
 }
 
 __device__ __forceinline__ void decode_fast(const DecTables &tb, int T, int C, const uint32_t *win,
                                             uint32_t win_last, uint32_t lo, uint32_t hi, uint8_t *obuf,
-                                            uint8_t *__restrict__ out_blk) {
-  decode_block_fast(tb, T, C, win, win_last, lo, hi, obuf, out_blk);
+                                            uint32_t *__restrict__ odst) {
+  decode_block_fast(tb, T, C, win, win_last, lo, hi, obuf, odst);
 }
 
 // One stream occupying [lo, hi) (addresses), symbols to o[0], o[C], ...
@@ -1457,30 +1455,60 @@ __device__ __forceinline__ void decode_stream(const Tab &tb, int T, int C,
   }
 }
 
+// Layer and channel of a stream `k` streams after (l, c); streams are
+// numbered over the layers, channels fastest.
+struct StreamAt {
+  int64_t l;
+  int c;
+};
+__device__ __forceinline__ StreamAt stream_at(int64_t l, int c, uint32_t k, int C) {
+  const uint32_t x = static_cast<uint32_t>(c) + k;
+  const uint32_t up = x / static_cast<uint32_t>(C);
+  return {l + up, static_cast<int>(x - up * static_cast<uint32_t>(C))};
+}
+
 // Stream geometry of one decode block: lane i of a wave owns stream
 // s0 + i; bytes of the block's streams are [B0, B1) of the byte buffer.
 struct DecBlock {
-  int l, c0, cnt;
+  int cnt;  // streams of the block: 64 but for the last
   int64_t s0, start, end, B0, B1;
+  int64_t l0;  // layer and channel of stream s0
+  int c0;
   uintptr_t R0, R1, r_lo;
 
   __device__ __forceinline__ void init(const int16_t *cdf, int64_t nbytes, const int32_t *prefix,
-                                       int C, int nb, int tiles, int lane) {
-    l = blockIdx.x / tiles;
-    c0 = (blockIdx.x % tiles) * kDecLanes;
-    cnt = C - c0 < kDecLanes ? C - c0 : kDecLanes;
-    s0 = static_cast<int64_t>(l) * C + c0;
+                                       int64_t n_streams, int C, int nb, int lane) {
+    s0 = static_cast<int64_t>(blockIdx.x) * kDecLanes;
+    l0 = s0 < (int64_t(1) << 32) ? static_cast<uint32_t>(s0) / static_cast<uint32_t>(C) : s0 / C;
+    c0 = static_cast<int>(s0 - l0 * C);
+    cnt = n_streams - s0 < kDecLanes ? static_cast<int>(n_streams - s0) : kDecLanes;
     const int64_t stream = s0 + (lane < cnt ? lane : 0);
     auto clampb = [&](int64_t x) { return x < 0 ? 0 : (x > nbytes ? nbytes : x); };
     start = clampb(stream == 0 ? 0 : prefix[stream - 1]);
     end = clampb(prefix[stream]);
-    end = end < start ? start : end;
+    end = end < start || lane >= cnt ? start : end;
     B0 = clampb(s0 == 0 ? 0 : prefix[s0 - 1]);
     B1 = clampb(prefix[s0 + cnt - 1]);
     // Rows: bytes [R0, R1) from the 16-byte aligned address at or below R0.
     R0 = reinterpret_cast<uintptr_t>(cdf + s0 * (nb + 1));
     R1 = R0 + static_cast<uintptr_t>(cnt) * (nb + 1) * 2;
     r_lo = R0 & ~uintptr_t(15);
+  }
+
+  // The transposed symbols of four tokens are stored as dwords: lane j's is
+  // dword `at` of the transpose (token at / 16 of the four, streams
+  // 4 * (at % 16) .. + 3, of one layer: C % 4 == 0), stored at `dst` for the
+  // first four tokens.  `at` is j in a full block; in a block of 32 streams
+  // (C % 32 == 0, so there is no other) the upper eight dwords of a token
+  // repeat the lower eight, so that no store is predicated.
+  struct Quad {
+    int at;
+    uint32_t *dst;
+  };
+  __device__ __forceinline__ Quad quad(uint8_t *out, int T, int C, int lane) const {
+    const int at = cnt == kDecLanes ? lane : lane & 0x37;
+    const StreamAt a = stream_at(l0, c0, 4u * static_cast<uint32_t>(at & 15), C);
+    return {at, reinterpret_cast<uint32_t *>(out + (a.l * T + (at >> 4)) * C + a.c)};
   }
 
   // 16-byte chunks of the window staged from a_lo: the block's bytes from
@@ -1501,14 +1529,14 @@ template <class Tab>
 __device__ __forceinline__ void decode_one_wave(uint8_t *lds, const int16_t *__restrict__ cdf,
                                                 const uint8_t *__restrict__ bytes, int64_t nbytes,
                                                 const int32_t *__restrict__ prefix, int T, int C,
-                                                int nb, uint8_t *__restrict__ out, int tiles,
+                                                int nb, uint8_t *__restrict__ out, int64_t n_streams,
                                                 int lane) {
   constexpr int kRowsOff = Tab::kBytes + kObufBytes;
   const int rows_cap = ((nb + 1) * kDecLanes * 2 + 32 + 15) & ~15;
   const int win_off = kRowsOff + rows_cap;
   const int win_cap = (kDecLds - win_off) & ~15;
   DecBlock bk;
-  bk.init(cdf, nbytes, prefix, C, nb, tiles, lane);
+  bk.init(cdf, nbytes, prefix, n_streams, C, nb, lane);
   const int live = lane < bk.cnt;
   const uintptr_t base0 = reinterpret_cast<uintptr_t>(bytes);
   const uintptr_t a_lo = (base0 + bk.B0) & ~uintptr_t(15);
@@ -1549,17 +1577,19 @@ __device__ __forceinline__ void decode_one_wave(uint8_t *lds, const int16_t *__r
                     __all(in_win);
   if (!live) return;
   const uint32_t *win = reinterpret_cast<const uint32_t *>(lds + win_off);
-  uint8_t *out_blk = out + static_cast<int64_t>(bk.l) * T * C + bk.c0;
   if (fast) {
+    uint32_t *odst = bk.quad(out, T, C, lane).dst;  // a full block
     decode_fast(tb, T, C, win, static_cast<uint32_t>(a_hi - a_lo) - 4,
                 static_cast<uint32_t>(lo - a_lo), static_cast<uint32_t>(hi - a_lo),
-                lds + Tab::kBytes, out_blk);
+                lds + Tab::kBytes, odst);
   } else {
     tb.finish();
+    const StreamAt at = stream_at(bk.l0, bk.c0, static_cast<uint32_t>(lane), C);
+    uint8_t *o = out + at.l * T * C + at.c;
     if (in_win)
-      decode_stream<true>(tb, T, C, bytes, win, a_lo, a_hi, lo, hi, out_blk + lane);
+      decode_stream<true>(tb, T, C, bytes, win, a_lo, a_hi, lo, hi, o);
     else
-      decode_stream<false>(tb, T, C, bytes, win, a_lo, a_hi, lo, hi, out_blk + lane);
+      decode_stream<false>(tb, T, C, bytes, win, a_lo, a_hi, lo, hi, o);
   }
 }
 
@@ -1576,7 +1606,8 @@ __device__ __forceinline__ void decode_one_wave(uint8_t *lds, const int16_t *__r
 __device__ __forceinline__ bool decode_one_wave_lanes(uint8_t *lds, const int16_t *__restrict__ cdf,
                                                       const uint8_t *__restrict__ bytes, int64_t nbytes,
                                                       const int32_t *__restrict__ prefix, int T, int C, int nb,
-                                                      uint8_t *__restrict__ out, int tiles, int lane) {
+                                                      uint8_t *__restrict__ out, int64_t n_streams,
+                                                      int lane) {
   using Tab = cgdec::ByteTables;
   constexpr int kRowsOff = Tab::kBytes + kObufBytes;
   constexpr int kLaneBatch = 8;  // 16-byte chunks per lane and load batch
@@ -1588,9 +1619,8 @@ __device__ __forceinline__ bool decode_one_wave_lanes(uint8_t *lds, const int16_
   const uint32_t lds_at =
       static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t *)lds));
   DecBlock bk;
-  bk.init(cdf, nbytes, prefix, C, nb, tiles, lane);
-  if (bk.cnt != kDecLanes || (reinterpret_cast<uintptr_t>(out) & 3) != 0 || (C & 3) != 0 ||
-      (lds_at & (Tab::kBytes - 1)) != 0)
+  bk.init(cdf, nbytes, prefix, n_streams, C, nb, lane);
+  if ((reinterpret_cast<uintptr_t>(out) & 3) != 0 || (C & 3) != 0 || (lds_at & (Tab::kBytes - 1)) != 0)
     return false;
   // The rows' loads depend on the block alone: issued before the stream
   // lengths (prefix loads) are waited for.
@@ -1634,7 +1664,10 @@ __device__ __forceinline__ bool decode_one_wave_lanes(uint8_t *lds, const int16_
   for (int u = 0; u < kLaneBatch; ++u)
     if (static_cast<uint32_t>(u) < n_ch) cv[u] = reinterpret_cast<global_chunk16 *>(a0)[u];
   wave_sync();
-  tb.row.r = reinterpret_cast<const int16_t *>(lds + kRowsOff + (bk.R0 - bk.r_lo)) + lane * (nb + 1);
+  // A lane without a stream (the last block) decodes stream s0's row over an
+  // empty region and stores nothing.
+  tb.row.r = reinterpret_cast<const int16_t *>(lds + kRowsOff + (bk.R0 - bk.r_lo)) +
+             (lane < bk.cnt ? lane : 0) * (nb + 1);
   tb.nb = nb;
   tb.build(lds + Tab::kBytes + lane);  // obuf byte: scratch for skipped writes
 #pragma unroll
@@ -1651,9 +1684,8 @@ __device__ __forceinline__ bool decode_one_wave_lanes(uint8_t *lds, const int16_
   uint32_t *reg32 = reinterpret_cast<uint32_t *>(region);
   cgdec::LaneRegion::seal(reg32, static_cast<uint32_t>(s_lo - a0), len);
   uint8_t *obuf = lds + Tab::kBytes;
-  uint8_t *out_blk = out + static_cast<int64_t>(bk.l) * T * C + bk.c0;
-  // Lane j stores token (t0 + j / 16), channels 4 * (j % 16) .. + 3.
-  uint32_t *odst = reinterpret_cast<uint32_t *>(out_blk + static_cast<int64_t>(lane >> 4) * C) + (lane & 15);
+  const DecBlock::Quad quad = bk.quad(out, T, C, lane);
+  uint32_t *odst = quad.dst;
   const int64_t step4 = static_cast<int64_t>(C);  // in dwords: 4 tokens of C bytes
   if (!__any(tb.escapes)) {
     // Four tokens per group (cgdec::GroupCursor): the four table entries go
@@ -1688,7 +1720,7 @@ __device__ __forceinline__ bool decode_one_wave_lanes(uint8_t *lds, const int16_
       obuf[2 * kDecLanes + lane] = static_cast<uint8_t>(e2);
       obuf[3 * kDecLanes + lane] = static_cast<uint8_t>(e3);
       wave_sync();
-      word = reinterpret_cast<const uint32_t *>(obuf)[lane];
+      word = reinterpret_cast<const uint32_t *>(obuf)[quad.at];
       wave_sync();
     }
     if (t > 0) {
@@ -1698,7 +1730,7 @@ __device__ __forceinline__ bool decode_one_wave_lanes(uint8_t *lds, const int16_
     if (t < T) {
       for (int i = 0; t + i < T; ++i) obuf[i * kDecLanes + lane] = static_cast<uint8_t>(gc.single(tb));
       wave_sync();
-      if ((lane >> 4) < T - t) cg_st(odst, reinterpret_cast<const uint32_t *>(obuf)[lane]);
+      if ((quad.at >> 4) < T - t) cg_st(odst, reinterpret_cast<const uint32_t *>(obuf)[quad.at]);
     }
   } else {
     tb.finish();
@@ -1716,14 +1748,14 @@ __device__ __forceinline__ bool decode_one_wave_lanes(uint8_t *lds, const int16_
 #pragma unroll
       for (int i = 0; i < 4; ++i) obuf[i * kDecLanes + lane] = step();
       wave_sync();
-      cg_st(odst, reinterpret_cast<const uint32_t *>(obuf)[lane]);
+      cg_st(odst, reinterpret_cast<const uint32_t *>(obuf)[quad.at]);
       odst += step4;
       wave_sync();
     }
     if (t < T) {
       for (int i = 0; t + i < T; ++i) obuf[i * kDecLanes + lane] = step();
       wave_sync();
-      if ((lane >> 4) < T - t) cg_st(odst, reinterpret_cast<const uint32_t *>(obuf)[lane]);
+      if ((quad.at >> 4) < T - t) cg_st(odst, reinterpret_cast<const uint32_t *>(obuf)[quad.at]);
     }
   }
   return true;
@@ -1734,15 +1766,178 @@ __global__ void __launch_bounds__(kDecLanes)
     decode_kernel(const int16_t *__restrict__ cdf,
                   const uint8_t *__restrict__ bytes, int64_t nbytes,
                   const int32_t *__restrict__ prefix, int T, int C, int nb,
-                  uint8_t *__restrict__ out, int tiles) {
+                  uint8_t *__restrict__ out, int64_t n_streams) {
   extern __shared__ uint32_t lds_words[];
   uint8_t *lds = reinterpret_cast<uint8_t *>(lds_words);
   const int lane = static_cast<int>(threadIdx.x);
   if constexpr (std::is_same<Tab, cgdec::ByteTables>::value) {
-    if (LMC_DEC_LANES && decode_one_wave_lanes(lds, cdf, bytes, nbytes, prefix, T, C, nb, out, tiles, lane))
+    if (LMC_DEC_LANES && decode_one_wave_lanes(lds, cdf, bytes, nbytes, prefix, T, C, nb, out, n_streams, lane))
       return;
   }
-  decode_one_wave<Tab>(lds, cdf, bytes, nbytes, prefix, T, C, nb, out, tiles, lane);
+  decode_one_wave<Tab>(lds, cdf, bytes, nbytes, prefix, T, C, nb, out, n_streams, lane);
+}
+
+// Decode of streams longer than the lane regions hold (n_bins <= 32, more
+// than kLaneMaxT tokens): one wave per 64 streams, the codes looked up in
+// cgdec::LongTables (chunks of more than 256 tokens have codes of up to 12
+// bits), the streams read through per-lane rings (cgdec::RingCursor), so the
+// LDS a block takes does not grow with the chunk.  A block takes kEpoch
+// tokens at a time: the chunks that refill the ring over an epoch are loaded
+// at its start and stored at its end, so nothing waits for them.  A ring
+// holds 256 bytes; kEpoch codes of at most 16 bits take 64 of them, and an
+// epoch loads as many chunks as there is room for, up to 64 bytes, so at
+// least 100 bytes lie ahead of the cursor at the start of every epoch.
+// Bound by the serial chain of each stream (one wave per 64 streams): about
+// 220 cycles a code, two table reads and their select.  56 planes x 1000
+// tokens x 256 channels: 101 us; the shared-window kernel took 1307 us, since
+// the streams of a block outgrow its LDS window and were read a dword at a
+// time from memory, with a binary search per symbol after the first long code.
+// The line is at 256 tokens because calculate_cdf's codes are at most 8 bits
+// long up to there, which the byte tables and lane regions of decode_kernel
+// hold whole.
+constexpr int kEpoch = 32;
+constexpr int kEpochChunks = 4;  // 16-byte chunks per lane and epoch
+constexpr int kFirstChunks = 8;
+constexpr int kLaneMaxT = 256;
+constexpr int kLongRing = cgdec::LongTables::kBytes;
+constexpr int kLongObuf = kLongRing + static_cast<int>(cgdec::RingCursor::kBytes) * kDecLanes;
+constexpr int kLongRows = kLongObuf + kObufBytes;
+constexpr int long_lds_bytes(int nb) { return kLongRows + (((nb + 1) * kDecLanes * 2 + 32 + 15) & ~15); }
+
+__global__ void __launch_bounds__(kDecLanes)
+    decode_long_kernel(const int16_t *__restrict__ cdf, const uint8_t *__restrict__ bytes, int64_t nbytes,
+                       const int32_t *__restrict__ prefix, int T, int C, int nb, uint8_t *__restrict__ out,
+                       int64_t n_streams) {
+  extern __shared__ uint32_t lds_words[];
+  uint8_t *lds = reinterpret_cast<uint8_t *>(lds_words);
+  const uint32_t lds_at =
+      static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t *)lds));
+  const int lane = static_cast<int>(threadIdx.x);
+  DecBlock bk;
+  bk.init(cdf, nbytes, prefix, n_streams, C, nb, lane);
+  const int nrow = static_cast<int>((bk.R1 - bk.r_lo + 15) >> 4);
+  chunk16 rv[kRowChunks], cv[kFirstChunks];
+  load_chunks(bk.r_lo, nrow, 0, lane, rv);
+  const uintptr_t s_lo = reinterpret_cast<uintptr_t>(bytes) + static_cast<uintptr_t>(bk.start);
+  const uint32_t len = static_cast<uint32_t>(bk.end - bk.start);
+  const uintptr_t a0 = s_lo & ~uintptr_t(15);
+  const uint32_t end = static_cast<uint32_t>(s_lo - a0) + len;  // the stream's end from a0
+  // Chunks [a0, a0 + 16 n_ch) each hold a byte of the stream, so no load
+  // leaves the buffer's pages.
+  const uint32_t n_ch = len ? (end + 15u) >> 4 : 0u;
+#pragma unroll
+  for (int u = 0; u < kFirstChunks; ++u)
+    if (static_cast<uint32_t>(u) < n_ch) cv[u] = reinterpret_cast<global_chunk16 *>(a0)[u];
+  cgdec::LongTables tb;
+  tb.bind(lds, lane, lds_at);
+  tb.clear();
+  store_chunks<false>(lds + kLongRows, nrow, 0, lane, rv);
+  for (int j0 = kDecLanes * kRowChunks; j0 < nrow; j0 += kDecLanes * kRowChunks) {
+    load_chunks(bk.r_lo, nrow, j0, lane, rv);
+    store_chunks<false>(lds + kLongRows, nrow, j0, lane, rv);
+  }
+  wave_sync();
+  tb.one.row.r = reinterpret_cast<const int16_t *>(lds + kLongRows + (bk.R0 - bk.r_lo)) +
+                 (lane < bk.cnt ? lane : 0) * (nb + 1);
+  tb.one.nb = nb;
+  uint8_t *obuf = lds + kLongObuf;
+  tb.build(obuf + lane);
+  // Dword d of the stream's chunks with its bytes past the stream's end zero,
+  // to the ring.
+  uint32_t *ring = reinterpret_cast<uint32_t *>(lds + kLongRing) + lane;
+  constexpr uint32_t kRingDw = cgdec::RingCursor::kBytes / 4;
+  auto put = [&](uint32_t chunk, const chunk16 &v) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t d = 4u * chunk + static_cast<uint32_t>(i);
+      const int left = static_cast<int>(end) - static_cast<int>(4u * d);
+      const uint32_t x = i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w;
+      const uint32_t keep = left >= 4 ? ~0u : left <= 0 ? 0u : (1u << (8 * left)) - 1u;
+      ring[(d & (kRingDw - 1u)) * kDecLanes] = x & keep;
+    }
+  };
+  chunk16 zero = {0u, 0u, 0u, 0u};
+#pragma unroll
+  for (int u = 0; u < kFirstChunks; ++u) put(static_cast<uint32_t>(u), static_cast<uint32_t>(u) < n_ch ? cv[u] : zero);
+  uint32_t filled = kFirstChunks;  // chunks in the ring or before it
+  wave_sync();
+  const DecBlock::Quad quad = bk.quad(out, T, C, lane);
+  uint32_t *odst = quad.dst;
+  const int64_t step4 = static_cast<int64_t>(C);  // in dwords: 4 tokens of C bytes
+  const int groups = (T + 3) / 4;
+  const uint32_t first_bit = 8u * static_cast<uint32_t>(s_lo - a0);
+  const uint32_t column = lds_at + kLongRing + 4u * static_cast<uint32_t>(lane);
+  // The chunks of one epoch: loads, then (after its tokens) the ring.
+  chunk16 nv[kEpochChunks];
+  uint32_t room = 0;
+  auto load_epoch = [&](uint32_t q) {
+    room = (cgdec::RingCursor::kBytes - (16u * filled - q)) >> 4;
+    room = room < kEpochChunks ? room : kEpochChunks;
+#pragma unroll
+    for (uint32_t u = 0; u < kEpochChunks; ++u) {
+      nv[u] = zero;
+      if (u < room && filled + u < n_ch) nv[u] = reinterpret_cast<global_chunk16 *>(a0)[filled + u];
+    }
+  };
+  auto store_epoch = [&]() {
+#pragma unroll
+    for (uint32_t u = 0; u < kEpochChunks; ++u)
+      if (u < room) put(filled + u, nv[u]);
+    filled += room;
+    wave_sync();
+  };
+  if (!__any(tb.irregular)) {
+    cgdec::PairCursor cur;
+    cur.start(tb, column, first_bit);
+    uint32_t word = 0;
+    // Four tokens; each transposed word is stored one group late, as in
+    // decode_one_wave_lanes.
+    auto group = [&](bool store_prev) {
+      uint32_t e0, e1, e2, e3;
+      cur.pair(tb, e0, e1);
+      obuf[lane] = static_cast<uint8_t>(e0);
+      obuf[kDecLanes + lane] = static_cast<uint8_t>(e1);
+      if (store_prev) {
+        cg_st(odst, (word >> 3) & 0x1F1F1F1Fu);
+        odst += step4;
+      }
+      cur.pair(tb, e2, e3);
+      obuf[2 * kDecLanes + lane] = static_cast<uint8_t>(e2);
+      obuf[3 * kDecLanes + lane] = static_cast<uint8_t>(e3);
+      wave_sync();
+      word = reinterpret_cast<const uint32_t *>(obuf)[quad.at];
+      wave_sync();
+    };
+    constexpr int kGroups = kEpoch / 4;
+    int g = 0;
+    for (; g + kGroups <= groups; g += kGroups) {
+      load_epoch(cur.ring.q);
+#pragma unroll
+      for (int i = 0; i < kGroups; ++i) group(i > 0 || g > 0);
+      store_epoch();
+    }
+    for (; g < groups; ++g) group(g > 0);
+    if ((quad.at >> 4) < T - 4 * (groups - 1)) cg_st(odst, (word >> 3) & 0x1F1F1F1Fu);
+  } else {
+    tb.one.finish();
+    cgdec::RingCursor cur;
+    cur.start(column, first_bit);
+    for (int g = 0; g < groups; ++g) {
+      if (g % (kEpoch / 4) == 0) load_epoch(cur.q);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        int sym, n;
+        tb.search(cur.hi() >> 16, sym, n);
+        obuf[i * kDecLanes + lane] = static_cast<uint8_t>(sym);
+        cur.advance(static_cast<uint32_t>(n));
+      }
+      wave_sync();
+      if ((quad.at >> 4) < T - 4 * g) cg_st(odst, reinterpret_cast<const uint32_t *>(obuf)[quad.at]);
+      odst += step4;
+      wave_sync();
+      if (g % (kEpoch / 4) == kEpoch / 4 - 1) store_epoch();
+    }
+  }
 }
 
 // Exclusive prefix sums of the blocks' byte counts, in one workgroup: off[b]
@@ -2205,16 +2400,21 @@ int lmc_decode_fast_prefsum(const lmc_tensor *cdf_t,
     check(numel(o) == L * T * C, "output must hold L * T * C symbols");
     if (L == 0 || C == 0 || T == 0) return;
     DeviceGuard guard(bs.device);
-    const int tiles = static_cast<int>((C + kDecLanes - 1) / kDecLanes);
-    const size_t lds = kDecLds;
-    hipLaunchKernelGGL(nb <= cgdec::ByteTables::kMaxBins ? decode_kernel<cgdec::ByteTables>
-                                                       : decode_kernel<DecTables>,
-                       dim3(L * tiles), dim3(kDecLanes), lds,
+    const int64_t n_streams = L * C;
+    const int64_t blocks = (n_streams + kDecLanes - 1) / kDecLanes;
+    check(blocks < (int64_t(1) << 31), "too many streams");
+    const bool long_streams = nb <= cgdec::ByteTables::kMaxBins && T > kLaneMaxT &&
+                              (reinterpret_cast<uintptr_t>(o.data) & 3) == 0;
+    const auto kern = long_streams                          ? decode_long_kernel
+                      : nb <= cgdec::ByteTables::kMaxBins ? decode_kernel<cgdec::ByteTables>
+                                                            : decode_kernel<DecTables>;
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(kDecLanes),
+                       long_streams ? long_lds_bytes(static_cast<int>(nb)) : kDecLds,
                        static_cast<hipStream_t>(stream),
                        static_cast<const int16_t *>(cdf.data),
                        static_cast<const uint8_t *>(bs.data), numel(bs),
                        static_cast<const int32_t *>(ln.data), (int)T, (int)C,
-                       (int)nb, static_cast<uint8_t *>(o.data), tiles);
+                       (int)nb, static_cast<uint8_t *>(o.data), n_streams);
     hip_check(hipGetLastError(), "decode_kernel launch");
   });
 }

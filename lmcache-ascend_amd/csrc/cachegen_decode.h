@@ -311,6 +311,22 @@ struct ByteTables {
   // table, which the caller keeps as scratch while the table is built.
   __device__ __forceinline__ void mark(uint8_t *dummy) {
     uint32_t rw[kMaxBins], eff[kMaxBins];
+    unwrap(rw, eff);
+    bool aligned = false;
+    if (nb == kMaxBins) {
+      uint32_t acc = 0;
+#pragma unroll
+      for (int s = 0; s < kMaxBins; ++s) acc |= rw[s];
+      aligned = !wave_any((acc & 0xF0u) != 0);
+    }
+    if (aligned)
+      mark_rows<true>(rw, eff, dummy);
+    else
+      mark_rows<false>(rw, eff, dummy);
+  }
+
+  // The row's entries and unwrapped bases.
+  __device__ __forceinline__ void unwrap(uint32_t (&rw)[kMaxBins], uint32_t (&eff)[kMaxBins]) const {
 #pragma unroll
     for (int s = 0; s < kMaxBins; ++s) rw[s] = static_cast<uint16_t>(row.r[s]);
     bool wrapped = false;
@@ -323,17 +339,6 @@ struct ByteTables {
       eff[s] = wrapped ? 0x10000u : v;
       prev = v;
     }
-    bool aligned = false;
-    if (nb == kMaxBins) {
-      uint32_t acc = 0;
-#pragma unroll
-      for (int s = 0; s < kMaxBins; ++s) acc |= rw[s];
-      aligned = !wave_any((acc & 0xF0u) != 0);
-    }
-    if (aligned)
-      mark_rows<true>(rw, eff, dummy);
-    else
-      mark_rows<false>(rw, eff, dummy);
   }
 
   template <bool kAligned>
@@ -580,6 +585,211 @@ struct GroupCursor {
     const uint32_t e = lds_dword(((hh >> 18) & 0x3F00u) | tb.lane_at) >> s8;
     o += (e & 7u) + 1u;
     return (e >> 3) & 31u;
+  }
+};
+
+// Two tables for streams with codes of up to 15 bits (n_bins <= 32): the
+// byte table above, and behind it a second one of the same layout indexed by
+// window bits 4 .. 11.  A prefix of the first table that holds longer codes
+// is kEscape there and its window is looked up in the second table, whose
+// entry is (s << 3) | (length - 8).  The two indexes come from the window
+// alone, so both tables are read at once and a long code costs a select.
+//
+// The second table has 256 entries for the 4096 12-bit prefixes: prefix p of
+// the first table takes entries (p % 16) * 16 .. + 15.  A row is `irregular`
+// when the tables cannot hold it (two escaped prefixes with the same p % 16,
+// a base off its place, a code of length 0); such rows take the binary
+// search.  calculate_cdf's rows have their long codes at the ends of the
+// symbol range, so that is rare, but any row is decoded either way: the
+// conditions below are checked symbol by symbol.
+//
+// Build: mark() writes both tables' entries at the symbols' bases, scan()
+// carries them forward (over the whole first table, and within each 16
+// entries of the second), and escapes() then puts kEscape at the prefixes of
+// long codes, after the scan so that it does not spread.
+struct LongTables {
+  static constexpr int kBytes = 2 * ByteTables::kBytes;
+  static constexpr int kMaxBins = ByteTables::kMaxBins;
+  ByteTables one;
+  bool irregular;
+  uint32_t longs;  // bit s: symbol s has its entry in the second table
+  uint32_t eff[kMaxBins];
+
+  // `lds_at` is the LDS address of `lds` (a multiple of ByteTables::kBytes).
+  __device__ __forceinline__ void bind(uint8_t *lds, int lane, uint32_t lds_at = 0) { one.bind(lds, lane, lds_at); }
+
+  __device__ __forceinline__ void clear() {
+    uint32_t *t32 = reinterpret_cast<uint32_t *>(one.tab);
+    for (int d = 0; d < 128; ++d) t32[d * kLanes] = 0;
+  }
+
+  // Writes that do not apply go to `dummy`, so the loop has no branches.
+  __device__ __forceinline__ void mark(uint8_t *dummy) {
+    uint32_t rw[kMaxBins];
+    one.unwrap(rw, eff);
+    uint32_t slots = 0, open = 0xFFFFu;
+    irregular = false;
+    longs = 0;
+#pragma unroll
+    for (int s = 0; s < kMaxBins; ++s) {
+      const uint32_t lo = s == 0 ? 0u : eff[s];  // symbol 0 also owns what lies below its base
+      const uint32_t next = s + 1 < kMaxBins ? eff[s + 1 < kMaxBins ? s + 1 : 0] : 0x10000u;
+      const bool owns = next > lo && s < one.nb;
+      const uint32_t nib = rw[s] & 0xFu;
+      const uint32_t width = next - eff[s];
+      const uint32_t wl = width ? static_cast<uint32_t>(__builtin_clz(width)) - 15u : 0u;
+      const uint32_t len = nib != 0 ? nib : wl;
+      const bool is_short = len - 1u < 8u && !(s == 31 && len == 8u);
+      const bool is_long = owns && !is_short;
+      const bool at_prefix = (lo & 0xFFu) == 0;
+      const uint32_t p = lo >> 8;
+      *(owns && is_short && at_prefix ? one.entry(p) : dummy) =
+          static_cast<uint8_t>((static_cast<uint32_t>(s) << 3) | ((len - 1u) & 7u));
+      *(is_long ? one.entry((lo >> 4) & 0xFFu) + ByteTables::kBytes : dummy) =
+          static_cast<uint8_t>((static_cast<uint32_t>(s) << 3) | ((len - 8u) & 7u));
+      const bool first = p != open;
+      const uint32_t slot = 1u << (p & 15u);
+      const bool bad_short = owns && is_short && !at_prefix;
+      const bool bad_long = is_long && (len - 8u > 7u || next > ((p + 1u) << 8) ||
+                                        (first && (!at_prefix || (slots & slot) != 0)));
+      irregular = irregular || bad_short || bad_long;
+      slots |= is_long ? slot : 0u;
+      open = is_long ? p : open;
+      longs |= is_long ? 1u << s : 0u;
+    }
+  }
+
+  __device__ __forceinline__ void scan() {
+    one.scan(0, 64, 0);
+    uint32_t *t32 = reinterpret_cast<uint32_t *>(one.tab + ByteTables::kBytes);
+    for (int d = 0; d < 64; d += 4) {
+      uint32_t w[4], prev = 0;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) w[k] = t32[(d + k) * kLanes];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        prev = ByteTables::scan_dword(w[k], prev);
+        t32[(d + k) * kLanes] = prev;
+      }
+    }
+  }
+
+  __device__ __forceinline__ void escapes(uint8_t *dummy) {
+#pragma unroll
+    for (int s = 0; s < kMaxBins; ++s) {
+      const uint32_t lo = s == 0 ? 0u : eff[s];
+      *((longs >> s) & 1u ? one.entry(lo >> 8) : dummy) = static_cast<uint8_t>(ByteTables::kEscape);
+    }
+  }
+
+  __device__ __forceinline__ void build(uint8_t *dummy) {
+    mark(dummy);
+    scan();
+    escapes(dummy);
+  }
+
+  // Symbol and length for the 16-bit window v by the binary search over the
+  // row (after one.finish()).
+  __device__ __forceinline__ void search(uint32_t v, int &s, int &len) const {
+    s = 0;
+    for (int step = one.top; step > 0; step >>= 1)
+      if (s + step < one.nb && one.row.base(s + step) <= v) s += step;
+    len = one.row.len(s);
+  }
+};
+
+// Bit cursor over a lane's ring of stream bytes: kBytes bytes of LDS in the
+// block's [dword][lane] layout (the 64 lanes' reads hit 64 banks), holding
+// the raw little-endian dwords of the stream's 16-byte aligned chunks in
+// turn, zeros past the stream's end.  `at` is the LDS address of the lane's
+// column (the ring starts at a multiple of its size of all lanes).  a, b, c
+// and `ahead` are as in BitCursor; the dwords before q are consumed, so a
+// chunk may be written over them.
+struct RingCursor {
+  static constexpr uint32_t kBytes = 256;
+  static constexpr uint32_t kMask = (kBytes / 4 - 1) * kLanes * 4;
+  uint32_t at, a, b, c, ahead, q;
+  int sh;
+
+  __device__ __forceinline__ uint32_t raw(uint32_t o) const { return lds_dword(((o * kLanes) & kMask) | at); }
+  static __device__ __forceinline__ uint32_t be(uint32_t x) { return byte_perm(x, x, 0x00010203u); }
+
+  // Starts at bit `bit` of the chunks (bit 0 the top bit of byte 0).
+  __device__ __forceinline__ void start(uint32_t column, uint32_t bit) {
+    at = column;
+    q = (bit >> 5) << 2;
+    const uint32_t o = bit & 31u;
+    const uint32_t w0 = be(raw(q)), w1 = be(raw(q + 4)), w2 = be(raw(q + 8));
+    sh = static_cast<int>((32u - o) & 31u);
+    a = o ? w0 : 0u;
+    b = o ? w1 : w0;
+    c = o ? w2 : w1;
+    q += o ? 12u : 8u;
+    ahead = raw(q);
+  }
+  __device__ __forceinline__ uint32_t hi() const { return align_bits(a, b, static_cast<uint32_t>(sh)); }
+  __device__ __forceinline__ uint32_t lo() const { return align_bits(b, c, static_cast<uint32_t>(sh)); }
+  // Consumes n < 32 bits.
+  __device__ __forceinline__ void advance(uint32_t n) {
+    sh -= static_cast<int>(n);
+    const bool s = sh < 0;
+    a = s ? b : a;
+    b = s ? c : b;
+    c = s ? be(ahead) : c;
+    sh &= 31;
+    q += s ? 4u : 0u;
+    ahead = raw(q);
+  }
+};
+
+// Two codes per step of LongTables over a ring.  The chain from one code to
+// the next is the two tables' reads (issued together), the select of the
+// entry and its length, and the next code's table addresses, taken from the
+// current code's window bits shifted by that length; the cursor advances
+// once for both codes, under the second one's reads.
+struct PairCursor {
+  RingCursor ring;
+  uint32_t h, w;        // the next 64 bits at the pair's first code
+  uint32_t d1, d2;      // the current code's table dwords (reads in flight)
+  uint32_t s1, s2;      // 8 x its byte in each
+
+  __device__ __forceinline__ void place(uint32_t x) {
+    s1 = (x >> 21) & 0x18u;
+    s2 = (x >> 17) & 0x18u;
+  }
+  // Reads the tables for the code whose window bits start x (24 bits of it
+  // count).
+  __device__ __forceinline__ void read(const LongTables &tb, uint32_t x) {
+    d1 = lds_dword(((x >> 18) & 0x3F00u) | tb.one.lane_at);
+    d2 = lds_dword((((x >> 14) & 0x3F00u) | tb.one.lane_at) + ByteTables::kBytes);
+  }
+  __device__ __forceinline__ void start(const LongTables &tb, uint32_t column, uint32_t bit) {
+    ring.start(column, bit);
+    h = ring.hi();
+    w = ring.lo();
+    place(h);
+    read(tb, h);
+  }
+  // The current code's entry (symbol e >> 3) and length; reads the tables
+  // for the next one.
+  __device__ __forceinline__ uint32_t take(const LongTables &tb, uint32_t x, uint32_t &len) {
+    const uint32_t x1 = (d1 >> s1) & 0xFFu, x2 = (d2 >> s2) & 0xFFu;
+    const bool esc = x1 == ByteTables::kEscape;
+    const uint32_t e = esc ? x2 : x1;
+    len = (e & 7u) + (esc ? 8u : 1u);
+    read(tb, x << len);
+    return e;
+  }
+  __device__ __forceinline__ void pair(const LongTables &tb, uint32_t &e0, uint32_t &e1) {
+    uint32_t l0, l1;
+    e0 = take(tb, h, l0);
+    const uint32_t x = align_bits(h, w, 32u - l0);
+    place(x);
+    e1 = take(tb, x, l1);
+    ring.advance(l0 + l1);
+    h = ring.hi();
+    w = ring.lo();
+    place(h);
   }
 };
 

@@ -57,3 +57,42 @@ def test_encode_chunk_without_tokens_or_streams(F):
         chunk = F.encode_chunk(torch.zeros(shape, dtype=torch.uint8, device=DEV), 16)
         assert chunk.streams.numel() == 0
         assert chunk.lengths.shape == (shape[0], shape[2]) and int(chunk.lengths.sum()) == 0
+
+
+@pytest.mark.parametrize("kind", ["normal", "constant", "skewed"])
+@pytest.mark.parametrize("L,T,C,nb", [
+    (1, 1, 32, 16), (1, 255, 96, 32), (3, 256, 160, 32), (1, 257, 32, 32), (2, 288, 96, 16), (3, 1000, 32, 32),
+    (1, 1023, 64, 32), (5, 289, 96, 31), (1, 4097, 64, 32), (3, 300, 96, 48),
+])
+def test_chunk_round_trip(F, L, T, C, nb, kind):
+    sym = np.minimum(_symbols(L, T, C, nb, T + C + nb, kind), nb - 1).astype(np.uint8)
+    chunk = F.encode_chunk(torch.from_numpy(sym).to(DEV), nb)
+    assert np.array_equal(F.decode_chunk(chunk).cpu().numpy(), sym)
+
+
+# Rows that calculate_cdf does not make (long codes anywhere, bases off their
+# place, zero-length codes) over random streams, some of them short of their
+# symbols, at lengths around the decoder's epochs.
+@pytest.mark.parametrize("T", [257, 260, 287, 288, 289, 1000])
+@pytest.mark.parametrize("kind", ["codes", "sorted", "random"])
+def test_decode_long_foreign_rows(kind, T):
+    from lmcache_amd import c_ops
+
+    L, C, nb = 3, 96, 32
+    rng = np.random.default_rng(T + len(kind))
+    if kind == "codes":
+        sym = _symbols(L, 700, C, nb, T, "skewed")
+        cdf = oc.calculate_cdf(np.minimum(sym, nb - 1).astype(np.uint8), nb)
+    elif kind == "sorted":
+        base = np.sort(rng.integers(0, 4096, size=(L, C, nb + 1)) * 16, axis=2)
+        cdf = (base | rng.integers(0, 16, size=base.shape)).astype(np.uint16).view(np.int16)
+    else:
+        cdf = rng.integers(0, 65536, size=(L, C, nb + 1)).astype(np.uint16).view(np.int16)
+    lens = rng.integers(0, T, size=(L, C)).astype(np.int32)
+    prefix = np.cumsum(lens.reshape(-1), dtype=np.int64).astype(np.int32).reshape(L, C)
+    stream = rng.integers(0, 256, size=int(prefix[-1, -1]), dtype=np.uint8)
+    want = oc.decode(cdf, stream, prefix, T)
+    out = torch.full((L, T, C), 255, dtype=torch.uint8, device=DEV)
+    c_ops.decode_fast_prefsum(torch.from_numpy(cdf).to(DEV), torch.from_numpy(stream).to(DEV),
+                              torch.from_numpy(prefix).to(DEV), out)
+    assert np.array_equal(out.cpu().numpy(), want)
