@@ -338,11 +338,12 @@ int lmc_encode_fast_new(const lmc_tensor *cdf, const lmc_tensor *input_sym,
 
 /* No counterpart in the reference: calculate_cdf and encode_fast_new of one
  * chunk, with what the concatenation of its streams needs.  input: [L, T, C]
- * u8/i8 symbols; cdf: int16 [L, C, n_bins + 1]; rows: u8 [L, C, cap], stream
- * s's bytes up to min(length, cap); lengths: int32 [L, C], bytes per stream;
- * offsets: int64 [2 B + 1], B the number of 64-stream blocks: entry b is
- * where block b's streams (each cut to cap) start in the concatenation,
- * entry B the concatenation's size, the rest scratch.  All are written.
+ * u8/i8 symbols; cdf: int16 [L, C, n_bins + 1]; rows: u8 [L, C, cap], where
+ * each block of 64 streams takes its 64 rows for its streams' bytes one after
+ * the other, each cut to cap; lengths: int32 [L, C], bytes per stream (before
+ * the cut); offsets: int64 [2 B + 1], B the number of blocks: entry b is
+ * where block b's streams start in the concatenation, entry B the
+ * concatenation's size, the rest scratch.  All are written.
  * *total (host) receives the size; the call returns once it is known, with
  * the rows' encoding still running on the stream, and so cannot be captured
  * into a graph. */
@@ -354,8 +355,7 @@ int lmc_cachegen_encode_rows(const lmc_tensor *input, int32_t n_bins,
 
 /* Concatenates the streams lmc_cachegen_encode_rows left in rows, in
  * (layer, channel) order, into streams: u8 [*total]. */
-int lmc_cachegen_pack_rows(const lmc_tensor *rows, const lmc_tensor *lengths,
-                           const lmc_tensor *offsets,
+int lmc_cachegen_pack_rows(const lmc_tensor *rows, const lmc_tensor *offsets,
                            const lmc_tensor *streams, void *stream);
 
 /* Replaces decode_fast_new (csrc/cachegen_kernels.cpp:60-65; pybind

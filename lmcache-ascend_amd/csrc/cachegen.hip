@@ -61,55 +61,6 @@ constexpr int kPrec = 16;
 constexpr int kMaxLen = 12;
 constexpr int kBatch = 32;  // symbol loads in flight per lane
 
-// Copies `count` (>= 1) consecutive int16 CDF entries into LDS with every
-// lane of the block, 8 loads per lane in flight: each load address is
-// clamped into [0, count) so the batch has no branches between its loads.
-template <int LANES>
-__device__ __forceinline__ void stage_rows(const int16_t *__restrict__ src,
-                                           int count, int16_t *dst) {
-  constexpr int kB = 8;
-  for (int i0 = 0; i0 < count; i0 += LANES * kB) {
-    int16_t v[kB];
-#pragma unroll
-    for (int k = 0; k < kB; ++k) {
-      const int i = i0 + k * LANES + static_cast<int>(threadIdx.x);
-      v[k] = src[i < count ? i : count - 1];
-    }
-#pragma unroll
-    for (int k = 0; k < kB; ++k) {
-      const int i = i0 + k * LANES + static_cast<int>(threadIdx.x);
-      if (i < count) dst[i] = v[k];
-    }
-  }
-}
-
-// Unpacks one stream's CDF row (staged in LDS) into the LDS column `col`
-// (stride LANES) as (base << 8) | length per symbol (rules L1-L3).  `cur`
-// is the unwrapped base of symbol s, `next` that of s + 1; once a base has
-// wrapped to 0x10000, every later one is 0x10000 as well.
-template <int LANES>
-__device__ __forceinline__ void unpack_row(const int16_t *row, int nb,
-                                           uint32_t *col) {
-  uint32_t cur_raw = static_cast<uint16_t>(row[0]);
-  uint32_t cur = cur_raw & 0xFFF0u;
-  for (int s = 0; s < nb; ++s) {
-    uint32_t next = 0x10000u, next_raw = 0;
-    if (s + 1 < nb) {
-      next_raw = static_cast<uint16_t>(row[s + 1]);
-      next = next_raw & 0xFFF0u;
-      if (next < cur) next = 0x10000u;
-    }
-    int len = static_cast<int>(cur_raw & 0xFu);
-    if (len == 0) {
-      const uint32_t w = next - cur;
-      if (w != 0) len = kPrec - (31 - __builtin_clz(w));
-    }
-    col[s * LANES] = (cur << 8) | static_cast<uint32_t>(len);
-    cur = next;
-    cur_raw = next_raw;
-  }
-}
-
 // Inclusive prefix sum over the 64 lanes of a wave with DPP moves: shifts
 // by 1, 2, 4 and 8 within each row of 16 lanes, then the last lane of row
 // 0 (row_bcast:15) and of row 1 (row_bcast:31) added to the rows after it.
@@ -579,288 +530,14 @@ __global__ void __launch_bounds__(kCdfThreads)
   }
 }
 
-__device__ __forceinline__ void put_bytes(uint8_t *row, int64_t chunk,
-                                          int64_t at, uint32_t word, int n) {
-  // `n` most significant bytes of `word` at byte offset `at`.
-  for (int b = 0; b < n; ++b)
-    if (at + b < chunk) row[at + b] = static_cast<uint8_t>(word >> (24 - 8 * b));
-}
-
-// Encode: 64 streams per block (one wave); the block's 64 CDF rows are
-// contiguous in memory and staged through LDS with coalesced loads.
-constexpr int kEncLanes = 64;
-
-__global__ void __launch_bounds__(kEncLanes)
-    encode_kernel(const int16_t *__restrict__ cdf,
-                  const uint8_t *__restrict__ in, int T, int C, int nb,
-                  uint8_t *__restrict__ out, int64_t chunk,
-                  int32_t *__restrict__ lens, int tiles, int word_stores) {
-  extern __shared__ uint32_t lds[];
-  // [nb][kEncLanes] u32 code table, then [kEncLanes][nb + 1] int16 rows.
-  uint32_t *col = lds + threadIdx.x;
-  int16_t *stage = reinterpret_cast<int16_t *>(lds + nb * kEncLanes);
-  const int l = blockIdx.x / tiles;
-  const int c0 = (blockIdx.x % tiles) * kEncLanes;
-  const int cnt = C - c0 < kEncLanes ? C - c0 : kEncLanes;
-  const int64_t s0 = static_cast<int64_t>(l) * C + c0;
-  stage_rows<kEncLanes>(cdf + s0 * (nb + 1), cnt * (nb + 1), stage);
-  __syncthreads();
-  if (static_cast<int>(threadIdx.x) >= cnt) return;
-  const int c = c0 + static_cast<int>(threadIdx.x);
-  const int64_t stream = s0 + threadIdx.x;
-  unpack_row<kEncLanes>(stage + threadIdx.x * (nb + 1), nb, col);
-  // Code table: (code << 5) | length.
-  for (int s = 0; s < nb; ++s) {
-    const uint32_t e = col[s * kEncLanes];
-    const uint32_t len = e & 0xFFu;
-    const uint32_t base = e >> 8;
-    const uint32_t code =
-        len ? (base >> (kPrec - len)) & ((1u << len) - 1u) : 0u;
-    col[s * kEncLanes] = (code << 5) | len;
-  }
-  uint8_t *row = out + stream * chunk;
-  const uint8_t *p = in + static_cast<int64_t>(l) * T * C + c;
-  uint64_t acc = 0;
-  int nbits = 0;
-  int64_t wpos = 0;  // bytes already written
-  for (int t0 = 0; t0 < T; t0 += kBatch) {
-    // All symbol loads of the batch in flight, then all table lookups, then
-    // the serial bit packing.
-    uint32_t e[kBatch];
-#pragma unroll
-    for (int i = 0; i < kBatch; ++i)
-      e[i] = t0 + i < T ? p[static_cast<int64_t>(t0 + i) * C] : 0xFFu;
-#pragma unroll
-    for (int i = 0; i < kBatch; ++i)
-      e[i] = e[i] < static_cast<uint32_t>(nb) ? col[e[i] * kEncLanes] : 0u;
-#pragma unroll
-    for (int i = 0; i < kBatch; ++i) {
-      const int len = static_cast<int>(e[i] & 31u);
-      acc = (acc << len) | (e[i] >> 5);
-      nbits += len;
-      if (nbits >= 32) {
-        const uint32_t word = static_cast<uint32_t>(acc >> (nbits - 32));
-        if (word_stores && wpos + 4 <= chunk)
-          cg_st(reinterpret_cast<uint32_t *>(row + wpos), __builtin_bswap32(word));
-        else
-          put_bytes(row, chunk, wpos, word, 4);
-        wpos += 4;
-        nbits -= 32;
-      }
-    }
-  }
-  if (nbits > 0) {
-    const uint32_t tail = static_cast<uint32_t>(acc << (32 - nbits));
-    put_bytes(row, chunk, wpos, tail, (nbits + 7) >> 3);
-  }
-  lens[stream] = static_cast<int32_t>(wpos + ((nbits + 7) >> 3));
-}
-
-// Wave encode (T <= 256): 64 streams per block, four waves; a wave encodes
-// one whole stream at a time, so no lane walks a serial chain of symbols.
-//   1. The block's CDF rows and symbols are staged into LDS with coalesced
-//      loads, all issued before any LDS store; the symbols are transposed
-//      to one row per stream (an odd number of words per row).
-//   2. Per stream, lane s builds symbol s's (code, length) from the staged
-//      row (the wrap of rule L2 found with a ballot), and lane j takes the
-//      stream's tokens 4j .. 4j + 3 with one LDS read and looks their codes
-//      up with cross-lane shuffles.
-//   3. The lane's four codes become one run of at most 64 bits; an
-//      exclusive prefix sum over the wave gives the run's bit offset, and
-//      the run is ORed into the (at most three) words it touches of the
-//      wave's LDS bit buffer.
-//   4. Lane k stores word k of the row: one coalesced store per 256 bytes,
-//      and only bytes below min(chunk, stream length), as the single-lane
-//      encoder writes them.
-constexpr int kEncWaves = 4;
-#ifndef LMC_ENC_SPLIT
-#define LMC_ENC_SPLIT 1     // split encoder for full 64-channel blocks
-#endif
-#ifndef LMC_ENC_PIECES
-#define LMC_ENC_PIECES 8    // waves (token pieces) per block of the split encoder
-#endif
-constexpr int kEncPieces = LMC_ENC_PIECES;
-constexpr int kEncTileThreads = kEncLanes * kEncWaves;
-constexpr int kEncTileMaxT = 4 * kEncLanes;
-
-__device__ __forceinline__ void put_word(uint8_t *row, int64_t chunk, uint32_t idx, uint32_t word,
-                                         int n, int word_stores) {
-  const int64_t at = static_cast<int64_t>(idx) * 4;
-  if (n == 4 && word_stores && at + 4 <= chunk)
-    cg_st(reinterpret_cast<uint32_t *>(row + at), __builtin_bswap32(word));
-  else
-    put_bytes(row, chunk, at, word, n);
-}
-
-// Encode staging: the block's CDF rows (contiguous in memory) into `stage`
-// and its symbols, transposed to one row of `sym_stride` words per stream,
-// into `tile`; every global load of a thread is issued before its LDS
-// stores.  With `vec_tile` (a full block of 64 channels, C % 16 == 0 and a
-// 16-byte aligned input) each token's 64 symbols are four 16-byte loads.
-template <int NT>
-__device__ __forceinline__ void enc_stage(const int16_t *__restrict__ cdf,
-                                          const uint8_t *__restrict__ in, int T, int C, int nb,
-                                          int l, int c0, int cnt, int64_t s0, int vec_tile,
-                                          int sym_stride, int16_t *stage, uint8_t *tile) {
-  const int tid = static_cast<int>(threadIdx.x);
-  const int16_t *rsrc = cdf + s0 * (nb + 1);
-  const int rcount = cnt * (nb + 1);
-  constexpr int kR = 4;
-  int16_t rv[kR];
-  int ri[kR];
-#pragma unroll
-  for (int k = 0; k < kR; ++k) {
-    const int i = k * NT + tid;
-    ri[k] = i < rcount ? i : rcount - 1;
-    rv[k] = rsrc[ri[k]];
-  }
-  const uint8_t *src = in + static_cast<int64_t>(l) * T * C + c0;
-  const int pieces = T * 4;
-  const int row_bytes = sym_stride * 4;
-  if (vec_tile && cnt == kEncLanes) {
-    constexpr int kV = (4 * kEncTileMaxT + NT - 1) / NT;  // 16-byte pieces per thread (T <= 256)
-    uint4 v[kV];
-    int pi[kV];
-#pragma unroll
-    for (int k = 0; k < kV; ++k) {
-      const int i = k * NT + tid;
-      pi[k] = i < pieces ? i : pieces - 1;
-      v[k] = *reinterpret_cast<const uint4 *>(src + static_cast<int64_t>(pi[k] >> 2) * C + (pi[k] & 3) * 16);
-    }
-#pragma unroll
-    for (int k = 0; k < kV; ++k) {
-      uint8_t *d = tile + (pi[k] & 3) * 16 * row_bytes + (pi[k] >> 2);
-      const uint32_t w[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
-#pragma unroll
-      for (int j = 0; j < 16; ++j) d[j * row_bytes] = static_cast<uint8_t>(w[j >> 2] >> (8 * (j & 3)));
-    }
-  } else {
-    for (int i = tid; i < T * kEncLanes; i += NT) {
-      const int c = i % kEncLanes, t = i / kEncLanes;
-      tile[c * row_bytes + t] = c < cnt ? src[static_cast<int64_t>(t) * C + c] : 0;
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < kR; ++k) stage[ri[k]] = rv[k];
-  for (int i = kR * NT + tid; i < rcount; i += NT) stage[i] = rsrc[i];
-}
-
-__global__ void __launch_bounds__(kEncTileThreads)
-    encode_wave_kernel(const int16_t *__restrict__ cdf,
-                       const uint8_t *__restrict__ in, int T, int C, int nb,
-                       uint8_t *__restrict__ out, int64_t chunk,
-                       int32_t *__restrict__ lens, int tiles, int word_stores, int vec_tile,
-                       int sym_stride, int cap_words) {
-  // [64][nb + 1] int16 rows | [64][sym_stride] u32 symbols | [4][2][cap_words] u32 bits
-  extern __shared__ uint32_t lds[];
-  const int tid = static_cast<int>(threadIdx.x);
-  const int wv = tid / kEncLanes;
-  const int lane = tid % kEncLanes;
-  const int l = blockIdx.x / tiles;
-  const int c0 = (blockIdx.x % tiles) * kEncLanes;
-  const int cnt = C - c0 < kEncLanes ? C - c0 : kEncLanes;
-  const int64_t s0 = static_cast<int64_t>(l) * C + c0;
-  int16_t *stage = reinterpret_cast<int16_t *>(lds);
-  const int rows_words = ((nb + 1) * kEncLanes * 2 + 15) / 16 * 4;
-  uint8_t *tile = reinterpret_cast<uint8_t *>(lds + rows_words);
-  uint32_t *bitbuf = lds + rows_words + kEncLanes * sym_stride + 2 * wv * cap_words;
-
-  // 1. Rows and symbols: every load of the thread, then the LDS stores.
-  enc_stage<kEncTileThreads>(cdf, in, T, C, nb, l, c0, cnt, s0, vec_tile, sym_stride, stage, tile);
-  __syncthreads();
-
-  // Two streams per step (st and st + kEncWaves), so their LDS round trips
-  // overlap.
-  for (int st0 = wv; st0 < cnt; st0 += 2 * kEncWaves) {
-    int stv[2];
-    bool on[2];
-    int entry[2];
-    uint32_t word[2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      stv[j] = st0 + j * kEncWaves;
-      on[j] = stv[j] < cnt;
-      // 2. Code table: lane s holds symbol s's (code << 5) | length.
-      const int16_t *row = stage + (on[j] ? stv[j] : st0) * (nb + 1);
-      const uint32_t raw = lane < nb ? static_cast<uint16_t>(row[lane]) : 0u;
-      const uint32_t raw_n = lane + 1 < nb ? static_cast<uint16_t>(row[lane + 1]) : 0u;
-      const bool dec = lane + 1 < nb && (raw_n & 0xFFF0u) < (raw & 0xFFF0u);
-      const uint64_t decs = __ballot(dec);
-      const int wrap = decs ? __builtin_ctzll(decs) + 1 : nb;  // bases from here on are 0x10000
-      const uint32_t base = lane < wrap ? (raw & 0xFFF0u) : 0x10000u;
-      const uint32_t next = lane + 1 < wrap ? (raw_n & 0xFFF0u) : 0x10000u;
-      uint32_t len = raw & 0xFu;
-      if (len == 0 && next != base) len = kPrec - (31 - __builtin_clz(next - base));
-      const uint32_t code = len ? (base >> (kPrec - len)) & ((1u << len) - 1u) : 0u;
-      entry[j] = lane < nb ? static_cast<int>((code << 5) | len) : 0;
-      // Tokens 4 * lane .. + 3.
-      word[j] = (on[j] && 4 * lane < T)
-                    ? reinterpret_cast<const uint32_t *>(tile)[stv[j] * sym_stride + lane] : 0u;
-    }
-    uint64_t run[2];
-    uint32_t run_bits[2], pos[2], total[2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      run[j] = 0;
-      run_bits[j] = 0;
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const uint32_t v = (word[j] >> (8 * b)) & 0xFFu;
-        const uint32_t e = static_cast<uint32_t>(__shfl(entry[j], static_cast<int>(v & 63u)));
-        const bool ok = on[j] && 4 * lane + b < T && v < static_cast<uint32_t>(nb);
-        const uint32_t n = ok ? (e & 31u) : 0u;
-        run[j] = (run[j] << n) | (ok ? (e >> 5) : 0u);
-        run_bits[j] += n;
-      }
-    }
-    // 3. Exclusive prefix sums of the runs' lengths.
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const uint32_t incl = wave_incl_scan(run_bits[j]);
-      pos[j] = incl - run_bits[j];
-      total[j] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(incl), kEncLanes - 1));
-    }
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-      for (int k = lane; k < cap_words; k += kEncLanes) bitbuf[j * cap_words + k] = 0;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      if (!run_bits[j]) continue;
-      uint32_t *bb = bitbuf + j * cap_words;
-      const uint64_t a = run[j] << (64 - run_bits[j]);  // top-aligned
-      const uint32_t hi = static_cast<uint32_t>(a >> 32), lo = static_cast<uint32_t>(a);
-      const uint32_t w0 = pos[j] >> 5, sh = pos[j] & 31u;
-      if (w0 < static_cast<uint32_t>(cap_words)) atomicOr(&bb[w0], hi >> sh);
-      if (sh + run_bits[j] > 32 && w0 + 1 < static_cast<uint32_t>(cap_words))
-        atomicOr(&bb[w0 + 1], sh ? (hi << (32 - sh)) | (lo >> sh) : lo);
-      if (sh + run_bits[j] > 64 && w0 + 2 < static_cast<uint32_t>(cap_words))
-        atomicOr(&bb[w0 + 2], lo << (32 - sh));
-    }
-    // 4. The rows.
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      if (!on[j]) continue;
-      const int64_t tbytes = (total[j] + 7) >> 3;
-      int64_t nbytes = tbytes < chunk ? tbytes : chunk;
-      nbytes = nbytes < 4 * static_cast<int64_t>(cap_words) ? nbytes : 4 * static_cast<int64_t>(cap_words);
-      uint8_t *orow = out + (s0 + stv[j]) * chunk;
-      for (int k = lane; static_cast<int64_t>(k) * 4 < nbytes; k += kEncLanes) {
-        const int64_t left = nbytes - 4 * static_cast<int64_t>(k);
-        put_word(orow, chunk, static_cast<uint32_t>(k), bitbuf[j * cap_words + k],
-                 left >= 4 ? 4 : static_cast<int>(left), word_stores);
-      }
-      if (lane == 0) lens[s0 + stv[j]] = static_cast<int32_t>(tbytes);
-    }
-  }
-}
-
-// Split encode (T <= 256, a full block of 64 channels): 64 streams per
-// block and PIECES waves, wave w taking tokens [w * Q, (w + 1) * Q) of every
-// stream (Q = 256 / PIECES), lane s stream s.  Each lane walks a serial
-// chain of only Q codes, and every wave instruction works for 64 streams.
+// Encode: 64 streams per block (consecutive ones, whatever their layer) and
+// PIECES waves, kEncTokens tokens at a time, wave w taking tokens
+// [w * Q, (w + 1) * Q) of every stream (Q = kEncTokens / PIECES), lane s
+// stream s.  Each lane walks a serial chain of only Q codes, and every wave
+// instruction works for 64 streams.
 //   1. The block's CDF rows (contiguous in memory) are staged with dword
 //      loads; its symbols are staged untransposed, [token][64 channels]
-//      bytes, with 16-byte stores (tokens T .. 255 read as 0xFF, not
+//      bytes, with 16-byte stores (tokens past T read as 0xFF, not
 //      coded).  Lane s then reads token t's symbol at t * 64 + s: the 64
 //      lanes read 16 consecutive words.
 //   2. Code table in LDS, [symbol][stream] words of (code << 11) | length
@@ -874,14 +551,38 @@ __global__ void __launch_bounds__(kEncTileThreads)
 //      lengths (the sum of the entries' low 11 bits: at most 64 x 15 bits,
 //      so no carry reaches the code field).  The piece lengths of a stream
 //      give each piece its bit offset.
-//   4. The staged data is dead; the same LDS holds one zeroed bit row per
-//      stream (2T bytes + a word: codes are at most 15 bits), and each lane
-//      ORs its codes in as runs of at most 32 bits: four codes per run when
-//      no code of the block is longer than 8 bits, else two.
-//   5. Rows leave as in the wave encoder: wave w stores the rows of streams
-//      w, w + PIECES, ..., lane k word k, only bytes below
-//      min(chunk, stream length).
-template <int PIECES>
+//   4. The staged symbols are dead; the same LDS holds the zeroed bits, and
+//      each lane ORs its codes in as runs of at most 32 bits: four codes per
+//      run when no code of the block is longer than 8 bits, else two.
+//   5. The bits leave as dwords, and the last bytes of a stream one by one.
+//
+// The streams' places: rows of `chunk` bytes (place 0), or one after the
+// other from the block's first row on, each cut to `chunk` bytes (place 1; a
+// later copy then moves whole blocks).  Three forms:
+//   kRows   place 0, at most kEncTokens tokens.
+//   kImage  place 1, at most kEncTokens tokens, no stream cut: the streams'
+//           bits lie one after the other in LDS as well, so only the bytes
+//           in use are cleared and they leave as 16-byte stores.
+//   kLong   the rest.  Steps 1, 3, 4 and 5 once per kEncTokens, the last
+//           dword of a stream carried over, the next symbols loaded under
+//           the present ones' coding.  A stream's bits are laid out in LDS
+//           from its address modulo 4, so LDS dwords are memory dwords
+//           wherever it starts; with place 1 its length is read from `lens`.
+//           It takes 94 registers, which leaves two blocks on a CU where the
+//           other forms have four (kRows' work in it: 22.2 us against 16.6).
+//
+// Measured on MI355X, 64 planes x 256 tokens x 1024 channels (32 bins in the
+// first 10 planes, 16 in the others): kRows 16.9 us, kImage 12.3 us; 56
+// planes x 1000 tokens x 256 channels, kLong 22 us, against 128 us for a lane
+// per stream walking all its tokens.
+enum class EncMode { kRows, kImage, kLong };
+constexpr int kEncLanes = 64;
+#ifndef LMC_ENC_PIECES
+#define LMC_ENC_PIECES 8    // waves (token pieces) per block of the encoder
+#endif
+constexpr int kEncPieces = LMC_ENC_PIECES;
+constexpr int kEncTokens = 256;
+
 __device__ __forceinline__ void enc_append(uint32_t *brow, uint32_t &pos, uint32_t run, uint32_t n) {
   // `run` holds n <= 32 bits (0 when n is 0); its top-aligned form is ORed
   // into the one or two words it touches.
@@ -892,72 +593,107 @@ __device__ __forceinline__ void enc_append(uint32_t *brow, uint32_t &pos, uint32
   pos += n;
 }
 
-template <int PIECES>
+// LDS of the encoder, in words: [64][nb + 1] int16 rows and [256][64] u8
+// symbols, and over them the bits (64 rows of row_words, or the block's bits
+// one stream after the other); [nb + 1][64] u32 codes, inside the bits' area
+// when the whole chunk is coded at once and after it otherwise; then
+// [PIECES][64] piece lengths, the long-code flag and [64] u64 decrease masks.
+struct EncLds {
+  int rows_words, tab_at, row_words, plen_at, bytes;
+};
+inline EncLds enc_lds(int64_t T, int nb) {
+  EncLds e;
+  const int tokens = static_cast<int>(std::min<int64_t>(T, kEncTokens));
+  e.rows_words = ((nb + 1) * kEncLanes * 2 + 15) / 16 * 4;
+  // Codes are at most 15 bits; a carried dword or a lead of 3 bytes before
+  // them, and a partial dword after.  An odd number of words, so that the
+  // streams' rows start in different banks.
+  e.row_words = ((tokens * 15 + 31) / 32 + 2) | 1;
+  const int staged = e.rows_words + kEncTokens * kEncLanes / 4;
+  const int bits = kEncLanes * e.row_words;
+  const int codes = (nb + 1) * kEncLanes;
+  e.tab_at = T > kEncTokens ? std::max(staged, bits) : staged;
+  e.plen_at = std::max(e.tab_at + codes, bits);
+  e.bytes = 4 * (((e.plen_at + kEncPieces * kEncLanes + 2) & ~1) + 2 * kEncLanes);
+  return e;
+}
+
+template <int PIECES, EncMode MODE>
 __global__ void __launch_bounds__(64 * PIECES)
-    encode_split_kernel(const int16_t *__restrict__ cdf,
-                        const uint8_t *__restrict__ in, int T, int C, int nb,
-                        uint8_t *__restrict__ out, int64_t chunk,
-                        int32_t *__restrict__ lens, int tiles, int word_stores, int row_words,
-                        int stage_words) {
+    encode_split_kernel(const int16_t *__restrict__ cdf, const uint8_t *__restrict__ in, int T, int C, int nb,
+                        int64_t n_streams, uint8_t *__restrict__ out, int64_t chunk, int32_t *__restrict__ lens,
+                        int place, int vec_tile, int rows_dw, const EncLds at) {
   constexpr int NT = 64 * PIECES;
-  constexpr int Q = kEncTileMaxT / PIECES;  // tokens per piece
-  // Phase 1: [64][nb + 1] int16 rows | [256][64] u8 symbols | [nb + 1][64] u32 codes
-  // Phase 2: [64][row_words] u32 bit rows (over phase 1)
-  // Always:  [PIECES][64] u32 piece lengths, the long-code flag and [64] u64
-  //          decrease masks, after both
+  constexpr int Q = kEncTokens / PIECES;  // tokens per piece
+  constexpr bool IMAGE = MODE == EncMode::kImage, LONG = MODE == EncMode::kLong;
   extern __shared__ uint32_t lds[];
   typedef unsigned int w4 __attribute__((ext_vector_type(4)));
   const int tid = static_cast<int>(threadIdx.x);
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
-  const int l = blockIdx.x / tiles;
-  const int c0 = (blockIdx.x % tiles) * kEncLanes;
-  const int64_t s0 = static_cast<int64_t>(l) * C + c0;
-  const int rows_words = ((nb + 1) * kEncLanes * 2 + 15) / 16 * 4;
+  const int64_t s0 = static_cast<int64_t>(blockIdx.x) * kEncLanes;
+  const int cnt = n_streams - s0 < kEncLanes ? static_cast<int>(n_streams - s0) : kEncLanes;
   int16_t *stage = reinterpret_cast<int16_t *>(lds);
-  uint8_t *tile = reinterpret_cast<uint8_t *>(lds + rows_words);
-  uint32_t *tab = lds + rows_words + kEncTileMaxT * kEncLanes / 4;
+  uint8_t *tile = reinterpret_cast<uint8_t *>(lds + at.rows_words);
+  uint32_t *tab = lds + at.tab_at;
   uint32_t *bits = lds;
-  uint32_t *plen = lds + stage_words;
+  uint32_t *plen = lds + at.plen_at;
   uint32_t *long_flag = plen + PIECES * kEncLanes;
-  uint64_t *dmask = reinterpret_cast<uint64_t *>(lds + ((stage_words + PIECES * kEncLanes + 2) & ~1));
+  uint64_t *dmask = reinterpret_cast<uint64_t *>(lds + ((at.plen_at + PIECES * kEncLanes + 2) & ~1));
 
   // 1. Staging: every global load of the thread, then its LDS stores.  The
-  //    block's rows start at an even entry (s0 is a multiple of 64) and hold
-  //    an even number of entries, so they are whole dwords.
+  //    thread stages one 16-byte piece of a token (vec_tile; it lies in one
+  //    layer, C % 16 == 0) or one byte.
+  const int col = vec_tile ? 16 * (tid & 3) : lane;
+  const bool col_on = col < cnt;
+  const uint8_t *src = stream_column(in, s0 + (col_on ? col : 0), T, C);
+  constexpr int kV = (4 * kEncTokens + NT - 1) / NT;  // 16-byte pieces per thread
+  const w4 none = {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu};
+  w4 v[kV];
+  auto load_symbols = [&](int t0) {
+#pragma unroll
+    for (int k = 0; k < kV; ++k) {
+      const int t = t0 + k * (NT / 4) + (tid >> 2);
+      v[k] = gload_nt(reinterpret_cast<const w4 *>(src + static_cast<int64_t>(t < T ? t : T - 1) * C));
+    }
+  };
+  auto store_symbols = [&](int t0) {
+    if (vec_tile) {
+#pragma unroll
+      for (int k = 0; k < kV; ++k)  // every piece of the 256 x 64 tile, in or past T
+        reinterpret_cast<w4 *>(tile)[k * NT + tid] =
+            col_on && t0 + k * (NT / 4) + (tid >> 2) < T ? v[k] : none;
+    } else {
+      for (int t = wv; t < kEncTokens; t += PIECES)
+        tile[t * kEncLanes + lane] =
+            col_on && t0 + t < T ? src[static_cast<int64_t>(t0 + t) * C] : static_cast<uint8_t>(0xFF);
+    }
+  };
   {
-    const uint32_t *rsrc = reinterpret_cast<const uint32_t *>(cdf + s0 * (nb + 1));
-    const int rcount = kEncLanes * (nb + 1) / 2;
-    constexpr int kR = (kEncLanes * 33 / 2 + NT - 1) / NT;  // row dwords per thread for nb <= 32
-    uint32_t rv[kR];
-    int ri[kR];
+    const int rcount = cnt * (nb + 1);
+    if (rows_dw && cnt == kEncLanes) {
+      const uint32_t *rsrc = reinterpret_cast<const uint32_t *>(cdf + s0 * (nb + 1));
+      constexpr int kR = (kEncLanes * 33 / 2 + NT - 1) / NT;  // row dwords per thread for nb <= 32
+      uint32_t rv[kR];
+      int ri[kR];
 #pragma unroll
-    for (int k = 0; k < kR; ++k) {
-      const int i = k * NT + tid;
-      ri[k] = i < rcount ? i : rcount - 1;
-      rv[k] = gload_nt(rsrc + ri[k]);
+      for (int k = 0; k < kR; ++k) {
+        const int i = k * NT + tid;
+        ri[k] = i < rcount / 2 ? i : rcount / 2 - 1;
+        rv[k] = gload_nt(rsrc + ri[k]);
+      }
+      if (vec_tile && T > 0) load_symbols(0);
+      store_symbols(0);
+      uint32_t *rdst = reinterpret_cast<uint32_t *>(stage);
+#pragma unroll
+      for (int k = 0; k < kR; ++k) rdst[ri[k]] = rv[k];
+      for (int i = kR * NT + tid; i < rcount / 2; i += NT) rdst[i] = rsrc[i];
+    } else {
+      if (vec_tile && T > 0) load_symbols(0);
+      store_symbols(0);
+      for (int i = tid; i < kEncLanes * (nb + 1); i += NT)
+        stage[i] = i < rcount ? cdf[s0 * (nb + 1) + i] : static_cast<int16_t>(0);
     }
-    const uint8_t *src = in + static_cast<int64_t>(l) * T * C + c0;
-    constexpr int kV = (4 * kEncTileMaxT + NT - 1) / NT;  // 16-byte pieces per thread
-    const int pieces = T * 4;
-    w4 v[kV];
-    int pi[kV];
-#pragma unroll
-    for (int k = 0; k < kV; ++k) {
-      const int i = k * NT + tid;
-      pi[k] = i < pieces ? i : pieces - 1;
-      v[k] = gload_nt(reinterpret_cast<const w4 *>(src + static_cast<int64_t>(pi[k] >> 2) * C + (pi[k] & 3) * 16));
-    }
-    const w4 none = {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu};
-#pragma unroll
-    for (int k = 0; k < kV; ++k) {
-      const int i = k * NT + tid;  // every piece of the 256 x 64 tile, in or past T
-      reinterpret_cast<w4 *>(tile)[i] = i < pieces ? v[k] : none;
-    }
-    uint32_t *rdst = reinterpret_cast<uint32_t *>(stage);
-#pragma unroll
-    for (int k = 0; k < kR; ++k) rdst[ri[k]] = rv[k];
-    for (int i = kR * NT + tid; i < rcount; i += NT) rdst[i] = rsrc[i];
     if (tid == 0) *long_flag = 0u;
     if (tid < kEncLanes) dmask[tid] = 0u;
   }
@@ -1014,41 +750,69 @@ __global__ void __launch_bounds__(64 * PIECES)
   __syncthreads();
   const bool long_codes = *long_flag != 0u;
 
-  // 3. Lookups into registers, and the piece's length.
-  uint32_t e[Q];
-  uint32_t sum = 0;
-  {
-    const uint8_t *scol = tile + wv * Q * kEncLanes + lane;
-    const uint32_t *tcol = tab + lane;
-#pragma unroll
-    for (int i = 0; i < Q; ++i) {
-      const uint32_t v = scol[i * kEncLanes];
-      e[i] = tcol[(v < static_cast<uint32_t>(nb) ? v : static_cast<uint32_t>(nb)) * kEncLanes];
-    }
-#pragma unroll
-    for (int i = 0; i < Q; i += 2) sum += e[i] + e[i + 1];
+  // Where the lane's stream goes: its bytes start `dst`, the LDS bits at
+  // bit 8 * (dst % 4); `bit` is the bits of the present dword already taken
+  // (the lead, then the carry), `carry` their value, `first` the index of
+  // that dword from dst - dst % 4.
+  uint8_t *block_out = out + s0 * chunk;
+  int64_t off = static_cast<int64_t>(lane) * chunk;
+  if (LONG && place == 1) {
+    const int64_t len = lane < cnt ? lens[s0 + lane] : 0;
+    const uint32_t kept = static_cast<uint32_t>(len < chunk ? len : chunk);
+    const uint32_t lo = wave_incl_scan(kept & 0xFFFFu), hi = wave_incl_scan(kept >> 16);
+    off = (static_cast<int64_t>(hi) << 16) + lo - kept;
   }
-  plen[wv * kEncLanes + lane] = sum & 0x7FFu;
-  __syncthreads();
+  const uint32_t lead = LONG ? static_cast<uint32_t>(reinterpret_cast<uintptr_t>(block_out + off) & 3) : 0u;
+  uint32_t bit = 8u * lead, carry = 0, first = 0;
 
-  // 4. Bit rows: zeroed, then each piece ORed in at its offset.
-  {
-    const int n4 = (kEncLanes * row_words) / 4;
-    w4 *b4 = reinterpret_cast<w4 *>(bits);
-    const w4 z = {0u, 0u, 0u, 0u};
-    for (int i = tid; i < n4; i += NT) b4[i] = z;
-    for (int i = 4 * n4 + tid; i < kEncLanes * row_words; i += NT) bits[i] = 0u;
-  }
-  uint32_t pos = 0, total = 0;
+  int t0 = 0;
+  do {
+    const bool more = LONG && t0 + kEncTokens < T;
+    // 3. Lookups into registers, and the piece's length.
+    uint32_t e[Q];
+    uint32_t sum = 0;
+    {
+      const uint8_t *scol = tile + wv * Q * kEncLanes + lane;
+      const uint32_t *tcol = tab + lane;
 #pragma unroll
-  for (int w = 0; w < PIECES; ++w) {
-    const uint32_t n = plen[w * kEncLanes + lane];
-    pos += w < wv ? n : 0u;
-    total += n;
-  }
-  __syncthreads();
-  {
-    uint32_t *brow = bits + lane * row_words;
+      for (int i = 0; i < Q; ++i) {
+        const uint32_t x = scol[i * kEncLanes];
+        e[i] = tcol[(x < static_cast<uint32_t>(nb) ? x : static_cast<uint32_t>(nb)) * kEncLanes];
+      }
+#pragma unroll
+      for (int i = 0; i < Q; i += 2) sum += e[i] + e[i + 1];
+    }
+    plen[wv * kEncLanes + lane] = sum & 0x7FFu;
+    if (more && vec_tile) load_symbols(t0 + kEncTokens);
+    __syncthreads();
+
+    // 4. The bits: cleared, then each piece ORed in at its offset.
+    uint32_t pos = bit, total = bit;
+#pragma unroll
+    for (int w = 0; w < PIECES; ++w) {
+      const uint32_t n = plen[w * kEncLanes + lane];
+      pos += w < wv ? n : 0u;
+      total += n;
+    }
+    uint32_t *brow = bits + lane * at.row_words;
+    uint32_t words = static_cast<uint32_t>(kEncLanes * at.row_words);
+    uint32_t image_bytes = 0;
+    if (IMAGE) {
+      const uint32_t nbytes = (total + 7) >> 3;
+      const uint32_t incl = wave_incl_scan(nbytes);
+      pos += 8u * (incl - nbytes);
+      brow = bits;
+      image_bytes = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(incl), kEncLanes - 1));
+      words = (image_bytes + 15) / 16 * 4;
+    }
+    {
+      w4 *b4 = reinterpret_cast<w4 *>(bits);
+      const w4 z = {0u, 0u, 0u, 0u};
+      for (uint32_t i = tid; i < words / 4; i += NT) b4[i] = z;
+      for (uint32_t i = words / 4 * 4 + tid; i < words; i += NT) bits[i] = 0u;
+    }
+    __syncthreads();
+    if (LONG && wv == 0 && carry != 0) atomicOr(brow, carry);
     if (!long_codes) {
       // Codes of at most 8 bits: four to a run.
 #pragma unroll
@@ -1058,34 +822,91 @@ __global__ void __launch_bounds__(64 * PIECES)
         run = (run << (e[i + 2] & 31u)) | (e[i + 2] >> 11);
         run = (run << (e[i + 3] & 31u)) | (e[i + 3] >> 11);
         const uint32_t n = (e[i] + e[i + 1] + e[i + 2] + e[i + 3]) & 0x7FFu;
-        enc_append<PIECES>(brow, pos, run, n);
+        enc_append(brow, pos, run, n);
       }
     } else {
 #pragma unroll
       for (int i = 0; i < Q; i += 2) {
         const uint32_t run = ((e[i] >> 11) << (e[i + 1] & 31u)) | (e[i + 1] >> 11);
         const uint32_t n = (e[i] + e[i + 1]) & 0x7FFu;  // <= 30
-        enc_append<PIECES>(brow, pos, run, n);
+        enc_append(brow, pos, run, n);
       }
     }
-  }
-  if (wv == 0) lens[s0 + lane] = static_cast<int32_t>((total + 7) >> 3);
-  __syncthreads();
+    if (IMAGE) {
+      if (wv == 0 && lane < cnt) lens[s0 + lane] = static_cast<int32_t>((total + 7) >> 3);
+      __syncthreads();
+      // 5. The block's bytes (its place holds 64 * chunk bytes, a multiple
+      //    of 16).
+      for (uint32_t i = tid; i < words / 4; i += NT) {
+        w4 x = reinterpret_cast<const w4 *>(bits)[i];
+        x.x = __builtin_bswap32(x.x);
+        x.y = __builtin_bswap32(x.y);
+        x.z = __builtin_bswap32(x.z);
+        x.w = __builtin_bswap32(x.w);
+        cg_st(reinterpret_cast<w4 *>(block_out) + i, x);
+      }
+      return;
+    }
+    if (!LONG) {
+      if (wv == 0 && lane < cnt) lens[s0 + lane] = static_cast<int32_t>((total + 7) >> 3);
+      __syncthreads();
+      // 5. A wave per stream: full words as dword stores where the rows start
+      //    on dwords, the bytes of a last partial word by one lane each.
+      const bool word_stores = chunk % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 3) == 0;
+      for (int st = wv; st < cnt; st += PIECES) {
+        const uint32_t tb = __builtin_amdgcn_readlane(static_cast<int>(total), st);  // wave-uniform
+        const uint32_t tbytes = (tb + 7) >> 3;
+        const uint32_t nbytes = chunk < static_cast<int64_t>(tbytes) ? static_cast<uint32_t>(chunk) : tbytes;
+        uint8_t *orow = block_out + st * chunk;
+        const uint32_t *sb = bits + st * at.row_words;
+        const uint32_t nw = word_stores ? nbytes >> 2 : 0u;
+        for (uint32_t k = lane; k < nw; k += kEncLanes)
+          cg_st(reinterpret_cast<uint32_t *>(orow) + k, __builtin_bswap32(sb[k]));
+        for (uint32_t b = 4 * nw + lane; b < nbytes; b += kEncLanes)
+          orow[b] = static_cast<uint8_t>(sb[b >> 2] >> (24 - 8 * (b & 3u)));
+      }
+      return;
+    }
+    // Bytes of the stream from dst - lead: [lead, end) may be stored.
+    const int64_t bytes = static_cast<int64_t>(first) * 4 + ((total + 7) >> 3);
+    const int64_t room = lead + chunk;
+    const int64_t end = more || bytes > room ? room : bytes;
+    if (wv == 0 && lane < cnt && !more) lens[s0 + lane] = static_cast<int32_t>(bytes - lead);
+    __syncthreads();
 
-  // 5. The rows: full words as dword stores, the bytes of a last partial
-  //    word by one lane each (a stream is at most 2T + 1 <= 513 bytes).
-  for (int st = wv; st < kEncLanes; st += PIECES) {
-    const uint32_t tb = __builtin_amdgcn_readlane(static_cast<int>(total), st);  // wave-uniform
-    const uint32_t tbytes = (tb + 7) >> 3;
-    const uint32_t nbytes = chunk < static_cast<int64_t>(tbytes) ? static_cast<uint32_t>(chunk) : tbytes;
-    uint8_t *orow = out + (s0 + st) * chunk;
-    const uint32_t *brow = bits + st * row_words;
-    const uint32_t nw = word_stores ? nbytes >> 2 : 0u;
-    for (uint32_t k = lane; k < nw; k += kEncLanes)
-      cg_st(reinterpret_cast<uint32_t *>(orow) + k, __builtin_bswap32(brow[k]));
-    for (uint32_t b = 4 * nw + lane; b < nbytes; b += kEncLanes)
-      orow[b] = static_cast<uint8_t>(brow[b >> 2] >> (24 - 8 * (b & 3u)));
-  }
+    // 5. Half a wave per stream, its dwords [first, first + nw).
+    const uint32_t nw = more ? total >> 5 : (total + 31) >> 5;
+    const int half = lane >> 5;
+#pragma unroll 2
+    for (int p = wv; 2 * p < cnt; p += PIECES) {
+      const int st = 2 * p + half;
+      const uint32_t st_nw = __shfl(nw, st, 64), st_first = __shfl(first, st, 64), st_lead = __shfl(lead, st, 64);
+      const int64_t st_end = __shfl(end, st, 64);
+      uint8_t *row = block_out + __shfl(off, st, 64) - st_lead;
+      const uint32_t *sb = bits + st * at.row_words;
+      if (st < cnt) {
+        for (uint32_t k = lane & 31; k < st_nw; k += 32) {
+          const int64_t b0 = 4 * (static_cast<int64_t>(st_first) + k);
+          const uint32_t x = __builtin_bswap32(sb[k]);
+          if (b0 >= st_lead && b0 + 4 <= st_end) {
+            cg_st(reinterpret_cast<uint32_t *>(row + b0), x);
+          } else {
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+              if (b0 + b >= st_lead && b0 + b < st_end) row[b0 + b] = static_cast<uint8_t>(x >> (8 * b));
+          }
+        }
+      }
+    }
+    if (!more) return;
+    carry = (total & 31u) ? brow[total >> 5] : 0u;
+    first += total >> 5;
+    bit = total & 31u;
+    __syncthreads();  // the bits are dead
+    t0 += kEncTokens;
+    store_symbols(t0);
+    __syncthreads();
+  } while (true);
 }
 
 // Decode: 64 streams per block (one wave) and 40 KiB of LDS per block, so
@@ -1979,78 +1800,41 @@ __global__ void __launch_bounds__(kOffThreads)
   }
 }
 
-// Concatenates the used bytes of the streams' rows ([n_streams, cap], stream
-// s using min(lens[s], cap)): 64 streams per block, whose bytes start at
-// off[block] of `out`.  Half a wave copies a stream, kPackU of its
-// destination dwords in flight per lane; a destination dword inside the
-// stream takes two source dwords of the row and one align, and the bytes of
-// the dwords shared with the streams before and after are stored one by one.
-// Every source dword read holds a byte of the stream's own row.  Measured on
-// MI355X (64 planes x 256 tokens x 1024 channels, 7.3 MB of streams): 11.5 us,
-// in place of about 330 us for a boolean mask over the rows and a masked
-// select (a mask, its count, a partition and an index pass over every byte of
-// the rows' capacity); the whole chunk 408 -> 54 us.
-constexpr int kPackThreads = 512;
-constexpr int kPackHalves = kPackThreads / 32;
-constexpr int kPackU = 64 / kPackHalves;  // streams per half wave
+// Moves the blocks' bytes together: block b's off[b + 1] - off[b] bytes, from
+// b * stride of `blocks`, to off[b] of `out`.  A thread takes 16-byte aligned
+// pieces of the destination, each from five source dwords shifted together;
+// the bytes of the pieces shared with the blocks before and after are stored
+// one by one.  Every source dword read holds a byte of the block.  Measured
+// on MI355X (64 planes x 256 tokens x 1024 channels, 7.3 MB): 6.0 us.  (A
+// copy stream by stream from rows of their own, each with such edges: 11.5
+// us.  A boolean mask over the rows and a masked select: about 330 us.)
+constexpr int kPackThreads = 256;
 __global__ void __launch_bounds__(kPackThreads)
-    pack_streams_kernel(const uint8_t *__restrict__ rows, int64_t cap, const int32_t *__restrict__ lens,
-                        int64_t n_streams, const int64_t *__restrict__ off, uint8_t *__restrict__ out) {
-  __shared__ int64_t start[64];
-  __shared__ uint32_t size[64];
-  const int tid = static_cast<int>(threadIdx.x);
-  const int64_t s0 = static_cast<int64_t>(blockIdx.x) * 64;
-  if (tid < 64) {
-    const int64_t len = s0 + tid < n_streams ? lens[s0 + tid] : 0;
-    const uint32_t kept = static_cast<uint32_t>(len < cap ? len : cap);
-    const uint32_t lo = wave_incl_scan(kept & 0xFFFFu), hi = wave_incl_scan(kept >> 16);
-    start[tid] = off[blockIdx.x] + (static_cast<int64_t>(hi) << 16) + lo - kept;
-    size[tid] = kept;
-  }
-  __syncthreads();
-  const int half = tid >> 5, hl = tid & 31;
-  const uint8_t *src[kPackU];
-  uint8_t *dst[kPackU];
-  uint32_t n[kPackU], longest = 0;
-#pragma unroll
-  for (int u = 0; u < kPackU; ++u) {
-    const int st = u * kPackHalves + half;
-    src[u] = rows + (s0 + st) * cap;
-    dst[u] = out + start[st];
-    n[u] = size[st];
-    longest = max(longest, n[u]);
-  }
-  // Dword k of a stream is the aligned destination dword at dst - lead + 4k.
-  for (uint32_t k0 = 0; 4 * k0 < longest + 3; k0 += 32) {
-    uint32_t w[kPackU];
-    int64_t at[kPackU];  // stream byte at the dword's first byte
-#pragma unroll
-    for (int u = 0; u < kPackU; ++u) {
-      at[u] = static_cast<int64_t>(4) * (k0 + hl) - static_cast<int64_t>(reinterpret_cast<uintptr_t>(dst[u]) & 3);
-      const int64_t end = n[u];
-      w[u] = 0;
-      if (at[u] < end && n[u] != 0) {
-        // The aligned source dwords holding bytes at .. at + 3, each read
-        // only if it holds a byte of [0, n).
-        const uint8_t *p = src[u] + at[u];
-        const uint32_t sh = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(p) & 3);
-        const uint32_t *a = reinterpret_cast<const uint32_t *>(p - sh);
-        const int64_t lo_at = at[u] - sh;  // stream byte at a[0]
-        const uint32_t x = lo_at + 4 > 0 ? gload(a) : 0u;
-        const uint32_t y = sh != 0 && lo_at + 4 < end ? gload(a + 1) : 0u;
-        w[u] = __builtin_amdgcn_alignbyte(y, x, sh);
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < kPackU; ++u) {
-      const int64_t end = n[u];
-      if (at[u] >= 0 && at[u] + 4 <= end) {
-        gstore(reinterpret_cast<uint32_t *>(dst[u] + at[u]), w[u]);
-      } else if (at[u] < end) {
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
-          if (at[u] + b >= 0 && at[u] + b < end) dst[u][at[u] + b] = static_cast<uint8_t>(w[u] >> (8 * b));
-      }
+    pack_blocks_kernel(const uint8_t *__restrict__ blocks, int64_t stride, const int64_t *__restrict__ off,
+                       uint8_t *__restrict__ out) {
+  typedef unsigned int w4 __attribute__((ext_vector_type(4)));
+  typedef unsigned int w4u __attribute__((ext_vector_type(4), aligned(4)));
+  const int64_t begin = off[blockIdx.x];
+  const int64_t n = off[blockIdx.x + 1] - begin;
+  const uint8_t *src = blocks + static_cast<int64_t>(blockIdx.x) * stride;
+  uint8_t *dst = out + begin;
+  const int64_t lead = static_cast<int64_t>(reinterpret_cast<uintptr_t>(dst) & 15);
+  // Piece i of the destination holds the block's bytes 16 i - lead .. + 15.
+  for (int64_t at = 16 * static_cast<int64_t>(threadIdx.x) - lead; at < n; at += 16 * kPackThreads) {
+    if (at >= 0 && at + 16 <= n) {
+      const uint8_t *p = src + at;
+      const uint32_t sh = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(p) & 3);
+      const w4u x = *reinterpret_cast<const __attribute__((address_space(1))) w4u *>(
+          reinterpret_cast<uintptr_t>(p - sh));
+      const uint32_t y = sh ? gload(reinterpret_cast<const uint32_t *>(p - sh) + 4) : 0u;
+      w4 r;
+      r.x = __builtin_amdgcn_alignbyte(x.y, x.x, sh);
+      r.y = __builtin_amdgcn_alignbyte(x.z, x.y, sh);
+      r.z = __builtin_amdgcn_alignbyte(x.w, x.z, sh);
+      r.w = __builtin_amdgcn_alignbyte(y, x.w, sh);
+      gstore(reinterpret_cast<w4 *>(dst + at), r);
+    } else {
+      for (int64_t b = at < 0 ? 0 : at; b < at + 16 && b < n; ++b) dst[b] = src[b];
     }
   }
 }
@@ -2181,8 +1965,10 @@ void make_cdf(const lmc_tensor &in, int32_t n_bins, const lmc_tensor &o, int32_t
   hip_check(hipGetLastError(), "cdf_tile_kernel launch");
 }
 
-// encode_fast_new (csrc/cachegen_kernels.cpp:17-58).
-void encode_rows(const lmc_tensor &cdf, const lmc_tensor &in, const lmc_tensor &ob, const lmc_tensor &ol,
+// encode_fast_new (csrc/cachegen_kernels.cpp:17-58) with place 0; with place
+// 1 the streams of each block of 64 one after the other (encode_split_kernel;
+// `ol` then holds their lengths already, and cdf is calculate_cdf's).
+void encode_rows(const lmc_tensor &cdf, const lmc_tensor &in, const lmc_tensor &ob, const lmc_tensor &ol, int place,
                  hipStream_t stream) {
   need_device(cdf, "cdf");
   need_device(in, "input_sym");
@@ -2205,61 +1991,25 @@ void encode_rows(const lmc_tensor &cdf, const lmc_tensor &in, const lmc_tensor &
   check(ob.sizes[0] == L && ob.sizes[1] == C, "output_buffer must be [L, C, chunk]");
   if (L == 0 || C == 0) return;
   DeviceGuard guard(in.device);
-  const int tiles = static_cast<int>((C + kEncLanes - 1) / kEncLanes);
-  const int word_stores =
-      (chunk % 4 == 0 && (reinterpret_cast<uintptr_t>(ob.data) & 3) == 0) ? 1 : 0;
+  const int64_t n_streams = L * C;
+  const int64_t blocks = (n_streams + kEncLanes - 1) / kEncLanes;
+  check(blocks < (int64_t(1) << 31) && T < (int64_t(1) << 31), "input too large");
   const int vec_in = (C % 16 == 0 && (reinterpret_cast<uintptr_t>(in.data) & 15) == 0) ? 1 : 0;
-  const bool rows_dw = (reinterpret_cast<uintptr_t>(cdf.data) & 3) == 0;
-  if (LMC_ENC_SPLIT && T > 0 && T <= kEncTileMaxT && nb <= kEncLanes && C % kEncLanes == 0 && vec_in &&
-      rows_dw) {
-    // Split encoder: bit rows of 2T bytes plus one word (codes are at
-    // most 16 bits), an odd number of words so that the lanes' rows start
-    // in different banks.
-    const int row_words = (static_cast<int>(T + 1) / 2 + 1) | 1;
-    const int rows_words = static_cast<int>(((nb + 1) * kEncLanes * 2 + 15) / 16 * 4);
-    const int phase1 = rows_words + kEncTileMaxT * kEncLanes / 4 + static_cast<int>(nb + 1) * kEncLanes;
-    const int stage_words = std::max(phase1, kEncLanes * row_words);
-    const size_t lds = 4 * (static_cast<size_t>((stage_words + kEncPieces * kEncLanes + 2) & ~1) + 2 * kEncLanes);
-    check(lds <= 65536, "encode: LDS budget exceeded");
-    hipLaunchKernelGGL(encode_split_kernel<kEncPieces>, dim3(L * tiles), dim3(64 * kEncPieces), lds,
-                       stream,
-                       static_cast<const int16_t *>(cdf.data),
-                       static_cast<const uint8_t *>(in.data), (int)T, (int)C,
-                       (int)nb, static_cast<uint8_t *>(ob.data), chunk,
-                       static_cast<int32_t *>(ol.data), tiles, word_stores, row_words, stage_words);
-    hip_check(hipGetLastError(), "encode_split_kernel launch");
-    return;
-  }
-  if (T > 0 && T <= kEncTileMaxT && nb <= kEncLanes) {
-    // Bits past min(chunk, 2 bytes per symbol) are never written (codes
-    // are at most 16 bits), so a wave's bit buffer holds that many bytes.
-    const int64_t cap_bytes = std::min<int64_t>(chunk, 2 * T);
-    const int cap_words = static_cast<int>((cap_bytes + 3) / 4);
-    const int sym_stride = (((T + 3) / 4) + 1) | 1;
-    const size_t lds = 4 * ((static_cast<size_t>(nb + 1) * kEncLanes * 2 + 15) / 16 * 4 +
-                            static_cast<size_t>(kEncLanes) * sym_stride +
-                            static_cast<size_t>(2 * kEncWaves) * cap_words);
-    const int vec_tile = vec_in;
-    check(lds <= 65536, "encode: LDS budget exceeded");
-    hipLaunchKernelGGL(encode_wave_kernel, dim3(L * tiles), dim3(kEncTileThreads), lds,
-                       stream,
-                       static_cast<const int16_t *>(cdf.data),
-                       static_cast<const uint8_t *>(in.data), (int)T, (int)C,
-                       (int)nb, static_cast<uint8_t *>(ob.data), chunk,
-                       static_cast<int32_t *>(ol.data), tiles, word_stores, vec_tile, sym_stride,
-                       cap_words);
-    hip_check(hipGetLastError(), "encode_wave_kernel launch");
-    return;
-  }
-  const size_t lds = static_cast<size_t>(nb) * kEncLanes * 4 +
-                     static_cast<size_t>(nb + 1) * kEncLanes * 2;
-  hipLaunchKernelGGL(encode_kernel, dim3(L * tiles), dim3(kEncLanes), lds,
-                     stream,
-                     static_cast<const int16_t *>(cdf.data),
-                     static_cast<const uint8_t *>(in.data), (int)T, (int)C,
-                     (int)nb, static_cast<uint8_t *>(ob.data), chunk,
-                     static_cast<int32_t *>(ol.data), tiles, word_stores);
-  hip_check(hipGetLastError(), "encode_kernel launch");
+  const int rows_dw = (reinterpret_cast<uintptr_t>(cdf.data) & 3) == 0 ? 1 : 0;
+  const EncLds at = enc_lds(T, static_cast<int>(nb));
+  // calculate_cdf's codes are at most 12 bits, so rows of 2 bytes a symbol
+  // cut no stream.
+  const bool image = place == 1 && T <= kEncTokens && chunk >= 2 * T &&
+                     (reinterpret_cast<uintptr_t>(ob.data) & 15) == 0;
+  const auto kern = image                                ? encode_split_kernel<kEncPieces, EncMode::kImage>
+                    : place == 0 && T <= kEncTokens ? encode_split_kernel<kEncPieces, EncMode::kRows>
+                                                         : encode_split_kernel<kEncPieces, EncMode::kLong>;
+  check(at.bytes <= 65536, "encode: LDS budget exceeded");
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(64 * kEncPieces), at.bytes, stream,
+                     static_cast<const int16_t *>(cdf.data), static_cast<const uint8_t *>(in.data), (int)T, (int)C,
+                     (int)nb, n_streams, static_cast<uint8_t *>(ob.data), chunk, static_cast<int32_t *>(ol.data),
+                     place, vec_in, rows_dw, at);
+  hip_check(hipGetLastError(), "encode_split_kernel launch");
 }
 
 } // namespace
@@ -2283,7 +2033,7 @@ int lmc_encode_fast_new(const lmc_tensor *cdf_t, const lmc_tensor *input_sym,
                         const lmc_tensor *output_lengths, void *stream) {
   return guarded([&] {
     encode_rows(deref(cdf_t, "cdf"), deref(input_sym, "input_sym"), deref(output_buffer, "output_buffer"),
-                deref(output_lengths, "output_lengths"), static_cast<hipStream_t>(stream));
+                deref(output_lengths, "output_lengths"), 0, static_cast<hipStream_t>(stream));
   });
 }
 
@@ -2329,35 +2079,32 @@ int lmc_cachegen_encode_rows(const lmc_tensor *input, int32_t n_bins, const lmc_
                        word.word());
     hip_check(hipGetLastError(), "stream_offsets_kernel launch");
     word.record();
-    encode_rows(cdf, in, rows, lens, stream);
+    encode_rows(cdf, in, rows, lens, 1, stream);
     *total = word.wait();
   });
 }
 
-int lmc_cachegen_pack_rows(const lmc_tensor *rows_t, const lmc_tensor *lengths_t, const lmc_tensor *offsets_t,
-                           const lmc_tensor *streams_t, void *stream) {
+int lmc_cachegen_pack_rows(const lmc_tensor *rows_t, const lmc_tensor *offsets_t, const lmc_tensor *streams_t,
+                           void *stream) {
   return guarded([&] {
     const lmc_tensor &rows = deref(rows_t, "rows");
-    const lmc_tensor &lens = deref(lengths_t, "lengths");
     const lmc_tensor &off = deref(offsets_t, "offsets");
     const lmc_tensor &o = deref(streams_t, "streams");
     need_device(rows, "rows");
-    need_device(lens, "lengths");
     need_device(off, "offsets");
     need_device(o, "streams");
     check(rows.ndim == 3 && rows.dtype == LMC_U8 && o.dtype == LMC_U8, "rows and streams must be uint8");
     const int64_t n_streams = rows.sizes[0] * rows.sizes[1];
     const int64_t blocks = (n_streams + 63) / 64;
-    check(lens.dtype == LMC_I32 && numel(lens) == n_streams, "lengths must be int32 [L, C]");
     check(off.dtype == LMC_I64 && numel(off) == 2 * blocks + 1, "offsets do not match the rows");
     if (n_streams == 0 || numel(o) == 0) return;
     check(blocks < (int64_t(1) << 31), "too many streams");
     DeviceGuard guard(rows.device);
-    hipLaunchKernelGGL(pack_streams_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kPackThreads), 0,
-                       static_cast<hipStream_t>(stream), static_cast<const uint8_t *>(rows.data), rows.sizes[2],
-                       static_cast<const int32_t *>(lens.data), n_streams, static_cast<const int64_t *>(off.data),
+    hipLaunchKernelGGL(pack_blocks_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kPackThreads), 0,
+                       static_cast<hipStream_t>(stream), static_cast<const uint8_t *>(rows.data),
+                       kEncLanes * rows.sizes[2], static_cast<const int64_t *>(off.data),
                        static_cast<uint8_t *>(o.data));
-    hip_check(hipGetLastError(), "pack_streams_kernel launch");
+    hip_check(hipGetLastError(), "pack_blocks_kernel launch");
   });
 }
 

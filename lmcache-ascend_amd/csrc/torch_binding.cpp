@@ -38,6 +38,7 @@ using CdfFn = int (*)(const lmc_tensor *, int32_t, const lmc_tensor *, void *);
 using Codec4Fn = int (*)(const lmc_tensor *, const lmc_tensor *, const lmc_tensor *, const lmc_tensor *, void *);
 using EncodeRowsFn = int (*)(const lmc_tensor *, int32_t, const lmc_tensor *, const lmc_tensor *, const lmc_tensor *,
                              const lmc_tensor *, int64_t *, void *);
+using PackRowsFn = int (*)(const lmc_tensor *, const lmc_tensor *, const lmc_tensor *, void *);
 using ErrFn = const char *(*)();
 
 struct Table {
@@ -51,7 +52,7 @@ struct Table {
   Codec4Fn encode = nullptr;
   Codec4Fn decode = nullptr;
   EncodeRowsFn encode_rows = nullptr;
-  Codec4Fn pack_rows = nullptr;
+  PackRowsFn pack_rows = nullptr;
   ErrFn last_error = nullptr;
 } g;
 
@@ -257,7 +258,7 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> cachegen_encode_chunk(const at::T
   raise_for(status);
   at::Tensor streams = at::empty({total}, opt.dtype(at::kByte));
   const lmc_tensor s = desc(streams);
-  raise_for(g.pack_rows(&r, &n, &o, &s, stream));
+  raise_for(g.pack_rows(&r, &o, &s, stream));
   return {cdf, lengths, streams};
 }
 
@@ -274,7 +275,7 @@ void bind(uintptr_t multi, uintptr_t single, uintptr_t load_flash, uintptr_t res
   g.encode = reinterpret_cast<Codec4Fn>(encode);
   g.decode = reinterpret_cast<Codec4Fn>(decode);
   g.encode_rows = reinterpret_cast<EncodeRowsFn>(encode_rows);
-  g.pack_rows = reinterpret_cast<Codec4Fn>(pack_rows);
+  g.pack_rows = reinterpret_cast<PackRowsFn>(pack_rows);
   g.last_error = reinterpret_cast<ErrFn>(last_error);
 }
 

@@ -88,7 +88,7 @@ SIGNATURES = {
     "lmc_calculate_cdf": [_T, _i32, _T, _vp],
     "lmc_encode_fast_new": [_T, _T, _T, _T, _vp],
     "lmc_cachegen_encode_rows": [_T, _i32, _T, _T, _T, _T, ctypes.POINTER(_i64), _vp],
-    "lmc_cachegen_pack_rows": [_T, _T, _T, _T, _vp],
+    "lmc_cachegen_pack_rows": [_T, _T, _T, _vp],
     "lmc_decode_fast_new": [_T, _T, _T, _T, _vp],
     "lmc_decode_fast_prefsum": [_T, _T, _T, _T, _vp],
     "lmc_rotary_embedding_k_fused": [_T, _T, _T, _i64, _T, _i32, _vp],

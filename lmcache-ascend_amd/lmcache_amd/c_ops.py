@@ -406,8 +406,8 @@ def encode_fast_new(cdf, input_sym, output_buffer, output_lengths) -> None:
 def cachegen_encode_chunk(symbols, n_bins: int, cap: int):
     """CDF int16 [L, C, n_bins + 1], stream lengths int32 [L, C] and the
     concatenated streams of uint8 symbols [L, T, C]: calculate_cdf and
-    encode_fast_new into rows of `cap` bytes, then the rows' used bytes
-    one after the other.  Waits for the streams' total size."""
+    encode_fast_new's bytes, each stream cut to `cap`, one after the other.
+    Waits for the streams' total size."""
     if _ext is not None:
         return _ext.cachegen_encode_chunk(symbols, int(n_bins), int(cap))
     L, _, C = symbols.shape
@@ -422,7 +422,7 @@ def cachegen_encode_chunk(symbols, n_bins: int, cap: int):
                                      _stream(dev.index)))
     streams = torch.empty(total.value, dtype=torch.uint8, device=dev)
     s = _desc(streams)
-    _run(_L.lmc_cachegen_pack_rows(_ref(r), _ref(n), _ref(o), _ref(s), _stream(dev.index)))
+    _run(_L.lmc_cachegen_pack_rows(_ref(r), _ref(o), _ref(s), _stream(dev.index)))
     return cdf, lengths, streams
 
 

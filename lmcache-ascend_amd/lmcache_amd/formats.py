@@ -196,9 +196,9 @@ def _array(data: bytes, off: int, size: int, dtype, shape) -> torch.Tensor:
 
 def encode_chunk(symbols: torch.Tensor, n_bins: int, max_stream_bytes: int = 0) -> CacheGenChunk:
     """Encodes uint8 symbols [L, T, C] (values below n_bins) on the GPU:
-    calculate_cdf, encode_fast_new into per-stream rows of
-    `max_stream_bytes` (default: enough for 16 bits per symbol), then the
-    rows' used bytes concatenated in (layer, channel) order.  The streams'
+    calculate_cdf, and the streams encode_fast_new writes into rows of
+    `max_stream_bytes` (default: enough for 16 bits per symbol),
+    concatenated in (layer, channel) order.  The streams'
     size is read on the host before the call returns."""
     if not symbols.is_cuda or symbols.dtype != torch.uint8 or symbols.dim() != 3:
         raise ValueError("encode_chunk takes uint8 GPU symbols [L, T, C]")

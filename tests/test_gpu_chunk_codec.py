@@ -96,3 +96,24 @@ def test_decode_long_foreign_rows(kind, T):
     c_ops.decode_fast_prefsum(torch.from_numpy(cdf).to(DEV), torch.from_numpy(stream).to(DEV),
                               torch.from_numpy(prefix).to(DEV), out)
     assert np.array_equal(out.cpu().numpy(), want)
+
+
+# Rows of encode_fast_new: every byte below min(chunk, length) and no other,
+# at row strides off the dword, rows that cut their streams, and one to four
+# 256-token pieces (a stream's last dword carried from one to the next).
+@pytest.mark.parametrize("kind", ["normal", "skewed"])
+@pytest.mark.parametrize("L,T,C,nb,chunk", [
+    (2, 256, 64, 32, 512), (1, 256, 96, 32, 201), (3, 5, 17, 16, 11), (2, 257, 64, 32, 514), (1, 512, 96, 16, 1024),
+    (2, 513, 33, 63, 333), (1, 1000, 64, 32, 1999), (1, 1000, 32, 64, 2), (3, 300, 48, 64, 1),
+])
+def test_encode_rows_vs_oracle(L, T, C, nb, chunk, kind):
+    from lmcache_amd import c_ops
+
+    sym = _symbols(L, T, C, nb, T + C + chunk, kind)
+    cdf = oc.calculate_cdf(sym, nb)
+    want, want_len = oc.encode(cdf, sym, chunk, out=np.full((L, C, chunk), 0xEE, np.uint8))
+    rows = torch.full((L, C, chunk), 0xEE, dtype=torch.uint8, device=DEV)
+    lens = torch.full((L, C), -1, dtype=torch.int32, device=DEV)
+    c_ops.encode_fast_new(torch.from_numpy(cdf).to(DEV), torch.from_numpy(sym).to(DEV), rows, lens)
+    assert np.array_equal(lens.cpu().numpy(), want_len)
+    assert np.array_equal(rows.cpu().numpy(), want)
