@@ -372,6 +372,14 @@ int lmc_decode_fast_prefsum(const lmc_tensor *cdf,
                             const lmc_tensor *lengths,
                             const lmc_tensor *output, void *stream);
 
+/* No counterpart in the reference: decode_fast_prefsum with the streams'
+ * lengths (int32 [L, C], bytes) in place of their inclusive prefix sums.
+ * sums: device scratch, int32, one entry per 64 streams and one per 4096
+ * (both rounded up). */
+int lmc_cachegen_decode(const lmc_tensor *cdf, const lmc_tensor *bytestreams,
+                        const lmc_tensor *lengths, const lmc_tensor *sums,
+                        const lmc_tensor *output, void *stream);
+
 /* ------------------------------------------------------------------------
  * Fused K re-rotation (CacheBlend)
  * ------------------------------------------------------------------------ */

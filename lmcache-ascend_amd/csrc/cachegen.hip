@@ -1288,6 +1288,19 @@ __device__ __forceinline__ StreamAt stream_at(int64_t l, int c, uint32_t k, int 
   return {l + up, static_cast<int>(x - up * static_cast<uint32_t>(C))};
 }
 
+// Where the streams lie in the byte buffer: inclusive prefix sums of their
+// lengths, or (prefix null) the lengths with the sums length_sums_kernel
+// makes of them.  Both give a stream's end as the same int32, the sum of the
+// lengths up to it modulo 2^32.
+struct StreamEnds {
+  const int32_t *prefix;
+  const int32_t *lens;
+  const uint32_t *sums;    // [64-stream blocks]: lengths before the block in its group of 64 blocks
+  const uint32_t *groups;  // [groups]: lengths of a group
+};
+constexpr int kSumThreads = 1024;
+constexpr int kGroupBlocks = 64;  // 64-stream blocks per group
+
 // Stream geometry of one decode block: lane i of a wave owns stream
 // s0 + i; bytes of the block's streams are [B0, B1) of the byte buffer.
 struct DecBlock {
@@ -1297,7 +1310,7 @@ struct DecBlock {
   int c0;
   uintptr_t R0, R1, r_lo;
 
-  __device__ __forceinline__ void init(const int16_t *cdf, int64_t nbytes, const int32_t *prefix,
+  __device__ __forceinline__ void init(const int16_t *cdf, int64_t nbytes, const StreamEnds &ends,
                                        int64_t n_streams, int C, int nb, int lane) {
     s0 = static_cast<int64_t>(blockIdx.x) * kDecLanes;
     l0 = s0 < (int64_t(1) << 32) ? static_cast<uint32_t>(s0) / static_cast<uint32_t>(C) : s0 / C;
@@ -1305,11 +1318,28 @@ struct DecBlock {
     cnt = n_streams - s0 < kDecLanes ? static_cast<int>(n_streams - s0) : kDecLanes;
     const int64_t stream = s0 + (lane < cnt ? lane : 0);
     auto clampb = [&](int64_t x) { return x < 0 ? 0 : (x > nbytes ? nbytes : x); };
-    start = clampb(stream == 0 ? 0 : prefix[stream - 1]);
-    end = clampb(prefix[stream]);
+    if (ends.prefix != nullptr) {
+      start = clampb(stream == 0 ? 0 : ends.prefix[stream - 1]);
+      end = clampb(ends.prefix[stream]);
+      B0 = clampb(s0 == 0 ? 0 : ends.prefix[s0 - 1]);
+      B1 = clampb(ends.prefix[s0 + cnt - 1]);
+    } else {
+      const uint32_t len = lane < cnt ? static_cast<uint32_t>(ends.lens[stream]) : 0u;
+      uint32_t base = ends.sums[blockIdx.x];
+      const int group = static_cast<int>(blockIdx.x) / kGroupBlocks;
+      uint32_t part = 0;
+      for (int g = lane; g < group; g += kDecLanes) part += ends.groups[g];
+      const uint32_t incl = wave_incl_scan(len);
+      base += static_cast<uint32_t>(
+          __builtin_amdgcn_readlane(static_cast<int>(wave_incl_scan(part)), kDecLanes - 1));
+      const uint32_t all = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(incl), kDecLanes - 1));
+      auto at = [&](uint32_t x) { return clampb(static_cast<int32_t>(base + x)); };
+      start = at(incl - len);
+      end = at(incl);
+      B0 = at(0);
+      B1 = at(all);
+    }
     end = end < start || lane >= cnt ? start : end;
-    B0 = clampb(s0 == 0 ? 0 : prefix[s0 - 1]);
-    B1 = clampb(prefix[s0 + cnt - 1]);
     // Rows: bytes [R0, R1) from the 16-byte aligned address at or below R0.
     R0 = reinterpret_cast<uintptr_t>(cdf + s0 * (nb + 1));
     R1 = R0 + static_cast<uintptr_t>(cnt) * (nb + 1) * 2;
@@ -1349,7 +1379,7 @@ struct DecBlock {
 template <class Tab>
 __device__ __forceinline__ void decode_one_wave(uint8_t *lds, const int16_t *__restrict__ cdf,
                                                 const uint8_t *__restrict__ bytes, int64_t nbytes,
-                                                const int32_t *__restrict__ prefix, int T, int C,
+                                                const StreamEnds ends, int T, int C,
                                                 int nb, uint8_t *__restrict__ out, int64_t n_streams,
                                                 int lane) {
   constexpr int kRowsOff = Tab::kBytes + kObufBytes;
@@ -1357,7 +1387,7 @@ __device__ __forceinline__ void decode_one_wave(uint8_t *lds, const int16_t *__r
   const int win_off = kRowsOff + rows_cap;
   const int win_cap = (kDecLds - win_off) & ~15;
   DecBlock bk;
-  bk.init(cdf, nbytes, prefix, n_streams, C, nb, lane);
+  bk.init(cdf, nbytes, ends, n_streams, C, nb, lane);
   const int live = lane < bk.cnt;
   const uintptr_t base0 = reinterpret_cast<uintptr_t>(bytes);
   const uintptr_t a_lo = (base0 + bk.B0) & ~uintptr_t(15);
@@ -1426,7 +1456,7 @@ __device__ __forceinline__ void decode_one_wave(uint8_t *lds, const int16_t *__r
 // nothing, for any other block, which then takes decode_one_wave.
 __device__ __forceinline__ bool decode_one_wave_lanes(uint8_t *lds, const int16_t *__restrict__ cdf,
                                                       const uint8_t *__restrict__ bytes, int64_t nbytes,
-                                                      const int32_t *__restrict__ prefix, int T, int C, int nb,
+                                                      const StreamEnds ends, int T, int C, int nb,
                                                       uint8_t *__restrict__ out, int64_t n_streams,
                                                       int lane) {
   using Tab = cgdec::ByteTables;
@@ -1440,7 +1470,7 @@ __device__ __forceinline__ bool decode_one_wave_lanes(uint8_t *lds, const int16_
   const uint32_t lds_at =
       static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t *)lds));
   DecBlock bk;
-  bk.init(cdf, nbytes, prefix, n_streams, C, nb, lane);
+  bk.init(cdf, nbytes, ends, n_streams, C, nb, lane);
   if ((reinterpret_cast<uintptr_t>(out) & 3) != 0 || (C & 3) != 0 || (lds_at & (Tab::kBytes - 1)) != 0)
     return false;
   // The rows' loads depend on the block alone: issued before the stream
@@ -1586,16 +1616,16 @@ template <class Tab>
 __global__ void __launch_bounds__(kDecLanes)
     decode_kernel(const int16_t *__restrict__ cdf,
                   const uint8_t *__restrict__ bytes, int64_t nbytes,
-                  const int32_t *__restrict__ prefix, int T, int C, int nb,
+                  const StreamEnds ends, int T, int C, int nb,
                   uint8_t *__restrict__ out, int64_t n_streams) {
   extern __shared__ uint32_t lds_words[];
   uint8_t *lds = reinterpret_cast<uint8_t *>(lds_words);
   const int lane = static_cast<int>(threadIdx.x);
   if constexpr (std::is_same<Tab, cgdec::ByteTables>::value) {
-    if (LMC_DEC_LANES && decode_one_wave_lanes(lds, cdf, bytes, nbytes, prefix, T, C, nb, out, n_streams, lane))
+    if (LMC_DEC_LANES && decode_one_wave_lanes(lds, cdf, bytes, nbytes, ends, T, C, nb, out, n_streams, lane))
       return;
   }
-  decode_one_wave<Tab>(lds, cdf, bytes, nbytes, prefix, T, C, nb, out, n_streams, lane);
+  decode_one_wave<Tab>(lds, cdf, bytes, nbytes, ends, T, C, nb, out, n_streams, lane);
 }
 
 // Decode of streams longer than the lane regions hold (n_bins <= 32, more
@@ -1627,7 +1657,7 @@ constexpr int long_lds_bytes(int nb) { return kLongRows + (((nb + 1) * kDecLanes
 
 __global__ void __launch_bounds__(kDecLanes)
     decode_long_kernel(const int16_t *__restrict__ cdf, const uint8_t *__restrict__ bytes, int64_t nbytes,
-                       const int32_t *__restrict__ prefix, int T, int C, int nb, uint8_t *__restrict__ out,
+                       const StreamEnds ends, int T, int C, int nb, uint8_t *__restrict__ out,
                        int64_t n_streams) {
   extern __shared__ uint32_t lds_words[];
   uint8_t *lds = reinterpret_cast<uint8_t *>(lds_words);
@@ -1635,7 +1665,7 @@ __global__ void __launch_bounds__(kDecLanes)
       static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t *)lds));
   const int lane = static_cast<int>(threadIdx.x);
   DecBlock bk;
-  bk.init(cdf, nbytes, prefix, n_streams, C, nb, lane);
+  bk.init(cdf, nbytes, ends, n_streams, C, nb, lane);
   const int nrow = static_cast<int>((bk.R1 - bk.r_lo + 15) >> 4);
   chunk16 rv[kRowChunks], cv[kFirstChunks];
   load_chunks(bk.r_lo, nrow, 0, lane, rv);
@@ -1915,6 +1945,37 @@ private:
   bool pending_ = false;
 };
 
+// The sums of StreamEnds: a workgroup takes a group of 64 blocks of 64
+// streams, four lengths per thread.  A decode block adds the groups before
+// its own to its block's sum, which for 65536 streams is one load per lane
+// and one wave sum, so the prefix sums of the streams are never written.
+// Measured on MI355X (65536 streams): 3.0 us and the decode kernel behind it
+// 20.7 us, against four launches of about 17 us for prefix sums in 64 bits
+// (widening, scan, narrowing) and 24.4 us for the decode kernel reading them;
+// decode_chunk 35.9 -> 22.4 us.
+__global__ void __launch_bounds__(kSumThreads)
+    length_sums_kernel(const int32_t *__restrict__ lens, int64_t n_streams, int64_t n_blocks,
+                       uint32_t *__restrict__ sums, uint32_t *__restrict__ groups) {
+  __shared__ uint32_t block_sum[kGroupBlocks];
+  const int tid = static_cast<int>(threadIdx.x);
+  const int64_t s = (static_cast<int64_t>(blockIdx.x) * kSumThreads + tid) * 4;
+  uint32_t own = 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) own += s + k < n_streams ? static_cast<uint32_t>(lens[s + k]) : 0u;
+  // 16 threads hold a block's lengths.
+#pragma unroll
+  for (int d = 1; d < 16; d <<= 1) own += __shfl_xor(own, d, 64);
+  if ((tid & 15) == 0) block_sum[tid >> 4] = own;
+  __syncthreads();
+  if (tid < kGroupBlocks) {
+    const uint32_t b = block_sum[tid];
+    const uint32_t incl = wave_incl_scan(b);
+    const int64_t block = static_cast<int64_t>(blockIdx.x) * kGroupBlocks + tid;
+    if (block < n_blocks) sums[block] = incl - b;
+    if (tid == kGroupBlocks - 1) groups[blockIdx.x] = incl;
+  }
+}
+
 // Row-major contiguity; a tensor without elements has no layout to check.
 bool contiguous(const lmc_tensor &t) {
   if (numel(t) == 0) return true;
@@ -2010,6 +2071,66 @@ void encode_rows(const lmc_tensor &cdf, const lmc_tensor &in, const lmc_tensor &
                      (int)nb, n_streams, static_cast<uint8_t *>(ob.data), chunk, static_cast<int32_t *>(ol.data),
                      place, vec_in, rows_dw, at);
   hip_check(hipGetLastError(), "encode_split_kernel launch");
+}
+
+// decode_fast_prefsum (csrc/cachegen_kernels.cpp:67-112); with `sums`,
+// scratch for StreamEnds, `ln` holds the streams' lengths in place of their
+// prefix sums.
+void decode_streams(const lmc_tensor &cdf, const lmc_tensor &bs, const lmc_tensor &ln, const lmc_tensor &o,
+                    const lmc_tensor *sums, hipStream_t stream) {
+  // csrc/cachegen_kernels.cpp:78-88
+  check(cdf.device >= 0, "cdf is not a GPU tensor");
+  check(bs.device >= 0, "bytestreams is not a GPU tensor");
+  check(ln.device >= 0, "lengths is not a GPU tensor");
+  check(o.device >= 0, "output is not a GPU tensor");
+  need_device(cdf, "cdf");
+  need_device(bs, "bytestreams");
+  need_device(ln, "lengths");
+  need_device(o, "output");
+  check(cdf.ndim == 3, "cdf must be [L, C, nbins + 1]");
+  const int64_t L = cdf.sizes[0], C = cdf.sizes[1], nb = cdf.sizes[2] - 1;
+  check(C % 32 == 0, "decode takes a channel count that is a multiple of 32");
+  check(nb < 64, "decode takes fewer than 64 bins per stream");
+  check(nb >= 1, "cdf needs at least one bin");
+  check(cdf.dtype == LMC_I16, "cdf must be int16");
+  check(bs.dtype == LMC_U8 || bs.dtype == LMC_I8, "bytestreams must be uint8");
+  check(ln.dtype == LMC_I32 && numel(ln) == L * C, "lengths must be int32 [L, C]");
+  check(o.dtype == LMC_U8 || o.dtype == LMC_I8, "output must be uint8");
+  check(o.ndim >= 2, "output must be [L, T, C]");
+  const int64_t T = o.sizes[1];
+  check(numel(o) == L * T * C, "output must hold L * T * C symbols");
+  if (L == 0 || C == 0 || T == 0) return;
+  DeviceGuard guard(bs.device);
+  const int64_t n_streams = L * C;
+  const int64_t blocks = (n_streams + kDecLanes - 1) / kDecLanes;
+  check(blocks < (int64_t(1) << 31), "too many streams");
+  StreamEnds ends = {nullptr, nullptr, nullptr, nullptr};
+  if (sums == nullptr) {
+    ends.prefix = static_cast<const int32_t *>(ln.data);
+  } else {
+    const int64_t groups = (blocks + kGroupBlocks - 1) / kGroupBlocks;
+    need_device(*sums, "sums");
+    check(sums->dtype == LMC_I32 && numel(*sums) >= blocks + groups,
+          "sums must be int32 with an entry per block of 64 streams and per 64 blocks");
+    uint32_t *b = static_cast<uint32_t *>(sums->data);
+    ends.lens = static_cast<const int32_t *>(ln.data);
+    ends.sums = b;
+    ends.groups = b + blocks;
+    hipLaunchKernelGGL(length_sums_kernel, dim3(static_cast<unsigned>(groups)), dim3(kSumThreads), 0, stream,
+                       ends.lens, n_streams, blocks, b, b + blocks);
+    hip_check(hipGetLastError(), "length_sums_kernel launch");
+  }
+  const bool long_streams = nb <= cgdec::ByteTables::kMaxBins && T > kLaneMaxT &&
+                            (reinterpret_cast<uintptr_t>(o.data) & 3) == 0;
+  const auto kern = long_streams                          ? decode_long_kernel
+                    : nb <= cgdec::ByteTables::kMaxBins ? decode_kernel<cgdec::ByteTables>
+                                                          : decode_kernel<DecTables>;
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(kDecLanes),
+                     long_streams ? long_lds_bytes(static_cast<int>(nb)) : kDecLds, stream,
+                     static_cast<const int16_t *>(cdf.data),
+                     static_cast<const uint8_t *>(bs.data), numel(bs), ends, (int)T, (int)C,
+                     (int)nb, static_cast<uint8_t *>(o.data), n_streams);
+  hip_check(hipGetLastError(), "decode_kernel launch");
 }
 
 } // namespace
@@ -2120,49 +2241,16 @@ int lmc_decode_fast_prefsum(const lmc_tensor *cdf_t,
                             const lmc_tensor *lengths,
                             const lmc_tensor *output, void *stream) {
   return guarded([&] {
-    const lmc_tensor &cdf = deref(cdf_t, "cdf");
-    const lmc_tensor &bs = deref(bytestreams, "bytestreams");
-    const lmc_tensor &ln = deref(lengths, "lengths");
-    const lmc_tensor &o = deref(output, "output");
-    // csrc/cachegen_kernels.cpp:78-88
-    check(cdf.device >= 0, "cdf is not a GPU tensor");
-    check(bs.device >= 0, "bytestreams is not a GPU tensor");
-    check(ln.device >= 0, "lengths is not a GPU tensor");
-    check(o.device >= 0, "output is not a GPU tensor");
-    need_device(cdf, "cdf");
-    need_device(bs, "bytestreams");
-    need_device(ln, "lengths");
-    need_device(o, "output");
-    check(cdf.ndim == 3, "cdf must be [L, C, nbins + 1]");
-    const int64_t L = cdf.sizes[0], C = cdf.sizes[1], nb = cdf.sizes[2] - 1;
-    check(C % 32 == 0, "decode takes a channel count that is a multiple of 32");
-    check(nb < 64, "decode takes fewer than 64 bins per stream");
-    check(nb >= 1, "cdf needs at least one bin");
-    check(cdf.dtype == LMC_I16, "cdf must be int16");
-    check(bs.dtype == LMC_U8 || bs.dtype == LMC_I8, "bytestreams must be uint8");
-    check(ln.dtype == LMC_I32 && numel(ln) == L * C, "lengths must be int32 [L, C]");
-    check(o.dtype == LMC_U8 || o.dtype == LMC_I8, "output must be uint8");
-    check(o.ndim >= 2, "output must be [L, T, C]");
-    const int64_t T = o.sizes[1];
-    check(numel(o) == L * T * C, "output must hold L * T * C symbols");
-    if (L == 0 || C == 0 || T == 0) return;
-    DeviceGuard guard(bs.device);
-    const int64_t n_streams = L * C;
-    const int64_t blocks = (n_streams + kDecLanes - 1) / kDecLanes;
-    check(blocks < (int64_t(1) << 31), "too many streams");
-    const bool long_streams = nb <= cgdec::ByteTables::kMaxBins && T > kLaneMaxT &&
-                              (reinterpret_cast<uintptr_t>(o.data) & 3) == 0;
-    const auto kern = long_streams                          ? decode_long_kernel
-                      : nb <= cgdec::ByteTables::kMaxBins ? decode_kernel<cgdec::ByteTables>
-                                                            : decode_kernel<DecTables>;
-    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(kDecLanes),
-                       long_streams ? long_lds_bytes(static_cast<int>(nb)) : kDecLds,
-                       static_cast<hipStream_t>(stream),
-                       static_cast<const int16_t *>(cdf.data),
-                       static_cast<const uint8_t *>(bs.data), numel(bs),
-                       static_cast<const int32_t *>(ln.data), (int)T, (int)C,
-                       (int)nb, static_cast<uint8_t *>(o.data), n_streams);
-    hip_check(hipGetLastError(), "decode_kernel launch");
+    decode_streams(deref(cdf_t, "cdf"), deref(bytestreams, "bytestreams"), deref(lengths, "lengths"),
+                   deref(output, "output"), nullptr, static_cast<hipStream_t>(stream));
+  });
+}
+
+int lmc_cachegen_decode(const lmc_tensor *cdf_t, const lmc_tensor *bytestreams, const lmc_tensor *lengths,
+                        const lmc_tensor *sums, const lmc_tensor *output, void *stream) {
+  return guarded([&] {
+    decode_streams(deref(cdf_t, "cdf"), deref(bytestreams, "bytestreams"), deref(lengths, "lengths"),
+                   deref(output, "output"), &deref(sums, "sums"), static_cast<hipStream_t>(stream));
   });
 }
 

@@ -39,6 +39,8 @@ using Codec4Fn = int (*)(const lmc_tensor *, const lmc_tensor *, const lmc_tenso
 using EncodeRowsFn = int (*)(const lmc_tensor *, int32_t, const lmc_tensor *, const lmc_tensor *, const lmc_tensor *,
                              const lmc_tensor *, int64_t *, void *);
 using PackRowsFn = int (*)(const lmc_tensor *, const lmc_tensor *, const lmc_tensor *, void *);
+using DecodeFn = int (*)(const lmc_tensor *, const lmc_tensor *, const lmc_tensor *, const lmc_tensor *,
+                         const lmc_tensor *, void *);
 using ErrFn = const char *(*)();
 
 struct Table {
@@ -53,6 +55,7 @@ struct Table {
   Codec4Fn decode = nullptr;
   EncodeRowsFn encode_rows = nullptr;
   PackRowsFn pack_rows = nullptr;
+  DecodeFn decode_chunk = nullptr;
   ErrFn last_error = nullptr;
 } g;
 
@@ -262,9 +265,26 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> cachegen_encode_chunk(const at::T
   return {cdf, lengths, streams};
 }
 
+// A chunk's symbols from its streams and their lengths (formats.py).
+at::Tensor cachegen_decode_chunk(const at::Tensor &cdf, const at::Tensor &streams, const at::Tensor &lengths,
+                                 int64_t num_tokens) {
+  check_bound();
+  if (!cdf.is_cuda() || cdf.dim() != 3)
+    throw std::runtime_error("cachegen_decode_chunk: cdf must be a GPU tensor [L, C, nbins + 1]");
+  const int64_t L = cdf.size(0), C = cdf.size(1), blocks = (L * C + 63) / 64;
+  at::Tensor out = at::empty({L, num_tokens, C}, cdf.options().dtype(at::kByte));
+  at::Tensor sums = at::empty({blocks + (blocks + 63) / 64}, cdf.options().dtype(at::kInt));
+  // The op needs an addressable buffer.
+  const at::Tensor bytes = streams.numel() ? streams : at::zeros({1}, cdf.options().dtype(at::kByte));
+  const lmc_tensor c = desc(cdf), b = desc(bytes), n = desc(lengths), t = desc(sums), o = desc(out);
+  raise_for(g.decode_chunk(&c, &b, &n, &t, &o, stream_of(cdf.get_device())));
+  return out;
+}
+
 void bind(uintptr_t multi, uintptr_t single, uintptr_t load_flash, uintptr_t reshape_flash,
           uintptr_t rope, uintptr_t blend, uintptr_t cdf, uintptr_t encode, uintptr_t decode,
-          uintptr_t encode_rows, uintptr_t pack_rows, uintptr_t last_error) {
+          uintptr_t encode_rows, uintptr_t pack_rows, uintptr_t decode_chunk,
+          uintptr_t last_error) {
   g.multi = reinterpret_cast<MultiFn>(multi);
   g.single = reinterpret_cast<SingleFn>(single);
   g.load_flash = reinterpret_cast<FlashFn>(load_flash);
@@ -276,6 +296,7 @@ void bind(uintptr_t multi, uintptr_t single, uintptr_t load_flash, uintptr_t res
   g.decode = reinterpret_cast<Codec4Fn>(decode);
   g.encode_rows = reinterpret_cast<EncodeRowsFn>(encode_rows);
   g.pack_rows = reinterpret_cast<PackRowsFn>(pack_rows);
+  g.decode_chunk = reinterpret_cast<DecodeFn>(decode_chunk);
   g.last_error = reinterpret_cast<ErrFn>(last_error);
 }
 
@@ -301,6 +322,7 @@ PYBIND11_MODULE(_c_ops_ext, m) {
   m.def("blend_layer_to_paged", &blend_layer_to_paged);
   m.def("calculate_cdf", &calculate_cdf);
   m.def("cachegen_encode_chunk", &cachegen_encode_chunk);
+  m.def("cachegen_decode_chunk", &cachegen_decode_chunk);
   m.def("encode_fast_new", [](const at::Tensor &cdf, const at::Tensor &sym, at::Tensor &out, at::Tensor &lens) {
     codec4(g.encode, cdf, sym, out, lens, sym);
   });

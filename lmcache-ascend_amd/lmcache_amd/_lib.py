@@ -91,6 +91,7 @@ SIGNATURES = {
     "lmc_cachegen_pack_rows": [_T, _T, _T, _vp],
     "lmc_decode_fast_new": [_T, _T, _T, _T, _vp],
     "lmc_decode_fast_prefsum": [_T, _T, _T, _T, _vp],
+    "lmc_cachegen_decode": [_T, _T, _T, _T, _T, _vp],
     "lmc_rotary_embedding_k_fused": [_T, _T, _T, _i64, _T, _i32, _vp],
     "lmc_get_device_ptr": [_up, _sz, ctypes.POINTER(_up)],
     "lmc_register_mapping": [_up, _up, _sz, ctypes.POINTER(_up)],

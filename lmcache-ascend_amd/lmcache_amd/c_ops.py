@@ -49,6 +49,7 @@ try:
         _addr("lmc_decode_fast_prefsum"),
         _addr("lmc_cachegen_encode_rows"),
         _addr("lmc_cachegen_pack_rows"),
+        _addr("lmc_cachegen_decode"),
         _addr("lmc_last_error"),
     )
 except ImportError:
@@ -429,6 +430,24 @@ def cachegen_encode_chunk(symbols, n_bins: int, cap: int):
 def decode_fast_new(cdf, bytestreams, lengths, output) -> None:
     """csrc/cachegen_kernels.cpp:60-65: raises NotImplementedError."""
     raise NotImplementedError("Please use decode_fast_prefsum.")
+
+
+def cachegen_decode_chunk(cdf, bytestreams, lengths, num_tokens: int):
+    """The uint8 symbols [L, T, C] of a chunk's concatenated streams:
+    decode_fast_prefsum with the streams' lengths (int32 [L, C]) in place of
+    their prefix sums."""
+    if _ext is not None:
+        return _ext.cachegen_decode_chunk(cdf, bytestreams, lengths, int(num_tokens))
+    L, C = int(cdf.shape[0]), int(cdf.shape[1])
+    dev = cdf.device
+    if bytestreams.numel() == 0:  # the op needs an addressable buffer
+        bytestreams = torch.zeros(1, dtype=torch.uint8, device=dev)
+    out = torch.empty((L, int(num_tokens), C), dtype=torch.uint8, device=dev)
+    blocks = (L * C + 63) // 64
+    sums = torch.empty(blocks + (blocks + 63) // 64, dtype=torch.int32, device=dev)
+    c, b, n, t, o = _desc(cdf), _desc(bytestreams), _desc(lengths), _desc(sums), _desc(out)
+    _run(_L.lmc_cachegen_decode(_ref(c), _ref(b), _ref(n), _ref(t), _ref(o), _stream(dev.index)))
+    return out
 
 
 def decode_fast_prefsum(cdf, bytestreams, lengths, output) -> None:

@@ -209,12 +209,17 @@ def encode_chunk(symbols: torch.Tensor, n_bins: int, max_stream_bytes: int = 0) 
 
 
 def decode_chunk(chunk: CacheGenChunk) -> torch.Tensor:
-    """Decodes a chunk on the GPU into uint8 symbols [L, T, C]
-    (decode_fast_prefsum over the concatenated streams)."""
+    """Decodes a chunk on the GPU into uint8 symbols [L, T, C]: the streams'
+    places come from their lengths on the way (cachegen_decode_chunk), or,
+    for lengths of another type or layout, from their prefix sums
+    (decode_fast_prefsum)."""
     L, T, C = chunk.shape
     dev = chunk.cdf.device
     if dev.type != "cuda":
         raise ValueError("decode_chunk takes a chunk on the GPU (CacheGenChunk.to)")
+    n = chunk.lengths
+    if n.dtype == torch.int32 and n.device == dev and n.is_contiguous() and n.numel() == L * C:
+        return c_ops.cachegen_decode_chunk(chunk.cdf, chunk.streams.to(dev), n, T)
     prefix = torch.cumsum(chunk.lengths.to(torch.int64).view(-1), 0).to(torch.int32).view(L, C)
     streams = chunk.streams.to(dev)
     if streams.numel() == 0:  # the op needs an addressable buffer

@@ -117,3 +117,14 @@ def test_encode_rows_vs_oracle(L, T, C, nb, chunk, kind):
     c_ops.encode_fast_new(torch.from_numpy(cdf).to(DEV), torch.from_numpy(sym).to(DEV), rows, lens)
     assert np.array_equal(lens.cpu().numpy(), want_len)
     assert np.array_equal(rows.cpu().numpy(), want)
+
+
+# Streams' places from their lengths (groups of 4096 streams, a last block of
+# 32) and from prefix sums, which lengths of another type take.
+@pytest.mark.parametrize("L,T,C", [(1, 4, 32), (64, 3, 64), (43, 5, 96), (64, 2, 160), (3, 300, 1056)])
+def test_decode_chunk_by_lengths(F, L, T, C):
+    sym = _symbols(L, T, C, 16, L + T + C)
+    chunk = F.encode_chunk(torch.from_numpy(sym).to(DEV), 16)
+    other = F.CacheGenChunk(chunk.cdf, chunk.lengths.to(torch.int64), chunk.streams, T)
+    assert np.array_equal(F.decode_chunk(chunk).cpu().numpy(), sym)
+    assert np.array_equal(F.decode_chunk(other).cpu().numpy(), sym)
