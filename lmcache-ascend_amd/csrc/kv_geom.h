@@ -66,13 +66,13 @@ typedef __attribute__((address_space(1))) u32x4 GlobalU32x4;
 // (agent) scope, which writes through the XCD's L2 instead of leaving the
 // line dirty there, so the kernel's end-of-launch L2 write-back has nothing
 // left to flush; without it (and for narrower vectors) the store carries the
-// streaming hint.  Which is faster depends on the kernel (MI355X, three
-// interleaved runs each): the row kernels are faster with streaming stores
-// (8B shape, 16 objects in one launch 0.172 -> 0.170 ms per direction; 32
-// per-layer flash stores 0.259 -> 0.244 ms; Qwen3-32B shape, 128 objects
-// stored in one launch 2.82 -> 2.70 ms), the tile kernel's stores to
-// memory objects are faster written through (MLA-576 store 0.388 -> 0.402
-// ms with streaming stores), and the direct kernels measure the same.
+// streaming hint.  Measured on MI355X with two or more buffer sets in turn,
+// streaming -> written through: the row kernels, 1024-column rows, 32 layers
+// x 256 tokens 13.1 / 13.4 -> 12.1 / 12.1 us (store / retrieve), 80 x 256
+// 29.1 / 29.3 -> 26.7 / 27.0, 64 x 8192 690 / 699 -> 685 / 677; the tile
+// kernel's stores to memory objects (MLA-576 store) 402 -> 388 us, its
+// retrieves stream; the group kernel's line is at its launch; the direct
+// kernels measure the same.
 template <typename T, bool NT, bool WT = true> __device__ __forceinline__ void st(T *p, T v) {
   if constexpr (NT && WT && LMC_KV_WT_STORES && sizeof(T) == 16)
     __builtin_amdgcn_global_store_b128((GlobalU32x4 *)(p),

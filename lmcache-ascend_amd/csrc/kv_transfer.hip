@@ -46,9 +46,6 @@ namespace lmc {
 #ifndef LMC_KV_SEGS
 #define LMC_KV_SEGS 2             // 64-lane accesses per work item
 #endif
-#ifndef LMC_KV_XCD_REMAP
-#define LMC_KV_XCD_REMAP 0        // give each XCD a contiguous block range
-#endif
 #ifndef LMC_KV_LEAN
 #define LMC_KV_LEAN 1             // lean row kernel for its geometry
 #endif
@@ -97,6 +94,19 @@ template <int NC> struct ChunkListT {
 };
 using ChunkList = ChunkListT<kMaxChunks>;
 
+
+// The work of block b of n: blocks are dispatched round-robin over the 8
+// XCDs, and each XCD takes one contiguous range of the work, so an XCD's
+// address translations cover its own eighth of the rows and not all of them.
+// Measured on MI355X, 1024-column rows, both directions (store / retrieve):
+// 64 layers x 8192 tokens with 128-token blocks 750 / 880 -> 671 / 672 us, 32
+// layers x 4096 tokens 190 / 222 -> 174 / 177 us; batches of 0.4 to 0.8 GB
+// are 1-2% slower, smaller ones the same.  (The tile kernel is up to 7%
+// slower with it and keeps the dispatch order.)
+__device__ __forceinline__ int xcd_block(int b, int n) {
+  const int per = n >> 3;
+  return b < 8 * per ? (b & 7) * per + (b >> 3) : b;
+}
 
 // Resolves row `row` of chunk `c` to (src, dst); returns the row's byte count,
 // or 0 when the slot is skipped.  All inputs are wave-uniform.
@@ -162,12 +172,9 @@ __global__ void __launch_bounds__(kThreads)
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   uint8_t *lmc = reinterpret_cast<uint8_t *>(chunks.lmc[c]);
-  int bx = blockIdx.x;
-#if LMC_KV_XCD_REMAP
-  // Blocks are dispatched round-robin over the 8 XCDs; map each XCD's
-  // blocks onto one contiguous range of work.
-  if ((gridDim.x & 7) == 0) bx = (bx & 7) * (gridDim.x >> 3) + (bx >> 3);
-#endif
+  // The chunk's own blocks: a ragged last chunk has fewer than the grid.
+  const int own = (items + kWaves * kRowsPerWave - 1) / (kWaves * kRowsPerWave);
+  const int bx = xcd_block(blockIdx.x, own < static_cast<int>(gridDim.x) ? own : static_cast<int>(gridDim.x));
   const int step = gridDim.x * kWaves * kRowsPerWave;
 
   for (int i0 = (bx * kWaves + wave) * kRowsPerWave; i0 < items; i0 += step) {
@@ -217,7 +224,7 @@ __global__ void __launch_bounds__(kThreads)
 #pragma unroll
       for (int s = 0; s < kSegs; ++s) {
         const int64_t o = off0[r] + (s * 64 + lane) * VEC;
-        if (o < nb[r]) st<V, NT, false>(reinterpret_cast<V *>(dst[r] + o), v[r][s]);
+        if (o < nb[r]) st<V, NT>(reinterpret_cast<V *>(dst[r] + o), v[r][s]);
       }
   }
 }
@@ -348,7 +355,130 @@ __global__ void __launch_bounds__(kThreads)
     if (live[r])
 #pragma unroll
       for (int s = 0; s < kSegs; ++s)
-        st<V, NT, false>(reinterpret_cast<V *>(dst[r] + (s * 64 + lane) * 16), v[r][s]);
+        st<V, NT>(reinterpret_cast<V *>(dst[r] + (s * 64 + lane) * 16), v[r][s]);
+}
+
+// Group kernel, for rows of U x 2^g_shift 16-byte vectors, the same in every
+// plane (see launch_group for U).  A group of G = 2^g_shift lanes owns a row:
+// lane e of it moves vectors e, e + G, ..., so each access of a wave covers
+// 64 / G rows' segments of at least 128 bytes.  A lane loads its own row's
+// slot, R rows per group, alongside the wave's pointer-table entry, then
+// issues all U x R loads, then the stores: the dependent chain is the lean
+// kernel's, kernel arguments -> {slots, table entry} -> rows -> stores, with
+// no division and no exchange between lanes.  The grid is (token groups,
+// plane x layer, chunk), or (`linear`, for launches that fill the chip) the
+// token groups and planes of a chunk in one dimension, for xcd_block.  Block
+// sizes are powers of two, or rows are flat (bs_shift 0, blk_stride =
+// row_pitch).
+//
+// Bound by latency for one object and by memory for a batch.  Against the
+// tile kernel, which took these rows before (MI355X, two or more buffer sets
+// in turn, store / retrieve): 80 layers x 199 tokens x 128 columns 7.1 / 9.6
+// -> 5.7 / 5.7 us, 4 x 256 x 64 4.9 / 5.6 -> 2.9 / 3.2, 32 x 256 x 896 13.2
+// / 17.0 -> 11.8 / 11.8, a 32768-token layer of 768 columns 33.2 / 42.3 ->
+// 30.7 / 30.8; batches: 32 x 2048 x 384 34.5 / 39.9 -> 31.6 / 31.7, 64 x 8192
+// x 512 360 / 419 -> 352 / 371.  A wave whose lanes take the wave's vectors
+// in address order, with a slot per access, was slower (32 x 256 x 896 17.5).
+template <bool NT, int NC, bool WT, int U, int R>
+__global__ void __launch_bounds__(kThreads)
+    kv_rows_group(const CopyJob job, const ChunkListT<NC> chunks, int g_shift, int linear) {
+  using V = u32x4;
+  const int step = 64 >> g_shift;  // rows per U accesses of the wave
+  const int per_block = kWaves * R * step;
+  const int L = job.n_layers;
+  int c, y, x;
+  if (linear) {
+    c = NC == 1 ? 0 : static_cast<int>(blockIdx.y);
+    const int groups = (chunks.tok_count[c] + per_block - 1) / per_block;
+    const int own = groups * L * job.n_planes;
+    if (static_cast<int>(blockIdx.x) >= own) return;
+    const int b = xcd_block(blockIdx.x, own);
+    y = b / groups;
+    x = b - y * groups;
+  } else {
+    c = NC == 1 ? 0 : static_cast<int>(blockIdx.z);
+    y = blockIdx.y;
+    x = blockIdx.x;
+  }
+  const int T = chunks.tok_count[c];
+  const int tok0 = chunks.tok_start[c];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int t0 = x * per_block + wave * R * step;
+  if (t0 >= T) return;
+  const int p = (y >= L) + (y >= 2 * L);
+  const int l = y - p * L;
+  // The plane's descriptor: all planes' fields are read and one is selected,
+  // so they come with the other kernel arguments.
+  const PlaneDesc &d0 = job.plane[0], &d1 = job.plane[1], &d2 = job.plane[2];
+  auto pick = [&](int64_t v0, int64_t v1, int64_t v2) -> int64_t { return p == 2 ? v2 : p == 1 ? v1 : v0; };
+  const int64_t paged_off = pick(d0.paged_off, d1.paged_off, d2.paged_off);
+  const int64_t blk_stride = pick(d0.blk_stride, d1.blk_stride, d2.blk_stride);
+  const int64_t row_pitch = pick(d0.row_pitch, d1.row_pitch, d2.row_pitch);
+  const int64_t lmc_fixed = pick(d0.lmc_off_fixed, d1.lmc_off_fixed, d2.lmc_off_fixed);
+  const int64_t lmc_per_t = pick(d0.lmc_off_per_t, d1.lmc_off_per_t, d2.lmc_off_per_t);
+  const int64_t layer_fixed = pick(d0.lmc_layer_fixed, d1.lmc_layer_fixed, d2.lmc_layer_fixed);
+  const int64_t layer_per_t = pick(d0.lmc_layer_per_t, d1.lmc_layer_per_t, d2.lmc_layer_per_t);
+  const int64_t tok_stride = pick(d0.lmc_token_stride, d1.lmc_token_stride, d2.lmc_token_stride);
+  // Independent loads: the plane's paged base and the slots.
+  const uint64_t pbase =
+      job.table != nullptr ? job.table[static_cast<int64_t>(l) * job.table_ppl + p * job.idx_step]
+                           : static_cast<uint64_t>(pick(static_cast<int64_t>(job.base[0]), static_cast<int64_t>(job.base[1]),
+                                                        static_cast<int64_t>(job.base[2])));
+  uint8_t *const lm = reinterpret_cast<uint8_t *>(chunks.lmc[c]) + lmc_fixed + lmc_per_t * T +
+                      static_cast<int64_t>(l) * (layer_fixed + layer_per_t * T);
+  const int bs_shift = job.bs_shift;
+  const bool page2lmc = job.page2lmc != 0;
+  const int e = lane & ((1 << g_shift) - 1);
+  int64_t slot[R];
+  int t[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    t[r] = t0 + r * step + (lane >> g_shift);
+    const int64_t i = tok0 + (t[r] < T ? t[r] : T - 1);  // in-range token for the slot load
+    slot[r] = job.slot_i32 ? static_cast<int64_t>(static_cast<const int32_t *>(job.slots)[i])
+                           : static_cast<const int64_t *>(job.slots)[i];
+  }
+  const uint8_t *src[R];
+  uint8_t *dst[R];
+  bool live[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int64_t blk = slot[r] >> bs_shift;
+    const int64_t in_blk = slot[r] & ((int64_t(1) << bs_shift) - 1);
+    uint8_t *paged = reinterpret_cast<uint8_t *>(pbase) + paged_off + blk * blk_stride + in_blk * row_pitch + 16 * e;
+    uint8_t *obj = lm + static_cast<int64_t>(t[r]) * tok_stride + 16 * e;
+    src[r] = page2lmc ? paged : obj;
+    dst[r] = page2lmc ? obj : paged;
+    live[r] = t[r] < T && static_cast<uint64_t>(slot[r]) < static_cast<uint64_t>(job.num_slots);
+  }
+  // The host checked every alignment it can see; a table entry (a device
+  // value) that is not 16-byte aligned sends the wave to the byte path.
+  if (((pbase + paged_off) & 15) != 0) {
+#pragma unroll 1
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        if (live[r])
+          for (int b = 0; b < 16; ++b) {
+            const int64_t o = (static_cast<int64_t>(u) << g_shift) * 16 + b;
+            dst[r][o] = src[r][o];
+          }
+    return;
+  }
+  V v[R][U];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+    if (live[r])
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        v[r][u] = ld<V, NT>(reinterpret_cast<const V *>(src[r]) + (static_cast<int64_t>(u) << g_shift));
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+    if (live[r])
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        st<V, NT, WT>(reinterpret_cast<V *>(dst[r]) + (static_cast<int64_t>(u) << g_shift), v[r][u]);
 }
 
 // Tile kernel.  A wave owns a tile of up to 64 consecutive tokens of one
@@ -563,6 +693,78 @@ void launch_lean(const CopyJob &job, const ChunkList &chunks, int n_chunks,
   else launch_lean_t<kMaxChunks>(job, chunks, grid, nt, stream);
 }
 
+// Where the group kernel's stores to the paged caches are written through
+// (see st()) and where they stream: copies that the 256 MB last-level cache
+// about holds are faster written through (268 MB, 32 layers x 2048 x 512:
+// 47.0 -> 40.3 us), larger ones the same to 4% slower (393 MB: 68.3 -> 69.7,
+// 537 MB: 96 -> 100).  Stores to memory objects are always written through.
+constexpr int64_t kGroupWriteThrough = int64_t(288) << 20;
+// Launches of more blocks than this (eight a CU) are laid out for xcd_block;
+// smaller ones skip its division.
+constexpr int64_t kGroupLinear = 2048;
+// One row per group (R = 1) up to this many blocks, two above: the smallest
+// launches are 0.5 us faster with more waves (80 layers x 16 tokens x 128
+// columns 2.7 against 3.3 us), and large ones with more in flight per wave
+// (32 x 8192 x 128 stored, 45.7 against 41.1).
+constexpr int64_t kGroupOneRow = 1024;
+// Long stores of rows of nine vector groups (576-column MLA rows in bf16)
+// stay with the tile kernel: 2.3 GB 395 against 420 us; 0.58 GB is faster here
+// (110 against 115 us).
+constexpr int64_t kGroupNineStore = int64_t(1) << 30;
+
+template <int U, int R>
+void launch_group_u(const CopyJob &job, const ChunkList &chunks, int n_chunks, int64_t max_tokens, int g_shift,
+                    int64_t bytes, bool nt, hipStream_t stream) {
+  const int64_t per_block = static_cast<int64_t>(kWaves) * R * (64 >> g_shift);
+  const int64_t groups = (max_tokens + per_block - 1) / per_block;
+  const int64_t planes = static_cast<int64_t>(job.n_layers) * job.n_planes;
+  check(groups * planes < (int64_t(1) << 31), "too many blocks in one chunk");
+  const bool linear = groups * planes * n_chunks > kGroupLinear || planes > 65535;
+  const dim3 grid = linear ? dim3(static_cast<unsigned>(groups * planes), n_chunks)
+                           : dim3(static_cast<unsigned>(groups), static_cast<unsigned>(planes), n_chunks);
+  const dim3 block(kThreads);
+  const bool wt = job.page2lmc != 0 || bytes <= kGroupWriteThrough;
+  if (n_chunks == 1) {
+    const ChunkListT<1> one = first_chunk(chunks);
+    const auto kern = nt ? (wt ? kv_rows_group<true, 1, true, U, R> : kv_rows_group<true, 1, false, U, R>)
+                         : kv_rows_group<false, 1, false, U, R>;
+    hipLaunchKernelGGL(kern, grid, block, 0, stream, job, one, g_shift, linear);
+  } else {
+    const auto kern = nt ? (wt ? kv_rows_group<true, kMaxChunks, true, U, R> : kv_rows_group<true, kMaxChunks, false, U, R>)
+                         : kv_rows_group<false, kMaxChunks, false, U, R>;
+    hipLaunchKernelGGL(kern, grid, block, 0, stream, job, chunks, g_shift, linear);
+  }
+}
+
+// Launches the group kernel and returns true, or returns false for rows it
+// does not take: rows of `row_bytes` (in every plane) are U groups of 2^g
+// 16-byte vectors, g the largest that divides them with 3 <= g <= 6.
+bool launch_group(const CopyJob &job, const ChunkList &chunks, int n_chunks, int64_t max_tokens, int64_t row_bytes,
+                  bool nt, hipStream_t stream) {
+  const int64_t vecs = row_bytes / 16;
+  const int g = std::min(6, __builtin_ctzll(static_cast<uint64_t>(vecs)));
+  if (g < 3) return false;
+  int64_t rows = 0;
+  for (int c = 0; c < n_chunks; ++c) rows += static_cast<int64_t>(chunks.tok_count[c]) * job.n_layers * job.n_planes;
+  const int64_t bytes = 2 * rows * row_bytes;  // read and written
+  switch (vecs >> g) {
+  case 1:
+    if ((rows << g) / (64 * kWaves) <= kGroupOneRow)
+      launch_group_u<1, 1>(job, chunks, n_chunks, max_tokens, g, bytes, nt, stream);
+    else
+      launch_group_u<1, 2>(job, chunks, n_chunks, max_tokens, g, bytes, nt, stream);
+    return true;
+  case 3: launch_group_u<3, 1>(job, chunks, n_chunks, max_tokens, g, bytes, nt, stream); return true;
+  case 5: launch_group_u<5, 1>(job, chunks, n_chunks, max_tokens, g, bytes, nt, stream); return true;
+  case 7: launch_group_u<7, 1>(job, chunks, n_chunks, max_tokens, g, bytes, nt, stream); return true;
+  case 9:
+    if (job.page2lmc != 0 && bytes > kGroupNineStore) return false;
+    launch_group_u<9, 1>(job, chunks, n_chunks, max_tokens, g, bytes, nt, stream);
+    return true;
+  default: return false;
+  }
+}
+
 template <int VEC>
 void launch_vec(const CopyJob &job_in, const ChunkList &chunks, int n_chunks,
                 int max_rows, bool nt, bool host_lmc, hipStream_t stream) {
@@ -592,6 +794,22 @@ void launch_vec(const CopyJob &job_in, const ChunkList &chunks, int n_chunks,
   // launches keep the general row kernel, which moved them 3-6% faster on
   // MI355X (8B shape, 16 objects; one 32768-token Qwen3-32B-shape layer).
   lean = lean && ((n_chunks == 1 && max_rows <= LMC_KV_LEAN_MAX_ROWS) || LMC_KV_LEAN_BATCH);
+  // Rows that are not whole slices: the group kernel where every plane's row
+  // has its form.
+  bool group = VEC == 16 && !whole_slices && (job.block_size == 0 || pow2(job.block_size)) && max_rows < (1 << 30);
+  for (int p = 0; p < job.n_planes; ++p)
+    group = group && job.plane[p].row_bytes == widest && job.table_idx[p] == p * job.idx_step;
+  if (group) {
+    CopyJob g = job;
+    if (g.block_size > 0) {
+      g.bs_shift = __builtin_ctzll(static_cast<uint64_t>(g.block_size));
+    } else {
+      // Flat rows as blocks of one row.
+      g.bs_shift = 0;
+      for (int p = 0; p < g.n_planes; ++p) g.plane[p].blk_stride = g.plane[p].row_pitch;
+    }
+    if (launch_group(g, chunks, n_chunks, max_rows / (job.n_planes * job.n_layers), widest, nt, stream)) return;
+  }
   if (lean) {
     job.spr_shift = __builtin_ctzll(static_cast<uint64_t>(job.slices_per_row));
     if (job.block_size > 0) {
