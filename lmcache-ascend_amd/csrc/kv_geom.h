@@ -66,13 +66,13 @@ typedef __attribute__((address_space(1))) u32x4 GlobalU32x4;
 // (agent) scope, which writes through the XCD's L2 instead of leaving the
 // line dirty there, so the kernel's end-of-launch L2 write-back has nothing
 // left to flush; without it (and for narrower vectors) the store carries the
-// streaming hint.  Measured on MI355X with two or more buffer sets in turn,
-// streaming -> written through: the row kernels, 1024-column rows, 32 layers
-// x 256 tokens 13.1 / 13.4 -> 12.1 / 12.1 us (store / retrieve), 80 x 256
-// 29.1 / 29.3 -> 26.7 / 27.0, 64 x 8192 690 / 699 -> 685 / 677; the tile
-// kernel's stores to memory objects (MLA-576 store) 402 -> 388 us, its
-// retrieves stream; the group kernel's line is at its launch; the direct
-// kernels measure the same.
+// streaming hint.  Which is faster depends on the kernel (MI355X): in
+// back-to-back calls the row and group kernels are 1-8% faster with streaming
+// stores up to 2 GB a call (32 layers x 256 tokens x 1024 columns 12.6 / 13.2
+// us against 13.1 / 13.7, store / retrieve), although a kernel that runs alone
+// is up to 10% faster written through; the tile kernel's stores to memory
+// objects are faster written through (MLA-576 store 0.388 -> 0.402 ms with
+// streaming stores), and the direct kernels measure the same.
 template <typename T, bool NT, bool WT = true> __device__ __forceinline__ void st(T *p, T v) {
   if constexpr (NT && WT && LMC_KV_WT_STORES && sizeof(T) == 16)
     __builtin_amdgcn_global_store_b128((GlobalU32x4 *)(p),

@@ -96,16 +96,18 @@ using ChunkList = ChunkListT<kMaxChunks>;
 
 
 // The work of block b of n: blocks are dispatched round-robin over the 8
-// XCDs, and each XCD takes one contiguous range of the work, so an XCD's
-// address translations cover its own eighth of the rows and not all of them.
-// Measured on MI355X, 1024-column rows, both directions (store / retrieve):
-// 64 layers x 8192 tokens with 128-token blocks 750 / 880 -> 671 / 672 us, 32
-// layers x 4096 tokens 190 / 222 -> 174 / 177 us; batches of 0.4 to 0.8 GB
-// are 1-2% slower, smaller ones the same.  (The tile kernel is up to 7%
-// slower with it and keeps the dispatch order.)
+// XCDs, and each XCD takes kXcdRun consecutive pieces of the work at a time
+// (512 KiB for the row kernel), so an XCD walks pages of its own instead of
+// every XCD touching every page.  Measured on MI355X, 1024-column rows, store
+// / retrieve: 64 layers x 8192 tokens with 128-token blocks 784 / 913 -> 669
+// / 674 us, 32 layers x 4096 tokens 190 / 222 -> 175 / 173, 32 x 2048 85 / 88
+// -> 84 / 86.  Runs of 16 and 256 pieces, or one run per XCD and object, lie
+// between (32 x 2048: 84 / 86, 84 / 88 and 87 / 89).  The tile kernel is up
+// to 7% slower with it and keeps the dispatch order.
+constexpr int kXcdRun = 64;
 __device__ __forceinline__ int xcd_block(int b, int n) {
-  const int per = n >> 3;
-  return b < 8 * per ? (b & 7) * per + (b >> 3) : b;
+  const int r = b & (8 * kXcdRun - 1), first = b - r;
+  return first + 8 * kXcdRun <= n ? first + (r & 7) * kXcdRun + (r >> 3) : b;
 }
 
 // Resolves row `row` of chunk `c` to (src, dst); returns the row's byte count,
@@ -158,7 +160,7 @@ __device__ __forceinline__ int64_t row_ptrs(const CopyJob &job, uint8_t *lmc,
 // (2 KiB with 16-byte accesses, a whole row at the Llama-3-8B shape).  A
 // wave owns kRowsPerWave items per pass: it resolves their addresses with
 // scalar work, issues every load, then every store.
-template <int VEC, bool NT, int NC, bool SLOT32, bool TABLE>
+template <int VEC, bool NT, bool WT, int NC, bool SLOT32, bool TABLE>
 __global__ void __launch_bounds__(kThreads)
     kv_rows_copy(const CopyJob job, const ChunkListT<NC> chunks) {
   using V = typename VecOf<VEC>::T;
@@ -224,7 +226,7 @@ __global__ void __launch_bounds__(kThreads)
 #pragma unroll
       for (int s = 0; s < kSegs; ++s) {
         const int64_t o = off0[r] + (s * 64 + lane) * VEC;
-        if (o < nb[r]) st<V, NT>(reinterpret_cast<V *>(dst[r] + o), v[r][s]);
+        if (o < nb[r]) st<V, NT, WT>(reinterpret_cast<V *>(dst[r] + o), v[r][s]);
       }
   }
 }
@@ -355,7 +357,7 @@ __global__ void __launch_bounds__(kThreads)
     if (live[r])
 #pragma unroll
       for (int s = 0; s < kSegs; ++s)
-        st<V, NT>(reinterpret_cast<V *>(dst[r] + (s * 64 + lane) * 16), v[r][s]);
+        st<V, NT, false>(reinterpret_cast<V *>(dst[r] + (s * 64 + lane) * 16), v[r][s]);
 }
 
 // Group kernel, for rows of U x 2^g_shift 16-byte vectors, the same in every
@@ -372,14 +374,16 @@ __global__ void __launch_bounds__(kThreads)
 // row_pitch).
 //
 // Bound by latency for one object and by memory for a batch.  Against the
-// tile kernel, which took these rows before (MI355X, two or more buffer sets
-// in turn, store / retrieve): 80 layers x 199 tokens x 128 columns 7.1 / 9.6
-// -> 5.7 / 5.7 us, 4 x 256 x 64 4.9 / 5.6 -> 2.9 / 3.2, 32 x 256 x 896 13.2
-// / 17.0 -> 11.8 / 11.8, a 32768-token layer of 768 columns 33.2 / 42.3 ->
-// 30.7 / 30.8; batches: 32 x 2048 x 384 34.5 / 39.9 -> 31.6 / 31.7, 64 x 8192
-// x 512 360 / 419 -> 352 / 371.  A wave whose lanes take the wave's vectors
-// in address order, with a slot per access, was slower (32 x 256 x 896 17.5).
-template <bool NT, int NC, bool WT, int U, int R>
+// tile kernel, which took these rows before (MI355X, back-to-back calls over
+// several buffer sets, store / retrieve): 32 layers x 256 tokens x 768 columns
+// 12.9 / 16.7 -> 11.0 / 11.4 us, x 512 columns 9.1 / 15.0 -> 8.2 / 8.7; a
+// 4096-token layer of 512 columns 6.6 / 14.2 -> 5.6 / 5.7, 16384 x 768 20.8 /
+// 22.7 -> 19.2 / 19.9; kernels alone: 80 x 199 x 128 7.1 / 9.6 -> 5.7 / 5.7,
+// 4 x 256 x 64 4.9 / 5.6 -> 2.9 / 3.2; batches: 64 x 8192 x 512 360 / 419 ->
+// 354 / 370.  A wave whose lanes take the wave's vectors in address order,
+// with a slot per access, was slower (32 x 256 x 896 17.5 against 11.8), and
+// so were stores written through (32 x 256 x 512 8.9 / 9.1).
+template <bool NT, int NC, int U, int R>
 __global__ void __launch_bounds__(kThreads)
     kv_rows_group(const CopyJob job, const ChunkListT<NC> chunks, int g_shift, int linear) {
   using V = u32x4;
@@ -478,7 +482,7 @@ __global__ void __launch_bounds__(kThreads)
     if (live[r])
 #pragma unroll
       for (int u = 0; u < U; ++u)
-        st<V, NT, WT>(reinterpret_cast<V *>(dst[r]) + (static_cast<int64_t>(u) << g_shift), v[r][u]);
+        st<V, NT, false>(reinterpret_cast<V *>(dst[r]) + (static_cast<int64_t>(u) << g_shift), v[r][u]);
 }
 
 // Tile kernel.  A wave owns a tile of up to 64 consecutive tokens of one
@@ -638,22 +642,31 @@ ChunkListT<1> first_chunk(const ChunkList &cl) {
   return one;
 }
 
+// The row kernel's stores are written through in copies larger than this
+// and stream in smaller ones (store / retrieve, back-to-back calls over
+// several buffer sets, streaming -> written through): 4.3 GB 675 / 697 -> 668
+// / 673 us, 2.1 GB 328 / 333 -> 328 / 338, 1.1 GB 164 / 167 -> 164 / 171, 157
+// MB 27.7 / 28.4 -> 28.3 / 30.0.
+constexpr int64_t kRowsWriteThrough = int64_t(3) << 30;
+
 template <int VEC, int NC, bool SLOT32, bool TABLE>
-void launch_rows_st(const CopyJob &job, const ChunkListT<NC> &chunks, dim3 grid, dim3 block, bool nt,
+void launch_rows_st(const CopyJob &job, const ChunkListT<NC> &chunks, dim3 grid, dim3 block, bool nt, bool wt,
                     hipStream_t stream) {
-  if (nt) hipLaunchKernelGGL((kv_rows_copy<VEC, true, NC, SLOT32, TABLE>), grid, block, 0, stream, job, chunks);
-  else hipLaunchKernelGGL((kv_rows_copy<VEC, false, NC, SLOT32, TABLE>), grid, block, 0, stream, job, chunks);
+  const auto kern = !nt                ? kv_rows_copy<VEC, false, false, NC, SLOT32, TABLE>
+                    : wt && VEC == 16 ? kv_rows_copy<VEC, true, VEC == 16, NC, SLOT32, TABLE>
+                                       : kv_rows_copy<VEC, true, false, NC, SLOT32, TABLE>;
+  hipLaunchKernelGGL(kern, grid, block, 0, stream, job, chunks);
 }
 
 template <int VEC, int NC>
-void launch_rows(const CopyJob &job, const ChunkListT<NC> &chunks, dim3 grid, dim3 block, bool nt,
+void launch_rows(const CopyJob &job, const ChunkListT<NC> &chunks, dim3 grid, dim3 block, bool nt, bool wt,
                  hipStream_t stream) {
   if (job.slot_i32) {
-    if (job.table != nullptr) launch_rows_st<VEC, NC, true, true>(job, chunks, grid, block, nt, stream);
-    else launch_rows_st<VEC, NC, true, false>(job, chunks, grid, block, nt, stream);
+    if (job.table != nullptr) launch_rows_st<VEC, NC, true, true>(job, chunks, grid, block, nt, wt, stream);
+    else launch_rows_st<VEC, NC, true, false>(job, chunks, grid, block, nt, wt, stream);
   } else {
-    if (job.table != nullptr) launch_rows_st<VEC, NC, false, true>(job, chunks, grid, block, nt, stream);
-    else launch_rows_st<VEC, NC, false, false>(job, chunks, grid, block, nt, stream);
+    if (job.table != nullptr) launch_rows_st<VEC, NC, false, true>(job, chunks, grid, block, nt, wt, stream);
+    else launch_rows_st<VEC, NC, false, false>(job, chunks, grid, block, nt, wt, stream);
   }
 }
 
@@ -693,12 +706,6 @@ void launch_lean(const CopyJob &job, const ChunkList &chunks, int n_chunks,
   else launch_lean_t<kMaxChunks>(job, chunks, grid, nt, stream);
 }
 
-// Where the group kernel's stores to the paged caches are written through
-// (see st()) and where they stream: copies that the 256 MB last-level cache
-// about holds are faster written through (268 MB, 32 layers x 2048 x 512:
-// 47.0 -> 40.3 us), larger ones the same to 4% slower (393 MB: 68.3 -> 69.7,
-// 537 MB: 96 -> 100).  Stores to memory objects are always written through.
-constexpr int64_t kGroupWriteThrough = int64_t(288) << 20;
 // Launches of more blocks than this (eight a CU) are laid out for xcd_block;
 // smaller ones skip its division.
 constexpr int64_t kGroupLinear = 2048;
@@ -714,7 +721,7 @@ constexpr int64_t kGroupNineStore = int64_t(1) << 30;
 
 template <int U, int R>
 void launch_group_u(const CopyJob &job, const ChunkList &chunks, int n_chunks, int64_t max_tokens, int g_shift,
-                    int64_t bytes, bool nt, hipStream_t stream) {
+                    bool nt, hipStream_t stream) {
   const int64_t per_block = static_cast<int64_t>(kWaves) * R * (64 >> g_shift);
   const int64_t groups = (max_tokens + per_block - 1) / per_block;
   const int64_t planes = static_cast<int64_t>(job.n_layers) * job.n_planes;
@@ -723,16 +730,13 @@ void launch_group_u(const CopyJob &job, const ChunkList &chunks, int n_chunks, i
   const dim3 grid = linear ? dim3(static_cast<unsigned>(groups * planes), n_chunks)
                            : dim3(static_cast<unsigned>(groups), static_cast<unsigned>(planes), n_chunks);
   const dim3 block(kThreads);
-  const bool wt = job.page2lmc != 0 || bytes <= kGroupWriteThrough;
   if (n_chunks == 1) {
     const ChunkListT<1> one = first_chunk(chunks);
-    const auto kern = nt ? (wt ? kv_rows_group<true, 1, true, U, R> : kv_rows_group<true, 1, false, U, R>)
-                         : kv_rows_group<false, 1, false, U, R>;
-    hipLaunchKernelGGL(kern, grid, block, 0, stream, job, one, g_shift, linear);
+    hipLaunchKernelGGL((nt ? kv_rows_group<true, 1, U, R> : kv_rows_group<false, 1, U, R>), grid, block, 0, stream,
+                       job, one, g_shift, linear);
   } else {
-    const auto kern = nt ? (wt ? kv_rows_group<true, kMaxChunks, true, U, R> : kv_rows_group<true, kMaxChunks, false, U, R>)
-                         : kv_rows_group<false, kMaxChunks, false, U, R>;
-    hipLaunchKernelGGL(kern, grid, block, 0, stream, job, chunks, g_shift, linear);
+    hipLaunchKernelGGL((nt ? kv_rows_group<true, kMaxChunks, U, R> : kv_rows_group<false, kMaxChunks, U, R>), grid,
+                       block, 0, stream, job, chunks, g_shift, linear);
   }
 }
 
@@ -746,20 +750,19 @@ bool launch_group(const CopyJob &job, const ChunkList &chunks, int n_chunks, int
   if (g < 3) return false;
   int64_t rows = 0;
   for (int c = 0; c < n_chunks; ++c) rows += static_cast<int64_t>(chunks.tok_count[c]) * job.n_layers * job.n_planes;
-  const int64_t bytes = 2 * rows * row_bytes;  // read and written
   switch (vecs >> g) {
   case 1:
     if ((rows << g) / (64 * kWaves) <= kGroupOneRow)
-      launch_group_u<1, 1>(job, chunks, n_chunks, max_tokens, g, bytes, nt, stream);
+      launch_group_u<1, 1>(job, chunks, n_chunks, max_tokens, g, nt, stream);
     else
-      launch_group_u<1, 2>(job, chunks, n_chunks, max_tokens, g, bytes, nt, stream);
+      launch_group_u<1, 2>(job, chunks, n_chunks, max_tokens, g, nt, stream);
     return true;
-  case 3: launch_group_u<3, 1>(job, chunks, n_chunks, max_tokens, g, bytes, nt, stream); return true;
-  case 5: launch_group_u<5, 1>(job, chunks, n_chunks, max_tokens, g, bytes, nt, stream); return true;
-  case 7: launch_group_u<7, 1>(job, chunks, n_chunks, max_tokens, g, bytes, nt, stream); return true;
+  case 3: launch_group_u<3, 1>(job, chunks, n_chunks, max_tokens, g, nt, stream); return true;
+  case 5: launch_group_u<5, 1>(job, chunks, n_chunks, max_tokens, g, nt, stream); return true;
+  case 7: launch_group_u<7, 1>(job, chunks, n_chunks, max_tokens, g, nt, stream); return true;
   case 9:
-    if (job.page2lmc != 0 && bytes > kGroupNineStore) return false;
-    launch_group_u<9, 1>(job, chunks, n_chunks, max_tokens, g, bytes, nt, stream);
+    if (job.page2lmc != 0 && 2 * rows * row_bytes > kGroupNineStore) return false;
+    launch_group_u<9, 1>(job, chunks, n_chunks, max_tokens, g, nt, stream);
     return true;
   default: return false;
   }
@@ -833,8 +836,12 @@ void launch_vec(const CopyJob &job_in, const ChunkList &chunks, int n_chunks,
     const int items_per_block = kWaves * kRowsPerWave;
     int gx = static_cast<int>((max_items + items_per_block - 1) / items_per_block);
     dim3 grid(std::max(1, std::min(gx, LMC_KV_GRID_CAP)), n_chunks);
-    if (n_chunks == 1) launch_rows<VEC>(job, first_chunk(chunks), grid, block, nt, stream);
-    else launch_rows<VEC>(job, chunks, grid, block, nt, stream);
+    int64_t bytes = 0;  // read and written
+    for (int p = 0; p < job.n_planes; ++p)
+      for (int c = 0; c < n_chunks; ++c) bytes += 2 * job.plane[p].row_bytes * chunks.tok_count[c] * job.n_layers;
+    const bool wt = bytes > kRowsWriteThrough;
+    if (n_chunks == 1) launch_rows<VEC>(job, first_chunk(chunks), grid, block, nt, wt, stream);
+    else launch_rows<VEC>(job, chunks, grid, block, nt, wt, stream);
   } else {
     // Narrower or odd rows: tiles of about 32 KiB of the widest plane,
     // 16..64 rows; a store between device buffers (paged reads) instead
