@@ -1628,118 +1628,99 @@ __global__ void __launch_bounds__(kDecLanes)
   decode_one_wave<Tab>(lds, cdf, bytes, nbytes, ends, T, C, nb, out, n_streams, lane);
 }
 
-// Decode of streams longer than the lane regions hold (n_bins <= 32, more
-// than kLaneMaxT tokens): one wave per 64 streams, the codes looked up in
-// cgdec::LongTables (chunks of more than 256 tokens have codes of up to 12
-// bits), the streams read through per-lane rings (cgdec::RingCursor), so the
-// LDS a block takes does not grow with the chunk.  A block takes kEpoch
+// Decode of chunks of more than kLaneMaxT tokens (n_bins <= 32).  Codes are
+// looked up in cgdec::LongTables (chunks of more than 256 tokens have codes
+// of up to 12 bits) and the streams are read through per-lane rings
+// (cgdec::RingCursorT), so the LDS this takes does not grow with the streams.
+// The line is at 256 tokens because calculate_cdf's codes are at most 8 bits
+// long up to there, which the byte tables and lane regions of decode_kernel
+// hold whole.
+constexpr int kLaneMaxT = 256;
+constexpr int kLongRing = cgdec::LongTables::kBytes;
+
+// A lane's stream in 16-byte aligned chunks from a0; `end` is the stream's
+// end from a0 in bytes.  Chunks 0 .. n_ch - 1 each hold a byte of the stream,
+// so no load leaves the buffer's pages.
+struct LaneChunks {
+  uintptr_t a0;
+  uint32_t off, end, n_ch;
+
+  __device__ __forceinline__ LaneChunks(const uint8_t *bytes, const DecBlock &bk) {
+    const uintptr_t s_lo = reinterpret_cast<uintptr_t>(bytes) + static_cast<uintptr_t>(bk.start);
+    const uint32_t len = static_cast<uint32_t>(bk.end - bk.start);
+    a0 = s_lo & ~uintptr_t(15);
+    off = static_cast<uint32_t>(s_lo - a0);
+    end = off + len;
+    n_ch = len ? (end + 15u) >> 4 : 0u;
+  }
+  __device__ __forceinline__ chunk16 load(uint32_t k) const {
+    chunk16 v = {0u, 0u, 0u, 0u};
+    if (k < n_ch) v = reinterpret_cast<global_chunk16 *>(a0)[k];
+    return v;
+  }
+  // Chunk k, its bytes past the stream's end zero, to slot `slot` of a ring
+  // of `dwords` dwords.
+  __device__ __forceinline__ void put(uint32_t *ring, uint32_t dwords, uint32_t slot, uint32_t k,
+                                      const chunk16 &v) const {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int left = static_cast<int>(end) - static_cast<int>(16u * k) - 4 * i;
+      const uint32_t x = i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w;
+      const uint32_t keep = left >= 4 ? ~0u : left <= 0 ? 0u : (1u << (8 * left)) - 1u;
+      ring[((4u * slot + static_cast<uint32_t>(i)) & (dwords - 1u)) * kDecLanes] = x & keep;
+    }
+  }
+};
+
+// One wave decodes a block's streams, one lane per stream.  It takes kEpoch
 // tokens at a time: the chunks that refill the ring over an epoch are loaded
 // at its start and stored at its end, so nothing waits for them.  A ring
 // holds 256 bytes; kEpoch codes of at most 16 bits take 64 of them, and an
 // epoch loads as many chunks as there is room for, up to 64 bytes, so at
 // least 100 bytes lie ahead of the cursor at the start of every epoch.
-// Bound by the serial chain of each stream (one wave per 64 streams): about
-// 220 cycles a code, two table reads and their select.  56 planes x 1000
-// tokens x 256 channels: 101 us; the shared-window kernel took 1307 us, since
-// the streams of a block outgrow its LDS window and were read a dword at a
-// time from memory, with a binary search per symbol after the first long code.
-// The line is at 256 tokens because calculate_cdf's codes are at most 8 bits
-// long up to there, which the byte tables and lane regions of decode_kernel
-// hold whole.
+// `irregular`: some row of the block takes the binary search.
+// Bound by the serial chain of each stream, about 210 cycles a code.
 constexpr int kEpoch = 32;
 constexpr int kEpochChunks = 4;  // 16-byte chunks per lane and epoch
 constexpr int kFirstChunks = 8;
-constexpr int kLaneMaxT = 256;
-constexpr int kLongRing = cgdec::LongTables::kBytes;
-constexpr int kLongObuf = kLongRing + static_cast<int>(cgdec::RingCursor::kBytes) * kDecLanes;
-constexpr int kLongRows = kLongObuf + kObufBytes;
-constexpr int long_lds_bytes(int nb) { return kLongRows + (((nb + 1) * kDecLanes * 2 + 32 + 15) & ~15); }
 
-__global__ void __launch_bounds__(kDecLanes)
-    decode_long_kernel(const int16_t *__restrict__ cdf, const uint8_t *__restrict__ bytes, int64_t nbytes,
-                       const StreamEnds ends, int T, int C, int nb, uint8_t *__restrict__ out,
-                       int64_t n_streams) {
-  extern __shared__ uint32_t lds_words[];
-  uint8_t *lds = reinterpret_cast<uint8_t *>(lds_words);
-  const uint32_t lds_at =
-      static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t *)lds));
-  const int lane = static_cast<int>(threadIdx.x);
-  DecBlock bk;
-  bk.init(cdf, nbytes, ends, n_streams, C, nb, lane);
-  const int nrow = static_cast<int>((bk.R1 - bk.r_lo + 15) >> 4);
-  chunk16 rv[kRowChunks], cv[kFirstChunks];
-  load_chunks(bk.r_lo, nrow, 0, lane, rv);
-  const uintptr_t s_lo = reinterpret_cast<uintptr_t>(bytes) + static_cast<uintptr_t>(bk.start);
-  const uint32_t len = static_cast<uint32_t>(bk.end - bk.start);
-  const uintptr_t a0 = s_lo & ~uintptr_t(15);
-  const uint32_t end = static_cast<uint32_t>(s_lo - a0) + len;  // the stream's end from a0
-  // Chunks [a0, a0 + 16 n_ch) each hold a byte of the stream, so no load
-  // leaves the buffer's pages.
-  const uint32_t n_ch = len ? (end + 15u) >> 4 : 0u;
-#pragma unroll
-  for (int u = 0; u < kFirstChunks; ++u)
-    if (static_cast<uint32_t>(u) < n_ch) cv[u] = reinterpret_cast<global_chunk16 *>(a0)[u];
-  cgdec::LongTables tb;
-  tb.bind(lds, lane, lds_at);
-  tb.clear();
-  store_chunks<false>(lds + kLongRows, nrow, 0, lane, rv);
-  for (int j0 = kDecLanes * kRowChunks; j0 < nrow; j0 += kDecLanes * kRowChunks) {
-    load_chunks(bk.r_lo, nrow, j0, lane, rv);
-    store_chunks<false>(lds + kLongRows, nrow, j0, lane, rv);
-  }
-  wave_sync();
-  tb.one.row.r = reinterpret_cast<const int16_t *>(lds + kLongRows + (bk.R0 - bk.r_lo)) +
-                 (lane < bk.cnt ? lane : 0) * (nb + 1);
-  tb.one.nb = nb;
-  uint8_t *obuf = lds + kLongObuf;
-  tb.build(obuf + lane);
-  // Dword d of the stream's chunks with its bytes past the stream's end zero,
-  // to the ring.
-  uint32_t *ring = reinterpret_cast<uint32_t *>(lds + kLongRing) + lane;
+__device__ __forceinline__ void decode_serial(cgdec::LongTables &tb, bool irregular, const DecBlock &bk,
+                                              const LaneChunks &ch, uint8_t *lds, uint32_t lds_at, int ring_off,
+                                              uint8_t *obuf, int T, int C, int lane, uint8_t *__restrict__ out) {
+  uint32_t *ring = reinterpret_cast<uint32_t *>(lds + ring_off) + lane;
   constexpr uint32_t kRingDw = cgdec::RingCursor::kBytes / 4;
-  auto put = [&](uint32_t chunk, const chunk16 &v) {
+  {
+    chunk16 cv[kFirstChunks];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t d = 4u * chunk + static_cast<uint32_t>(i);
-      const int left = static_cast<int>(end) - static_cast<int>(4u * d);
-      const uint32_t x = i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w;
-      const uint32_t keep = left >= 4 ? ~0u : left <= 0 ? 0u : (1u << (8 * left)) - 1u;
-      ring[(d & (kRingDw - 1u)) * kDecLanes] = x & keep;
-    }
-  };
-  chunk16 zero = {0u, 0u, 0u, 0u};
+    for (uint32_t u = 0; u < kFirstChunks; ++u) cv[u] = ch.load(u);
 #pragma unroll
-  for (int u = 0; u < kFirstChunks; ++u) put(static_cast<uint32_t>(u), static_cast<uint32_t>(u) < n_ch ? cv[u] : zero);
+    for (uint32_t u = 0; u < kFirstChunks; ++u) ch.put(ring, kRingDw, u, u, cv[u]);
+  }
   uint32_t filled = kFirstChunks;  // chunks in the ring or before it
   wave_sync();
   const DecBlock::Quad quad = bk.quad(out, T, C, lane);
   uint32_t *odst = quad.dst;
   const int64_t step4 = static_cast<int64_t>(C);  // in dwords: 4 tokens of C bytes
   const int groups = (T + 3) / 4;
-  const uint32_t first_bit = 8u * static_cast<uint32_t>(s_lo - a0);
-  const uint32_t column = lds_at + kLongRing + 4u * static_cast<uint32_t>(lane);
-  // The chunks of one epoch: loads, then (after its tokens) the ring.
+  const uint32_t column = lds_at + static_cast<uint32_t>(ring_off) + 4u * static_cast<uint32_t>(lane);
   chunk16 nv[kEpochChunks];
   uint32_t room = 0;
   auto load_epoch = [&](uint32_t q) {
     room = (cgdec::RingCursor::kBytes - (16u * filled - q)) >> 4;
     room = room < kEpochChunks ? room : kEpochChunks;
 #pragma unroll
-    for (uint32_t u = 0; u < kEpochChunks; ++u) {
-      nv[u] = zero;
-      if (u < room && filled + u < n_ch) nv[u] = reinterpret_cast<global_chunk16 *>(a0)[filled + u];
-    }
+    for (uint32_t u = 0; u < kEpochChunks; ++u) nv[u] = ch.load(u < room ? filled + u : ~0u);
   };
   auto store_epoch = [&]() {
 #pragma unroll
     for (uint32_t u = 0; u < kEpochChunks; ++u)
-      if (u < room) put(filled + u, nv[u]);
+      if (u < room) ch.put(ring, kRingDw, filled + u, filled + u, nv[u]);
     filled += room;
     wave_sync();
   };
-  if (!__any(tb.irregular)) {
+  if (!irregular) {
     cgdec::PairCursor cur;
-    cur.start(tb, column, first_bit);
+    cur.start(tb, column, 8u * ch.off);
     uint32_t word = 0;
     // Four tokens; each transposed word is stored one group late, as in
     // decode_one_wave_lanes.
@@ -1772,7 +1753,7 @@ __global__ void __launch_bounds__(kDecLanes)
   } else {
     tb.one.finish();
     cgdec::RingCursor cur;
-    cur.start(column, first_bit);
+    cur.start(column, 8u * ch.off);
     for (int g = 0; g < groups; ++g) {
       if (g % (kEpoch / 4) == 0) load_epoch(cur.q);
 #pragma unroll
@@ -1789,6 +1770,326 @@ __global__ void __launch_bounds__(kDecLanes)
       if (g % (kEpoch / 4) == kEpoch / 4 - 1) store_epoch();
     }
   }
+}
+
+constexpr int kLongObuf = kLongRing + static_cast<int>(cgdec::RingCursor::kBytes) * kDecLanes;
+constexpr int kLongRows = kLongObuf + kObufBytes;
+constexpr int rows_lds_bytes(int nb) { return ((nb + 1) * kDecLanes * 2 + 32 + 15) & ~15; }
+
+// Any length, one wave per block (56 planes x 1000 tokens x 256 channels: 100
+// us, where the shared-window kernel took 1307 us: the streams of a block
+// outgrow its LDS window and were read a dword at a time from memory, with a
+// binary search per symbol after the table's first long code).
+__global__ void __launch_bounds__(kDecLanes)
+    decode_long_kernel(const int16_t *__restrict__ cdf, const uint8_t *__restrict__ bytes, int64_t nbytes,
+                       const StreamEnds ends, int T, int C, int nb, uint8_t *__restrict__ out,
+                       int64_t n_streams) {
+  extern __shared__ uint32_t lds_words[];
+  uint8_t *lds = reinterpret_cast<uint8_t *>(lds_words);
+  const uint32_t lds_at =
+      static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t *)lds));
+  const int lane = static_cast<int>(threadIdx.x);
+  DecBlock bk;
+  bk.init(cdf, nbytes, ends, n_streams, C, nb, lane);
+  const int nrow = static_cast<int>((bk.R1 - bk.r_lo + 15) >> 4);
+  chunk16 rv[kRowChunks];
+  load_chunks(bk.r_lo, nrow, 0, lane, rv);
+  const LaneChunks ch(bytes, bk);
+  cgdec::LongTables tb;
+  tb.bind(lds, lane, lds_at);
+  tb.clear();
+  store_chunks<false>(lds + kLongRows, nrow, 0, lane, rv);
+  for (int j0 = kDecLanes * kRowChunks; j0 < nrow; j0 += kDecLanes * kRowChunks) {
+    load_chunks(bk.r_lo, nrow, j0, lane, rv);
+    store_chunks<false>(lds + kLongRows, nrow, j0, lane, rv);
+  }
+  wave_sync();
+  tb.one.row.r = reinterpret_cast<const int16_t *>(lds + kLongRows + (bk.R0 - bk.r_lo)) +
+                 (lane < bk.cnt ? lane : 0) * (nb + 1);
+  tb.one.nb = nb;
+  uint8_t *obuf = lds + kLongObuf;
+  tb.build(lds_at + static_cast<uint32_t>(kLongObuf + lane));
+  decode_serial(tb, __any(tb.irregular) != 0, bk, ch, lds, lds_at, kLongRing, obuf, T, C, lane, out);
+}
+
+// Split decode: four waves per block of 64 streams, each taking a quarter of
+// every stream (lane = stream).  Where a quarter's codes start is not stored,
+// so waves 1 to 3 begin at the bit where it should lie, less `warm` codes,
+// and decode those without keeping them: prefix codes resynchronise (Gaussian
+// data at 16 / 32 bins: 99.9% of decoders started anywhere are on the true
+// boundaries after 12 / 28 codes).  Each wave then keeps its symbols, in LDS
+// and in a column of the lane's, until it passes the bit the next wave began
+// keeping at.  If it stopped on that bit in every lane, the next wave was on
+// the boundaries; otherwise that wave decodes again from where it did stop,
+// so after at most three more rounds every quarter follows from the one
+// before, whatever the streams hold.  The symbols' counts then place the
+// quarters, and the waves write the block's tokens, each gathering four
+// streams' symbols per dword.
+//   A lane takes a long code in two table lookups (cgdec::StepCursor), so the
+// lanes are not on the same symbol, which the columns do not need.
+//   Bound by the steps' dependent instructions, about 213 cycles a step with
+// one wave per SIMD.  56 planes x 1000 tokens x 256 channels on MI355X: 58 us,
+// 100 us with one wave per block; of its 128k cycles 24k build the tables,
+// 71k decode and 25k write the tokens out.  Writing the symbols in rows of 64
+// bytes ([n][lane], up to four lanes on a bank) and gathering each dword of
+// the output from four streams byte by byte took 62 us.
+//   Blocks with an irregular row, with a stream that ends before its T
+// symbols, or with a quarter that outgrows its rows of the buffer (codes
+// bunched at one end) are decoded by one wave (decode_serial).
+struct SplitPlan {
+  int first, rest;          // tokens wave 0 and each other wave are meant to take
+  int warm;                 // codes decoded before a later wave's own, a multiple of 16
+  int cap0, cap;            // rows of the buffers of wave 0 and of each other wave
+  int meta_off, rows_off, lds;
+};
+constexpr int kSplit = 4;
+constexpr int kSplitThreads = kSplit * kDecLanes;
+constexpr int kSplitSteps = 16;  // steps per epoch: at most 16 bytes of the ring
+constexpr int kSplitRing = static_cast<int>(cgdec::StepCursor::Ring::kBytes) * kDecLanes;
+constexpr int kSplitBuf = kLongRing + kSplit * kSplitRing;
+constexpr int kSplitFlags = 16;
+// Its LDS holds chunks of up to kSplitMaxT tokens, and leaves one block on a
+// CU where decode_long_kernel has three, so it takes launches that leave it a
+// CU per block, and chunks long enough for the codes decoded before each
+// quarter's own not to matter (300 tokens, 96 blocks: 42 us against 39 for one
+// wave per block; 512 tokens, 512 blocks: 90 against 60; 1000 tokens, 224
+// blocks: 58 against 100).
+constexpr int kSplitMaxT = 1024;
+constexpr int kSplitMinT = 385;
+constexpr int kSplitMaxBlocks = 256;
+inline SplitPlan split_plan(int T, int nb) {
+  SplitPlan p;
+  p.warm = T <= 400 ? 32 : T <= 700 ? 48 : 64;
+  // Every wave decodes about as much: wave 0 has no codes before its own.
+  p.first = (T + 3 * p.warm + 3) / 4;
+  p.rest = std::max(p.first - p.warm, 0);
+  const auto cap = [](int n) { return (n + n / 8 + 32 + kSplitSteps - 1) / kSplitSteps * kSplitSteps; };
+  p.cap0 = cap(p.first);
+  p.cap = cap(p.rest);
+  p.meta_off = kSplitBuf + (p.cap0 + 3 * p.cap) * kDecLanes;
+  p.rows_off = p.meta_off + 4 * (3 * kSplit * kDecLanes + kSplitFlags);
+  p.lds = p.rows_off + rows_lds_bytes(nb);
+  return p;
+}
+
+// First row of wave w's buffer (rows of 64 bytes).
+__device__ __forceinline__ int split_base(const SplitPlan &p, int w) {
+  return w == 0 ? 0 : p.cap0 + (w - 1) * p.cap;
+}
+
+__global__ void __launch_bounds__(kSplitThreads)
+    decode_split_kernel(const int16_t *__restrict__ cdf, const uint8_t *__restrict__ bytes, int64_t nbytes,
+                        const StreamEnds ends, int T, int C, int nb, uint8_t *__restrict__ out, int64_t n_streams,
+                        const SplitPlan plan) {
+  extern __shared__ uint32_t lds_words[];
+  uint8_t *lds = reinterpret_cast<uint8_t *>(lds_words);
+  const uint32_t lds_at =
+      static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t *)lds));
+  const int lane = static_cast<int>(threadIdx.x) & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  uint32_t *starts = reinterpret_cast<uint32_t *>(lds + plan.meta_off);  // [wave][lane]: where its symbols start
+  uint32_t *stops = starts + kSplit * kDecLanes;                         // first boundary past its end
+  uint32_t *counts = stops + kSplit * kDecLanes;
+  // [0]: an irregular row; [1 + 2 r], [2 + 2 r]: round r left a wave off its
+  // boundaries, a wave out of room (each written in its own round, so that
+  // every wave reads the same).
+  uint32_t *flags = counts + kSplit * kDecLanes;
+  DecBlock bk;
+  bk.init(cdf, nbytes, ends, n_streams, C, nb, lane);
+  const bool live = lane < bk.cnt;
+  const LaneChunks ch(bytes, bk);
+  // T codes of at most 12 bits end before 2 T bytes: longer streams are of no
+  // use, and their bits would not fit 32 bits.
+  const uint32_t len = ch.n_ch ? ch.end - ch.off : 0u;
+  const uint32_t most = 2u * static_cast<uint32_t>(T) + 8u;
+  const uint32_t stream_bits = 8u * (len < most ? len : most);
+
+  // The segment's ring: local chunk 0 is the chunk of its first bit.
+  uint32_t *ring = reinterpret_cast<uint32_t *>(lds + kLongRing + wave * kSplitRing) + lane;
+  constexpr uint32_t kRingDw = cgdec::StepCursor::Ring::kBytes / 4;
+  const uint32_t column = lds_at + static_cast<uint32_t>(kLongRing + wave * kSplitRing) + 4u * static_cast<uint32_t>(lane);
+  uint32_t guess = static_cast<uint32_t>(static_cast<float>(stream_bits) * static_cast<float>(wave * plan.rest) /
+                                         static_cast<float>(T));
+  guess = guess < stream_bits ? guess : stream_bits;
+  uint32_t chunk0 = (8u * ch.off + guess) >> 7, filled = 0;
+  chunk16 cv[kFirstChunks];
+  auto load_first = [&]() {
+#pragma unroll
+    for (uint32_t u = 0; u < kFirstChunks; ++u) cv[u] = ch.load(chunk0 + u);
+  };
+  auto put_first = [&]() {
+#pragma unroll
+    for (uint32_t u = 0; u < kFirstChunks; ++u) ch.put(ring, kRingDw, u, chunk0 + u, cv[u]);
+    filled = kFirstChunks;
+    wave_sync();
+  };
+  load_first();
+
+  // Tables: cleared by every wave, marked by wave 0, scanned by all, the
+  // markers put in by wave 0.
+  cgdec::LongTables tb;
+  tb.bind(lds, lane, lds_at);
+  {
+    uint32_t *t32 = reinterpret_cast<uint32_t *>(tb.one.tab);
+    for (int d = wave * (128 / kSplit); d < (wave + 1) * (128 / kSplit); ++d) t32[d * kDecLanes] = 0;
+    const int nrow = static_cast<int>((bk.R1 - bk.r_lo + 15) >> 4);
+    for (int j = static_cast<int>(threadIdx.x); j < nrow; j += kSplitThreads)
+      reinterpret_cast<chunk16 *>(lds + plan.rows_off)[j] = reinterpret_cast<global_chunk16 *>(bk.r_lo)[j];
+    if (threadIdx.x < kSplitFlags) flags[threadIdx.x] = 0;
+  }
+  __syncthreads();
+  tb.one.row.r = reinterpret_cast<const int16_t *>(lds + plan.rows_off + (bk.R0 - bk.r_lo)) +
+                 (live ? lane : 0) * (nb + 1);
+  tb.one.nb = nb;
+  const uint32_t dummy = lds_at + static_cast<uint32_t>(kSplitBuf + lane);  // scratch for skipped writes
+  if (wave == 0) {
+    tb.mark(dummy);
+    if (__any(tb.irregular) && lane == 0) flags[0] = 1;
+  } else {
+    put_first();
+  }
+  __syncthreads();
+  if (wave == 0) tb.one.scan(0, 64, 0);
+  else tb.scan_second(wave - 1, kSplit - 1);
+  __syncthreads();
+  if (wave == 0) {
+    tb.escapes(dummy);
+    put_first();
+  }
+  __syncthreads();
+
+  bool one_wave = flags[0] != 0;  // the same in every wave, here and below
+  if (!one_wave) {
+    cgdec::StepCursor cur;
+    cur.start(tb, column, (8u * ch.off + guess) & 127u, guess);
+    auto epoch = [&](uint32_t to, auto &&each) {
+      // One chunk of room or more: the chunk read ahead over the epoch.
+      const bool room = 16u * filled - cur.ring.q <= cgdec::StepCursor::Ring::kBytes - 16u;
+      const chunk16 nv = ch.load(room ? chunk0 + filled : ~0u);
+#pragma unroll
+      for (int i = 0; i < kSplitSteps / 2; ++i) cur.pair(tb, to, each);
+      if (room) {
+        ch.put(ring, kRingDw, filled, chunk0 + filled, nv);
+        ++filled;
+      }
+      wave_sync();
+    };
+    if (wave > 0)
+      for (int w = 0; w < plan.warm; w += kSplitSteps) epoch(~0u, [](uint32_t, bool) {});
+    uint32_t start = cur.bd;
+    starts[wave * kDecLanes + lane] = start;
+    __syncthreads();
+    const uint32_t hi = wave + 1 < kSplit ? starts[(wave + 1) * kDecLanes + lane] : stream_bits;
+    const int cap = wave == 0 ? plan.cap0 : plan.cap;
+    const uint32_t buf = lds_at + static_cast<uint32_t>(kSplitBuf + split_base(plan, wave) * kDecLanes + 4 * lane);
+    bool run = true;
+    for (int round = 0;; ++round) {
+      if (run) {
+        // Symbol n of the lane is byte n % 4 of dword n / 4 of its column
+        // (dwords [n / 4][lane]: every lane in its own bank).
+        uint32_t n = 0;
+        for (int steps = 0; steps < cap && __any(cur.bd < hi); steps += kSplitSteps)
+          epoch(hi, [&](uint32_t e, bool counts) {
+            cgdec::lds_set_byte(buf + (n << 6) - 63u * (n & 3u), e >> 3);
+            n += counts ? 1u : 0u;
+          });
+        if (__any(live && cur.bd < hi) && lane == 0) flags[2 + 2 * round] = 1;
+        stops[wave * kDecLanes + lane] = cur.bd;
+        counts[wave * kDecLanes + lane] = n;
+      }
+      __syncthreads();
+      const uint32_t before = wave > 0 ? stops[(wave - 1) * kDecLanes + lane] : 0u;
+      const bool off_bound = wave > 0 && live && before != start;
+      run = __any(off_bound) != 0;
+      if (run && lane == 0) flags[1 + 2 * round] = 1;
+      __syncthreads();
+      const bool again = flags[1 + 2 * round] != 0;
+      one_wave = flags[2 + 2 * round] != 0 || (again && round + 1 == kSplit);
+      if (one_wave || !again) break;
+      if (run) {
+        start = off_bound ? before : start;
+        chunk0 = (8u * ch.off + start) >> 7;
+        load_first();
+        put_first();
+        cur.start(tb, column, (8u * ch.off + start) & 127u, start);
+      }
+    }
+    uint32_t symbols = 0;
+#pragma unroll
+    for (int w = 0; w < kSplit; ++w) symbols += counts[w * kDecLanes + lane];
+    one_wave = one_wave || __any(live && symbols < static_cast<uint32_t>(T)) != 0;
+  }
+  if (one_wave) {
+    __syncthreads();
+    if (wave == 0)
+      decode_serial(tb, flags[0] != 0, bk, ch, lds, lds_at, kLongRing, lds + kSplitBuf, T, C, lane, out);
+    return;
+  }
+  // The tokens, four at a time, a quarter of them per wave; lane = stream.  A
+  // lane's four symbols are four bytes of its column, two dwords shifted
+  // together, unless its tokens lie in two quarters; the dwords go through
+  // the transpose in the wave's (dead) ring and are stored one group late.
+  uint32_t until[kSplit];  // tokens up to the end of quarter k
+  uint32_t t0 = 0;
+#pragma unroll
+  for (int k = 0; k < kSplit; ++k) {
+    t0 += counts[k * kDecLanes + lane];
+    // (a lane without a stream: rows inside the buffers)
+    until[k] = live ? t0 : static_cast<uint32_t>(T);
+  }
+  // LDS byte of the lane's symbol of token t.
+  const uint32_t column0 = lds_at + static_cast<uint32_t>(kSplitBuf + 4 * lane);
+  auto place = [&](uint32_t t, uint32_t &row) {  // returns the quarter's first row in the buffers
+    uint32_t base = 0, before = 0;
+#pragma unroll
+    for (int k = 0; k + 1 < kSplit; ++k) {
+      const bool past = t >= until[k];
+      base = past ? static_cast<uint32_t>(split_base(plan, k + 1)) : base;
+      before = past ? until[k] : before;
+    }
+    row = t - before;
+    return base;
+  };
+  auto end_of = [&](uint32_t t) {
+    uint32_t e = until[0];
+#pragma unroll
+    for (int k = 0; k + 1 < kSplit; ++k) e = t >= until[k] ? until[k + 1] : e;
+    return e;
+  };
+  const DecBlock::Quad quad = bk.quad(out, T, C, lane);
+  uint8_t *obuf = lds + kLongRing + wave * kSplitRing;
+  const int groups = (T + 3) / 4, share = (groups + kSplit - 1) / kSplit;
+  const int g1 = (wave + 1) * share < groups ? (wave + 1) * share : groups;
+  uint32_t word = 0;
+  int stored = wave * share;  // groups stored
+  for (int g = wave * share; g < g1; ++g) {
+    const uint32_t t = 4u * static_cast<uint32_t>(g);
+    uint32_t row;
+    const uint32_t base = place(t, row);
+    const uint32_t at = column0 + (base + (row & ~3u)) * kDecLanes;
+    uint32_t four = __builtin_amdgcn_alignbyte(cgdec::lds_dword(at + 4u * kDecLanes), cgdec::lds_dword(at), row & 3u);
+    if (__any(live && end_of(t) < t + 4u)) {
+      four = 0;
+#pragma unroll
+      for (uint32_t i = 0; i < 4; ++i) {
+        uint32_t r;
+        // Tokens past T: any byte of the column.
+        const uint32_t b = place(t + i < static_cast<uint32_t>(T) ? t + i : t, r);
+        const uint32_t d = cgdec::lds_dword(column0 + (b + (r & ~3u)) * kDecLanes);
+        four |= ((d >> (8u * (r & 3u))) & 0xFFu) << (8u * i);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) obuf[i * kDecLanes + lane] = static_cast<uint8_t>(four >> (8 * i));
+    if (g > stored) {
+      cg_st(quad.dst + static_cast<int64_t>(stored) * C, word);
+      ++stored;
+    }
+    wave_sync();
+    word = reinterpret_cast<const uint32_t *>(obuf)[quad.at];
+    wave_sync();
+  }
+  if (stored < g1 && 4 * stored + (quad.at >> 4) < T) cg_st(quad.dst + static_cast<int64_t>(stored) * C, word);
 }
 
 // Exclusive prefix sums of the blocks' byte counts, in one workgroup: off[b]
@@ -2120,16 +2421,28 @@ void decode_streams(const lmc_tensor &cdf, const lmc_tensor &bs, const lmc_tenso
                        ends.lens, n_streams, blocks, b, b + blocks);
     hip_check(hipGetLastError(), "length_sums_kernel launch");
   }
-  const bool long_streams = nb <= cgdec::ByteTables::kMaxBins && T > kLaneMaxT &&
-                            (reinterpret_cast<uintptr_t>(o.data) & 3) == 0;
-  const auto kern = long_streams                          ? decode_long_kernel
-                    : nb <= cgdec::ByteTables::kMaxBins ? decode_kernel<cgdec::ByteTables>
-                                                          : decode_kernel<DecTables>;
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(kDecLanes),
-                     long_streams ? long_lds_bytes(static_cast<int>(nb)) : kDecLds, stream,
-                     static_cast<const int16_t *>(cdf.data),
-                     static_cast<const uint8_t *>(bs.data), numel(bs), ends, (int)T, (int)C,
-                     (int)nb, static_cast<uint8_t *>(o.data), n_streams);
+  const int16_t *rows = static_cast<const int16_t *>(cdf.data);
+  const uint8_t *bytes = static_cast<const uint8_t *>(bs.data);
+  uint8_t *out = static_cast<uint8_t *>(o.data);
+  const dim3 grid(static_cast<unsigned>(blocks));
+  if (nb <= cgdec::ByteTables::kMaxBins && T > kLaneMaxT && (reinterpret_cast<uintptr_t>(out) & 3) == 0) {
+    if (T >= kSplitMinT && T <= kSplitMaxT && blocks <= kSplitMaxBlocks) {
+      const SplitPlan plan = split_plan(static_cast<int>(T), static_cast<int>(nb));
+      hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(decode_split_kernel),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, plan.lds),
+                "decode LDS size");
+      hipLaunchKernelGGL(decode_split_kernel, grid, dim3(kSplitThreads), plan.lds, stream, rows, bytes, numel(bs), ends,
+                         (int)T, (int)C, (int)nb, out, n_streams, plan);
+    } else {
+      hipLaunchKernelGGL(decode_long_kernel, grid, dim3(kDecLanes),
+                         kLongRows + rows_lds_bytes(static_cast<int>(nb)), stream, rows, bytes, numel(bs), ends,
+                         (int)T, (int)C, (int)nb, out, n_streams);
+    }
+  } else {
+    hipLaunchKernelGGL(nb <= cgdec::ByteTables::kMaxBins ? decode_kernel<cgdec::ByteTables> : decode_kernel<DecTables>,
+                       grid, dim3(kDecLanes), kDecLds, stream, rows, bytes, numel(bs), ends, (int)T, (int)C, (int)nb,
+                       out, n_streams);
+  }
   hip_check(hipGetLastError(), "decode_kernel launch");
 }
 

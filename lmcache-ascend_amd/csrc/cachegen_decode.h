@@ -20,6 +20,9 @@ constexpr int kPrec = 16;
 __device__ __forceinline__ uint32_t lds_dword(uint32_t at) {
   return *reinterpret_cast<const __attribute__((address_space(3))) uint32_t *>(static_cast<uintptr_t>(at));
 }
+__device__ __forceinline__ void lds_set_byte(uint32_t at, uint32_t v) {
+  *reinterpret_cast<__attribute__((address_space(3))) uint8_t *>(static_cast<uintptr_t>(at)) = static_cast<uint8_t>(v);
+}
 // Byte k of the result is byte sel.byte[k] (0..7) of the 64-bit hi:lo.
 __device__ __forceinline__ uint32_t byte_perm(uint32_t hi, uint32_t lo, uint32_t sel) {
   return __builtin_amdgcn_perm(hi, lo, sel);
@@ -47,6 +50,7 @@ inline const uint8_t *&host_lds_base() {
   static const uint8_t *base = nullptr;
   return base;
 }
+inline void lds_set_byte(uint32_t at, uint32_t v) { const_cast<uint8_t *>(host_lds_base())[at] = static_cast<uint8_t>(v); }
 inline uint32_t lds_dword(uint32_t at) {
   uint32_t v;
   __builtin_memcpy(&v, host_lds_base() + at, 4);
@@ -588,28 +592,33 @@ struct GroupCursor {
   }
 };
 
-// Two tables for streams with codes of up to 15 bits (n_bins <= 32): the
+// Two tables for streams with codes of up to 12 bits (n_bins <= 32): the
 // byte table above, and behind it a second one of the same layout indexed by
 // window bits 4 .. 11.  A prefix of the first table that holds longer codes
-// is kEscape there and its window is looked up in the second table, whose
-// entry is (s << 3) | (length - 8).  The two indexes come from the window
-// alone, so both tables are read at once and a long code costs a select.
+// has kMarker there and its window is looked up in the second table, whose
+// entry is (s << 3) | (length - 5).  Read as an entry, the marker is a code of
+// 4 bits, after which the next 8 bits index the second table and its entry
+// holds the rest of the code: a decoder may either look a window up in both
+// tables at once (PairCursor) or take a long code in two lookups of the same
+// form (StepCursor).
 //
 // The second table has 256 entries for the 4096 12-bit prefixes: prefix p of
 // the first table takes entries (p % 16) * 16 .. + 15.  A row is `irregular`
 // when the tables cannot hold it (two escaped prefixes with the same p % 16,
-// a base off its place, a code of length 0); such rows take the binary
+// a base off its place, a code of length 0 or above 12, symbol 31 with a code
+// of 4 bits, which would read as the marker); such rows take the binary
 // search.  calculate_cdf's rows have their long codes at the ends of the
 // symbol range, so that is rare, but any row is decoded either way: the
 // conditions below are checked symbol by symbol.
 //
 // Build: mark() writes both tables' entries at the symbols' bases, scan()
 // carries them forward (over the whole first table, and within each 16
-// entries of the second), and escapes() then puts kEscape at the prefixes of
+// entries of the second), and escapes() then puts kMarker at the prefixes of
 // long codes, after the scan so that it does not spread.
 struct LongTables {
   static constexpr int kBytes = 2 * ByteTables::kBytes;
   static constexpr int kMaxBins = ByteTables::kMaxBins;
+  static constexpr uint32_t kMarker = (31u << 3) | 3u;
   ByteTables one;
   bool irregular;
   uint32_t longs;  // bit s: symbol s has its entry in the second table
@@ -623,46 +632,59 @@ struct LongTables {
     for (int d = 0; d < 128; ++d) t32[d * kLanes] = 0;
   }
 
-  // Writes that do not apply go to `dummy`, so the loop has no branches.
-  __device__ __forceinline__ void mark(uint8_t *dummy) {
+  // LDS address of entry e of the first table.
+  __device__ __forceinline__ uint32_t entry_at(uint32_t e) const {
+    return one.lane_at + ((e >> 2) * (kLanes * 4) | (e & 3u));
+  }
+
+  // Writes that do not apply go to the LDS address `dummy`: the choice is
+  // between two addresses, so the loop has no branches.
+  __device__ __forceinline__ void mark(uint32_t dummy) {
     uint32_t rw[kMaxBins];
     one.unwrap(rw, eff);
-    uint32_t slots = 0, open = 0xFFFFu;
-    irregular = false;
+    uint32_t slots = 0, open = 0xFFFFu, bad = 0;
     longs = 0;
 #pragma unroll
     for (int s = 0; s < kMaxBins; ++s) {
       const uint32_t lo = s == 0 ? 0u : eff[s];  // symbol 0 also owns what lies below its base
       const uint32_t next = s + 1 < kMaxBins ? eff[s + 1 < kMaxBins ? s + 1 : 0] : 0x10000u;
-      const bool owns = next > lo && s < one.nb;
+      // Flags are 0 / 1 words.  Symbols from nb on have base 0x10000 and own
+      // nothing.
+      const uint32_t owns = next > lo ? 1u : 0u;
       const uint32_t nib = rw[s] & 0xFu;
       const uint32_t width = next - eff[s];
       const uint32_t wl = width ? static_cast<uint32_t>(__builtin_clz(width)) - 15u : 0u;
       const uint32_t len = nib != 0 ? nib : wl;
-      const bool is_short = len - 1u < 8u && !(s == 31 && len == 8u);
-      const bool is_long = owns && !is_short;
-      const bool at_prefix = (lo & 0xFFu) == 0;
+      const uint32_t is_short = len - 1u < 8u ? owns : 0u;
+      const uint32_t is_long = owns ^ is_short;
+      const uint32_t inside = lo & 0xFFu;  // not at a prefix
       const uint32_t p = lo >> 8;
-      *(owns && is_short && at_prefix ? one.entry(p) : dummy) =
-          static_cast<uint8_t>((static_cast<uint32_t>(s) << 3) | ((len - 1u) & 7u));
-      *(is_long ? one.entry((lo >> 4) & 0xFFu) + ByteTables::kBytes : dummy) =
-          static_cast<uint8_t>((static_cast<uint32_t>(s) << 3) | ((len - 8u) & 7u));
-      const bool first = p != open;
+      lds_set_byte(is_short && !inside ? entry_at(p) : dummy, (static_cast<uint32_t>(s) << 3) | ((len - 1u) & 7u));
+      lds_set_byte(is_long ? entry_at((lo >> 4) & 0xFFu) + ByteTables::kBytes : dummy,
+                   (static_cast<uint32_t>(s) << 3) | ((len - 5u) & 7u));
       const uint32_t slot = 1u << (p & 15u);
-      const bool bad_short = owns && is_short && !at_prefix;
-      const bool bad_long = is_long && (len - 8u > 7u || next > ((p + 1u) << 8) ||
-                                        (first && (!at_prefix || (slots & slot) != 0)));
-      irregular = irregular || bad_short || bad_long;
+      // A prefix's first long code starts at the prefix and takes a slot that
+      // is free; a long code is at most 12 bits and ends inside its prefix.
+      const uint32_t misplaced = p != open ? (inside | (slots & slot)) : 0u;
+      const uint32_t outside = len - 9u > 3u || next > ((p + 1u) << 8) ? 1u : 0u;
+      bad |= is_short ? inside : 0u;
+      if (s == 31) bad |= is_short && len == 4u ? 1u : 0u;
+      bad |= is_long ? (misplaced | outside) : 0u;
       slots |= is_long ? slot : 0u;
       open = is_long ? p : open;
-      longs |= is_long ? 1u << s : 0u;
+      longs |= is_long << s;
     }
+    irregular = bad != 0;
   }
 
   __device__ __forceinline__ void scan() {
     one.scan(0, 64, 0);
+    scan_second(0, 1);
+  }
+  // The second table's groups of 16 entries, from group g0 every `step`.
+  __device__ __forceinline__ void scan_second(int g0, int step) {
     uint32_t *t32 = reinterpret_cast<uint32_t *>(one.tab + ByteTables::kBytes);
-    for (int d = 0; d < 64; d += 4) {
+    for (int d = 4 * g0; d < 64; d += 4 * step) {
       uint32_t w[4], prev = 0;
 #pragma unroll
       for (int k = 0; k < 4; ++k) w[k] = t32[(d + k) * kLanes];
@@ -674,15 +696,15 @@ struct LongTables {
     }
   }
 
-  __device__ __forceinline__ void escapes(uint8_t *dummy) {
+  __device__ __forceinline__ void escapes(uint32_t dummy) {
 #pragma unroll
     for (int s = 0; s < kMaxBins; ++s) {
       const uint32_t lo = s == 0 ? 0u : eff[s];
-      *((longs >> s) & 1u ? one.entry(lo >> 8) : dummy) = static_cast<uint8_t>(ByteTables::kEscape);
+      lds_set_byte((longs >> s) & 1u ? entry_at(lo >> 8) : dummy, kMarker);
     }
   }
 
-  __device__ __forceinline__ void build(uint8_t *dummy) {
+  __device__ __forceinline__ void build(uint32_t dummy) {
     mark(dummy);
     scan();
     escapes(dummy);
@@ -705,8 +727,8 @@ struct LongTables {
 // column (the ring starts at a multiple of its size of all lanes).  a, b, c
 // and `ahead` are as in BitCursor; the dwords before q are consumed, so a
 // chunk may be written over them.
-struct RingCursor {
-  static constexpr uint32_t kBytes = 256;
+template <uint32_t BYTES> struct RingCursorT {
+  static constexpr uint32_t kBytes = BYTES;
   static constexpr uint32_t kMask = (kBytes / 4 - 1) * kLanes * 4;
   uint32_t at, a, b, c, ahead, q;
   int sh;
@@ -741,6 +763,7 @@ struct RingCursor {
     ahead = raw(q);
   }
 };
+using RingCursor = RingCursorT<256>;
 
 // Two codes per step of LongTables over a ring.  The chain from one code to
 // the next is the two tables' reads (issued together), the select of the
@@ -774,9 +797,9 @@ struct PairCursor {
   // for the next one.
   __device__ __forceinline__ uint32_t take(const LongTables &tb, uint32_t x, uint32_t &len) {
     const uint32_t x1 = (d1 >> s1) & 0xFFu, x2 = (d2 >> s2) & 0xFFu;
-    const bool esc = x1 == ByteTables::kEscape;
+    const bool esc = x1 == LongTables::kMarker;
     const uint32_t e = esc ? x2 : x1;
-    len = (e & 7u) + (esc ? 8u : 1u);
+    len = (e & 7u) + (esc ? 5u : 1u);
     read(tb, x << len);
     return e;
   }
@@ -790,6 +813,63 @@ struct PairCursor {
     h = ring.hi();
     w = ring.lo();
     place(h);
+  }
+};
+
+// One table lookup per step of LongTables over a ring, a lane at a time: a
+// code of up to 8 bits is one step, a longer one two (the marker, then its
+// entry in the second table), so the lanes of a wave are not in step with
+// each other's symbols.  The chain from one step to the next is the read, the
+// entry and its length field, the select of the next table, and the next
+// address, taken from the current window bits as in GroupCursor; two steps
+// (at most 16 bits) share one advance of the ring.  `bd` is the bit position
+// of the last symbol boundary.
+struct StepCursor {
+  using Ring = RingCursorT<128>;
+  Ring ring;
+  uint32_t h, w;   // the next 64 bits at the pair's first step
+  uint32_t d, s1;  // the current step's table dword (its read in flight), 8 x its byte
+  uint32_t pos, bd;
+
+  __device__ __forceinline__ void start(const LongTables &tb, uint32_t column, uint32_t bit, uint32_t at) {
+    ring.start(column, bit);
+    h = ring.hi();
+    w = ring.lo();
+    s1 = (h >> 21) & 0x18u;
+    d = lds_dword(((h >> 18) & 0x3F00u) | tb.one.lane_at);
+    pos = at;
+    bd = at;
+  }
+  // One step at window bits x: returns the entry and its length - 1; reads
+  // the next step's table dword.
+  __device__ __forceinline__ uint32_t take(const LongTables &tb, uint32_t x, uint32_t &lm) {
+    const uint32_t e = (d >> s1) & 0xFFu;
+    lm = (d >> s1) & 7u;
+    const uint32_t table = e == LongTables::kMarker ? tb.one.lane_at + ByteTables::kBytes : tb.one.lane_at;
+    d = lds_dword((((x >> 17) << lm) & 0x3F00u) | table);
+    return e;
+  }
+  // Two steps.  `each(entry, counts)` is called for each; counts: the entry
+  // is that of a symbol which starts below `hi`.  bd stays at the first
+  // boundary not below hi.
+  template <class F> __device__ __forceinline__ void pair(const LongTables &tb, uint32_t hi, F &&each) {
+    uint32_t l0, l1;
+    const uint32_t e0 = take(tb, h, l0);
+    const uint32_t x = align_bits(h, w, 31u - l0);
+    s1 = (x >> 21) & 0x18u;
+    pos += l0 + 1u;
+    const bool c0 = e0 != LongTables::kMarker && bd < hi;
+    each(e0, c0);
+    bd = c0 ? pos : bd;
+    const uint32_t e1 = take(tb, x, l1);
+    ring.advance(l0 + l1 + 2u);
+    h = ring.hi();
+    w = ring.lo();
+    s1 = (h >> 21) & 0x18u;
+    pos += l1 + 1u;
+    const bool c1 = e1 != LongTables::kMarker && bd < hi;
+    each(e1, c1);
+    bd = c1 ? pos : bd;
   }
 };
 

@@ -1,5 +1,5 @@
-// Host build of the decoder for long chunks (LongTables, RingCursor and
-// PairCursor of lmcache-ascend_amd/csrc/cachegen_decode.h), checked against
+// Host build of the decoder for long chunks (LongTables, RingCursor,
+// PairCursor and StepCursor of lmcache-ascend_amd/csrc/cachegen_decode.h), checked against
 // the CPU oracle's decoder (oracle/cachegen.c, oc_decode) on random CDF rows
 // and byte streams.  Built and run by
 // tests/test_decode_long_cpu.py.
@@ -105,8 +105,9 @@ int main(int argc, char **argv) {
   const int rows = argc > 1 ? atoi(argv[1]) : 2000;
   std::mt19937_64 rng(argc > 2 ? strtoull(argv[2], nullptr, 10) : 1);
   constexpr uint32_t kRingAt = LongTables::kBytes;
-  std::vector<uint8_t> lds(kRingAt + RingCursor::kBytes * kLanes);
-  uint8_t dummy = 0;
+  // The tables, the rings and a scratch byte for skipped writes.
+  std::vector<uint8_t> lds(kRingAt + RingCursor::kBytes * kLanes + 1);
+  const uint32_t dummy = static_cast<uint32_t>(lds.size()) - 1;
   long long symbols = 0, regular = 0, with_long = 0, irregular = 0;
   for (int it = 0; it < rows; ++it) {
     const int nb = it % 3 == 1 ? LongTables::kMaxBins : 1 + static_cast<int>(rng() % LongTables::kMaxBins);
@@ -122,7 +123,7 @@ int main(int argc, char **argv) {
     tb.one.row.r = buf.data();
     tb.one.nb = nb;
     tb.clear();
-    tb.build(&dummy);
+    tb.build(dummy);
     tb.one.finish();
     (tb.irregular ? irregular : tb.longs ? with_long : regular) += 1;
     uint32_t *ring = reinterpret_cast<uint32_t *>(lds.data() + kRingAt) + lane;
@@ -186,6 +187,39 @@ int main(int argc, char **argv) {
                  kind, tb.irregular ? 1 : 0, k, t, T, got[t], want[t]);
           return 1;
         }
+      // The step cursor over its own smaller ring, refilled every 16 steps.
+      if (!tb.irregular) {
+        using lmc::cgdec::StepCursor;
+        constexpr uint32_t kDw = StepCursor::Ring::kBytes / 4;
+        auto put_small = [&](uint32_t chunk) {
+          for (uint32_t d = 4 * chunk; d < 4 * chunk + 4; ++d) {
+            uint32_t v = 0;
+            for (uint32_t b = 0; b < 4; ++b)
+              if (4 * d + b < end && len) v |= static_cast<uint32_t>(bytes[4 * d + b]) << (8 * b);
+            ring[(d & (kDw - 1)) * kLanes] = v;
+          }
+        };
+        uint32_t have = 8;
+        for (uint32_t c = 0; c < have; ++c) put_small(c);
+        StepCursor sc;
+        sc.start(tb, column, 8 * off, 0);
+        int t = 0;
+        while (t < T) {
+          const uint32_t q0 = sc.ring.q;
+          for (int i = 0; i < 8; ++i)
+            sc.pair(tb, ~0u, [&](uint32_t e, bool counts) {
+              if (counts && t < T) got[t] = static_cast<uint8_t>(e >> 3);
+              t += counts ? 1 : 0;
+            });
+          if (16 * have - q0 <= StepCursor::Ring::kBytes - 16) put_small(have++);
+        }
+        for (int u = 0; u < T; ++u)
+          if (got[u] != want[u]) {
+            printf("STEP MISMATCH row %d (nb %d, kind %d) stream %d token %d of %d: got %d want %d\n", it, nb, kind, k,
+                   u, T, got[u], want[u]);
+            return 1;
+          }
+      }
       symbols += T;
     }
   }

@@ -128,3 +128,23 @@ def test_decode_chunk_by_lengths(F, L, T, C):
     other = F.CacheGenChunk(chunk.cdf, chunk.lengths.to(torch.int64), chunk.streams, T)
     assert np.array_equal(F.decode_chunk(chunk).cpu().numpy(), sym)
     assert np.array_equal(F.decode_chunk(other).cpu().numpy(), sym)
+
+
+# Chunks whose quarters do not follow from where they should lie: streams of
+# one-bit and of long codes at either end (a quarter outgrows its buffer, or
+# starts well off its place), codes of one length (a decoder started between
+# boundaries stays between them), and the kernel's largest chunk and one past.
+@pytest.mark.parametrize("T", [257, 401, 1000, 1024, 1025])
+def test_long_chunk_uneven_streams(F, T):
+    L, C, nb = 3, 96, 32
+    rng = np.random.default_rng(T)
+    sym = np.empty((L, T, C), np.uint8)
+    sym[0] = 3
+    sym[0, -T // 6:] = rng.integers(0, nb - 1, size=(T // 6 + (T % 6 > 0), C))  # one-bit codes, then five-bit ones
+    sym[0, :, 1::2] = sym[0, ::-1, 1::2]
+    sym[1] = rng.integers(0, 16, size=(T, C))  # codes of (about) one length
+    sym[1, :, :48] = (np.arange(T) % 16)[:, None]  # of exactly one
+    sym[2] = _symbols(1, T, C, nb, T)[0]
+    sym[2, :, 5] = 7
+    chunk = F.encode_chunk(torch.from_numpy(sym).to(DEV), nb)
+    assert np.array_equal(F.decode_chunk(chunk).cpu().numpy(), sym)
