@@ -618,11 +618,55 @@ inline EncLds enc_lds(int64_t T, int nb) {
   return e;
 }
 
+// Exclusive prefix sums of n block byte counts by one workgroup of NT
+// threads: off[b] for block b, off[n] and *total the sum.  `total` is host
+// memory a thread may be watching: it is written last, at system scope.
+// `wave_sum` is scratch in LDS.
+struct BlockOffsets {
+  const int64_t *sums;  // null: no offsets to make
+  int64_t n;
+  int64_t *off;
+  int64_t *total;
+};
+template <int NT> __device__ __forceinline__ void block_offsets(const BlockOffsets &b, int64_t *wave_sum) {
+  const int lane = static_cast<int>(threadIdx.x) & 63;
+  const int wave = static_cast<int>(threadIdx.x) >> 6;
+  int64_t carry = 0;
+  for (int64_t i0 = 0; i0 < b.n; i0 += NT) {
+    const int64_t i = i0 + threadIdx.x;
+    const int64_t own = i < b.n ? b.sums[i] : 0;
+    int64_t incl = own;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int64_t v = __shfl_up(incl, d, 64);
+      incl += lane >= d ? v : 0;
+    }
+    if (lane == 63) wave_sum[wave] = incl;
+    __syncthreads();
+    int64_t before = 0, all = 0;
+#pragma unroll
+    for (int w = 0; w < NT / 64; ++w) {
+      before += w < wave ? wave_sum[w] : 0;
+      all += wave_sum[w];
+    }
+    if (i < b.n) b.off[i] = carry + before + incl - own;
+    carry += all;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    b.off[b.n] = carry;
+    __hip_atomic_store(b.total, carry, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
+// With `offsets` the launch has one block more, the first: it makes the
+// blocks' offsets while the others encode (as a kernel of its own before them
+// it took 4.1 us of the chunk's time).
 template <int PIECES, EncMode MODE>
 __global__ void __launch_bounds__(64 * PIECES)
     encode_split_kernel(const int16_t *__restrict__ cdf, const uint8_t *__restrict__ in, int T, int C, int nb,
                         int64_t n_streams, uint8_t *__restrict__ out, int64_t chunk, int32_t *__restrict__ lens,
-                        int place, int vec_tile, int rows_dw, const EncLds at) {
+                        int place, int vec_tile, int rows_dw, const EncLds at, const BlockOffsets offsets) {
   constexpr int NT = 64 * PIECES;
   constexpr int Q = kEncTokens / PIECES;  // tokens per piece
   constexpr bool IMAGE = MODE == EncMode::kImage, LONG = MODE == EncMode::kLong;
@@ -631,7 +675,15 @@ __global__ void __launch_bounds__(64 * PIECES)
   const int tid = static_cast<int>(threadIdx.x);
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
-  const int64_t s0 = static_cast<int64_t>(blockIdx.x) * kEncLanes;
+  int64_t block = blockIdx.x;
+  if (offsets.sums != nullptr) {
+    if (block == 0) {
+      block_offsets<NT>(offsets, reinterpret_cast<int64_t *>(lds));
+      return;
+    }
+    --block;
+  }
+  const int64_t s0 = block * kEncLanes;
   const int cnt = n_streams - s0 < kEncLanes ? static_cast<int>(n_streams - s0) : kEncLanes;
   int16_t *stage = reinterpret_cast<int16_t *>(lds);
   uint8_t *tile = reinterpret_cast<uint8_t *>(lds + at.rows_words);
@@ -2092,45 +2144,6 @@ __global__ void __launch_bounds__(kSplitThreads)
   if (stored < g1 && 4 * stored + (quad.at >> 4) < T) cg_st(quad.dst + static_cast<int64_t>(stored) * C, word);
 }
 
-// Exclusive prefix sums of the blocks' byte counts, in one workgroup: off[b]
-// for block b, off[n] and *total the sum.  `sums` and `off` may not overlap.
-// One workgroup: 1024 blocks (65536 streams) take 4.1 us, of which most is
-// the launch, under which nothing else has to wait but the encoder.
-constexpr int kOffThreads = 1024;
-__global__ void __launch_bounds__(kOffThreads)
-    stream_offsets_kernel(const int64_t *__restrict__ sums, int64_t n, int64_t *__restrict__ off,
-                          int64_t *total) {
-  __shared__ int64_t wave_sum[kOffThreads / 64];
-  const int lane = static_cast<int>(threadIdx.x) & 63;
-  const int wave = static_cast<int>(threadIdx.x) >> 6;
-  int64_t carry = 0;
-  for (int64_t i0 = 0; i0 < n; i0 += kOffThreads) {
-    const int64_t i = i0 + threadIdx.x;
-    const int64_t own = i < n ? sums[i] : 0;
-    int64_t incl = own;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int64_t v = __shfl_up(incl, d, 64);
-      incl += lane >= d ? v : 0;
-    }
-    if (lane == 63) wave_sum[wave] = incl;
-    __syncthreads();
-    int64_t before = 0, all = 0;
-#pragma unroll
-    for (int w = 0; w < kOffThreads / 64; ++w) {
-      before += w < wave ? wave_sum[w] : 0;
-      all += wave_sum[w];
-    }
-    if (i < n) off[i] = carry + before + incl - own;
-    carry += all;
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    off[n] = carry;
-    *total = carry;
-  }
-}
-
 // Moves the blocks' bytes together: block b's off[b + 1] - off[b] bytes, from
 // b * stride of `blocks`, to off[b] of `out`.  A thread takes 16-byte aligned
 // pieces of the destination, each from five source dwords shifted together;
@@ -2170,9 +2183,10 @@ __global__ void __launch_bounds__(kPackThreads)
   }
 }
 
-// What a call that waits for a device value needs: an event and a word of
-// pinned host memory.  Taken from a pool per call and given back once the
-// event has completed; the pool keeps at most kKept of them.
+// What a call that waits for a device value needs: a word of pinned host
+// memory, which the kernel writes and the host watches, and an event behind
+// the kernel, which bounds the watch.  Taken from a pool per call and given
+// back once the word has been written; the pool keeps at most kKept of them.
 class HostWord {
 public:
   explicit HostWord(int device) {
@@ -2189,7 +2203,7 @@ public:
     s_.device = device;
     hip_check(hipEventCreateWithFlags(&s_.event, hipEventDisableTiming), "hipEventCreate");
     const hipError_t e = hipHostMalloc(reinterpret_cast<void **>(&s_.word), sizeof(int64_t),
-                                       hipHostMallocMapped | hipHostMallocPortable);
+                                       hipHostMallocMapped | hipHostMallocPortable | hipHostMallocCoherent);
     if (e != hipSuccess) {
       (void)hipEventDestroy(s_.event);
       hip_check(e, "hipHostMalloc");
@@ -2197,9 +2211,9 @@ public:
   }
   HostWord(const HostWord &) = delete;
   HostWord &operator=(const HostWord &) = delete;
-  // The kernel that writes the word has to be over before it is given back:
-  // wait() sees to that, and a call that fails after its launch waits for
-  // the stream here.
+  // A word is given back only when no kernel may still write it: wait() has
+  // seen it written, and a call that fails after its launch waits for the
+  // stream here.
   ~HostWord() {
     if (pending_) (void)hipStreamSynchronize(stream_);
     {
@@ -2212,18 +2226,34 @@ public:
     (void)hipEventDestroy(s_.event);
     (void)hipHostFree(s_.word);
   }
-  int64_t *word() const { return s_.word; }
-  // Call before the launch of the kernel that writes the word, then record()
-  // after it.
-  void launching(hipStream_t stream) {
+  // Call before the launch of the kernel that writes the word (a value of 0
+  // or more), then record() after it.
+  int64_t *launching(hipStream_t stream) {
     stream_ = stream;
     pending_ = true;
+    __atomic_store_n(s_.word, int64_t(-1), __ATOMIC_RELEASE);
+    return s_.word;
   }
   void record() { hip_check(hipEventRecord(s_.event, stream_), "hipEventRecord"); }
   int64_t wait() {
-    hip_check(hipEventSynchronize(s_.event), "hipEventSynchronize");
-    pending_ = false;
-    return *static_cast<volatile int64_t *>(s_.word);
+    for (;;) {
+      for (int i = 0; i < 256; ++i) {
+        const int64_t v = __atomic_load_n(s_.word, __ATOMIC_ACQUIRE);
+        if (v >= 0) {
+          pending_ = false;
+          return v;
+        }
+        __builtin_ia32_pause();
+      }
+      const hipError_t e = hipEventQuery(s_.event);
+      if (e == hipErrorNotReady) continue;
+      hip_check(e, "hipEventQuery");
+      // The kernel is over: its word is there.
+      const int64_t v = __atomic_load_n(s_.word, __ATOMIC_ACQUIRE);
+      pending_ = false;
+      check(v >= 0, "the kernel left no value");
+      return v;
+    }
   }
 
 private:
@@ -2331,7 +2361,7 @@ void make_cdf(const lmc_tensor &in, int32_t n_bins, const lmc_tensor &o, int32_t
 // 1 the streams of each block of 64 one after the other (encode_split_kernel;
 // `ol` then holds their lengths already, and cdf is calculate_cdf's).
 void encode_rows(const lmc_tensor &cdf, const lmc_tensor &in, const lmc_tensor &ob, const lmc_tensor &ol, int place,
-                 hipStream_t stream) {
+                 const BlockOffsets &offsets, hipStream_t stream) {
   need_device(cdf, "cdf");
   need_device(in, "input_sym");
   need_device(ob, "output_buffer");
@@ -2367,10 +2397,11 @@ void encode_rows(const lmc_tensor &cdf, const lmc_tensor &in, const lmc_tensor &
                     : place == 0 && T <= kEncTokens ? encode_split_kernel<kEncPieces, EncMode::kRows>
                                                          : encode_split_kernel<kEncPieces, EncMode::kLong>;
   check(at.bytes <= 65536, "encode: LDS budget exceeded");
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks)), dim3(64 * kEncPieces), at.bytes, stream,
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks + (offsets.sums != nullptr ? 1 : 0))),
+                     dim3(64 * kEncPieces), at.bytes, stream,
                      static_cast<const int16_t *>(cdf.data), static_cast<const uint8_t *>(in.data), (int)T, (int)C,
                      (int)nb, n_streams, static_cast<uint8_t *>(ob.data), chunk, static_cast<int32_t *>(ol.data),
-                     place, vec_in, rows_dw, at);
+                     place, vec_in, rows_dw, at, offsets);
   hip_check(hipGetLastError(), "encode_split_kernel launch");
 }
 
@@ -2467,7 +2498,8 @@ int lmc_encode_fast_new(const lmc_tensor *cdf_t, const lmc_tensor *input_sym,
                         const lmc_tensor *output_lengths, void *stream) {
   return guarded([&] {
     encode_rows(deref(cdf_t, "cdf"), deref(input_sym, "input_sym"), deref(output_buffer, "output_buffer"),
-                deref(output_lengths, "output_lengths"), 0, static_cast<hipStream_t>(stream));
+                deref(output_lengths, "output_lengths"), 0, BlockOffsets{nullptr, 0, nullptr, nullptr},
+                static_cast<hipStream_t>(stream));
   });
 }
 
@@ -2506,14 +2538,10 @@ int lmc_cachegen_encode_rows(const lmc_tensor *input, int32_t n_bins, const lmc_
     int64_t *sums = offsets + blocks + 1;
     make_cdf(in, n_bins, cdf, static_cast<int32_t *>(lens.data), sums, rows.sizes[2], stream);
     // The sizes follow from the histograms, so the host learns the total
-    // while the rows are still being encoded.
+    // while the streams are still being encoded.
     HostWord word(in.device);
-    word.launching(stream);
-    hipLaunchKernelGGL(stream_offsets_kernel, dim3(1), dim3(kOffThreads), 0, stream, sums, blocks, offsets,
-                       word.word());
-    hip_check(hipGetLastError(), "stream_offsets_kernel launch");
+    encode_rows(cdf, in, rows, lens, 1, BlockOffsets{sums, blocks, offsets, word.launching(stream)}, stream);
     word.record();
-    encode_rows(cdf, in, rows, lens, 1, stream);
     *total = word.wait();
   });
 }
