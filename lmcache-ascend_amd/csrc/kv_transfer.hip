@@ -715,9 +715,9 @@ constexpr int64_t kGroupLinear = 2048;
 // (32 x 8192 x 128 stored, 45.7 against 41.1).
 constexpr int64_t kGroupOneRow = 1024;
 // Long stores of rows of nine vector groups (576-column MLA rows in bf16)
-// stay with the tile kernel: 2.3 GB 395 against 420 us; 0.58 GB is faster here
-// (110 against 115 us).
-constexpr int64_t kGroupNineStore = int64_t(1) << 30;
+// stay with the tile kernel: 2.3 GB 395 against 420 us, 1.0 GB 180 against
+// 185; 0.58 GB is faster here (112 against 117 us).
+constexpr int64_t kGroupNineStore = int64_t(768) << 20;
 
 template <int U, int R>
 void launch_group_u(const CopyJob &job, const ChunkList &chunks, int n_chunks, int64_t max_tokens, int g_shift,
@@ -799,7 +799,11 @@ void launch_vec(const CopyJob &job_in, const ChunkList &chunks, int n_chunks,
   lean = lean && ((n_chunks == 1 && max_rows <= LMC_KV_LEAN_MAX_ROWS) || LMC_KV_LEAN_BATCH);
   // Rows that are not whole slices: the group kernel where every plane's row
   // has its form.
-  bool group = VEC == 16 && !whole_slices && (job.block_size == 0 || pow2(job.block_size)) && max_rows < (1 << 30);
+  // Memory objects in host memory stay with the tile kernel, whose larger
+  // runs per wave suit PCIe better (64 layers x 22 tokens x 128 columns
+  // retrieved from pinned memory: 16.5 us against 19.2).
+  bool group = VEC == 16 && !whole_slices && !host_lmc && (job.block_size == 0 || pow2(job.block_size)) &&
+               max_rows < (1 << 30);
   for (int p = 0; p < job.n_planes; ++p)
     group = group && job.plane[p].row_bytes == widest && job.table_idx[p] == p * job.idx_step;
   if (group) {
