@@ -1837,7 +1837,9 @@ __device__ __forceinline__ void decode_serial(cgdec::LongTables &tb, bool irregu
 
 constexpr int kLongObuf = kLongRing + static_cast<int>(cgdec::RingCursor::kBytes) * kDecLanes;
 constexpr int kLongRows = kLongObuf + kObufBytes;
-constexpr int rows_lds_bytes(int nb) { return ((nb + 1) * kDecLanes * 2 + 32 + 15) & ~15; }
+// The staged rows, at up to 15 bytes past a 16-byte boundary; a table build
+// reads kMaxBins entries of a row whatever nb is.
+constexpr int rows_lds_bytes(int nb) { return ((nb + 1) * kDecLanes * 2 + 32 + 2 * cgdec::ByteTables::kMaxBins + 15) & ~15; }
 
 // Any length, one wave per block (56 planes x 1000 tokens x 256 channels: 100
 // us, where the shared-window kernel took 1307 us: the streams of a block

@@ -148,3 +148,77 @@ def test_long_chunk_uneven_streams(F, T):
     sym[2, :, 5] = 7
     chunk = F.encode_chunk(torch.from_numpy(sym).to(DEV), nb)
     assert np.array_equal(F.decode_chunk(chunk).cpu().numpy(), sym)
+
+
+# decode_chunk enqueues kernels only, also for the long chunk whose kernel
+# takes more than 64 KiB of LDS: captured once, it decodes whatever the chunk's
+# buffers hold at each replay.
+@pytest.mark.parametrize("T", [200, 300, 1000])
+def test_decode_chunk_captured(F, T):
+    L, C, nb = 2, 96, 32
+    syms = [_symbols(L, T, C, nb, T)]
+    rng = np.random.default_rng(T)
+    for _ in range(3):  # the same counts per stream: chunks of the same size
+        syms.append(np.ascontiguousarray(syms[0][:, rng.permutation(T)]))
+    chunks = [F.encode_chunk(torch.from_numpy(s).to(DEV), nb) for s in syms]
+    assert len({c.streams.numel() for c in chunks}) == 1
+    held = F.CacheGenChunk(chunks[0].cdf.clone(), chunks[0].lengths.clone(), chunks[0].streams.clone(), T)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        F.decode_chunk(held)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = F.decode_chunk(held)
+    for s, c in zip(syms[1:], chunks[1:]):
+        held.cdf.copy_(c.cdf)
+        held.lengths.copy_(c.lengths)
+        held.streams.copy_(c.streams)
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(out.cpu().numpy(), s)
+
+
+def test_encode_chunk_refuses_capture_and_goes_on(F):
+    sym = torch.from_numpy(_symbols(2, 40, 64, 16, 5)).to(DEV)
+    want = F.encode_chunk(sym, 16)
+    side = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(side):
+        graph.capture_begin()
+        try:
+            with pytest.raises(RuntimeError, match="cannot be captured"):
+                F.encode_chunk(sym, 16)
+        finally:
+            graph.capture_end()
+    torch.cuda.synchronize()
+    again = F.encode_chunk(sym, 16)
+    assert torch.equal(again.streams, want.streams) and torch.equal(again.cdf, want.cdf)
+
+
+def test_encode_chunk_from_threads(F):
+    """Each thread on its own stream: the words the sizes arrive in are taken
+    from one pool."""
+    import threading
+
+    syms = [torch.from_numpy(_symbols(2, 100 + 37 * i, 96, 32, i)).to(DEV) for i in range(6)]
+    want = [F.encode_chunk(s, 32) for s in syms]
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(20):
+                c = F.encode_chunk(syms[i], 32)
+                if not torch.equal(c.streams, want[i].streams):
+                    bad.append(i)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(syms))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
