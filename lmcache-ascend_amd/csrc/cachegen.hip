@@ -27,11 +27,11 @@
 //   L6  decode takes the largest symbol whose base is <= the next 16 bits.
 //
 // Work mapping: nothing here is a dense contraction, so there is no MFMA
-// work.  One lane owns one (layer, channel) stream; a 256-lane block covers
-// 256 consecutive channels of one layer, so symbol loads/stores of a token
-// are one coalesced 256-byte row.  Per-stream tables (histogram, code table,
-// decode table) live in LDS as [symbol][lane] so every lane works in its own
-// column without bank conflicts or barriers.
+// work.  A block takes 64 consecutive (layer, channel) streams, channels
+// fastest, and may span layers; lane i of each of its waves works on stream
+// i, so a token's symbols are a coalesced 64-byte row.  Per-stream tables
+// (histogram, code table, decode tables) live in LDS as [symbol][lane], so
+// every lane works in its own column without bank conflicts.
 #include <algorithm>
 #include <mutex>
 #include <type_traits>
@@ -55,7 +55,6 @@ namespace lmc {
 
 namespace {
 
-constexpr int kLanes = 256;
 constexpr int kMaxBins = 64;
 constexpr int kPrec = 16;
 constexpr int kMaxLen = 12;

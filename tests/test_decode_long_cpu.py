@@ -16,7 +16,7 @@ REPO = os.path.dirname(HERE)
 
 
 @pytest.fixture(scope="module")
-def checker(tmp_path_factory):
+def program(tmp_path_factory):
     if not shutil.which("g++") or not shutil.which("gcc"):
         pytest.skip("needs gcc and g++")
     d = tmp_path_factory.mktemp("declong")
@@ -29,7 +29,7 @@ def checker(tmp_path_factory):
 
 
 @pytest.mark.parametrize("seed", [1, 2, 3])
-def test_long_chunk_decoder_matches_oracle(checker, seed):
-    res = subprocess.run([checker, "3000", str(seed)], capture_output=True, text=True, timeout=300)
+def test_long_chunk_decoder_matches_oracle(program, seed):
+    res = subprocess.run([program, "3000", str(seed)], capture_output=True, text=True, timeout=300)
     assert res.returncode == 0, res.stdout + res.stderr
     assert res.stdout.startswith("ok"), res.stdout
