@@ -2169,11 +2169,12 @@ constexpr int64_t kPackWhole = 1024;
 constexpr unsigned kPackParts = 4;
 __global__ void __launch_bounds__(kPackThreads)
     pack_blocks_kernel(const uint8_t *__restrict__ blocks, int64_t stride, const int64_t *__restrict__ off,
-                       uint8_t *__restrict__ out) {
+                       uint8_t *__restrict__ out, int64_t size) {
   typedef unsigned int w4 __attribute__((ext_vector_type(4)));
   typedef unsigned int w4u __attribute__((ext_vector_type(4), aligned(4)));
   const int64_t begin = off[blockIdx.x];
-  const int64_t n = off[blockIdx.x + 1] - begin;
+  const int64_t end = off[blockIdx.x + 1];
+  const int64_t n = (end < size ? end : size) - begin;  // `out` holds `size` bytes
   const uint8_t *src = blocks + static_cast<int64_t>(blockIdx.x) * stride;
   uint8_t *dst = out + begin;
   const int64_t lead = static_cast<int64_t>(reinterpret_cast<uintptr_t>(dst) & 15);
@@ -2583,7 +2584,7 @@ int lmc_cachegen_pack_rows(const lmc_tensor *rows_t, const lmc_tensor *offsets_t
     hipLaunchKernelGGL(pack_blocks_kernel, dim3(static_cast<unsigned>(blocks), parts), dim3(kPackThreads), 0,
                        static_cast<hipStream_t>(stream), static_cast<const uint8_t *>(rows.data),
                        kEncLanes * rows.sizes[2], static_cast<const int64_t *>(off.data),
-                       static_cast<uint8_t *>(o.data));
+                       static_cast<uint8_t *>(o.data), numel(o));
     hip_check(hipGetLastError(), "pack_blocks_kernel launch");
   });
 }
