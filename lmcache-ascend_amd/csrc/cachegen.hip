@@ -897,9 +897,13 @@ __global__ void __launch_bounds__(64 * PIECES)
     if (IMAGE) {
       if (wv == 0 && lane < cnt) lens[s0 + lane] = static_cast<int32_t>((total + 7) >> 3);
       __syncthreads();
-      // 5. The block's bytes (its place holds 64 * chunk bytes, a multiple
-      //    of 16).
-      for (uint32_t i = tid; i < words / 4; i += NT) {
+      // 5. The block's bytes: whole 16-byte vectors as far as they lie in the
+      //    block's place, cnt * chunk bytes.  A last block of few streams and
+      //    tokens may end inside a vector of its place; those bytes leave one
+      //    by one.
+      const int64_t room = cnt * chunk / 16;
+      const uint32_t vecs = room < words / 4 ? static_cast<uint32_t>(room) : words / 4;
+      for (uint32_t i = tid; i < vecs; i += NT) {
         w4 x = reinterpret_cast<const w4 *>(bits)[i];
         x.x = __builtin_bswap32(x.x);
         x.y = __builtin_bswap32(x.y);
@@ -907,6 +911,8 @@ __global__ void __launch_bounds__(64 * PIECES)
         x.w = __builtin_bswap32(x.w);
         cg_st(reinterpret_cast<w4 *>(block_out) + i, x);
       }
+      for (uint32_t b = 16 * vecs + tid; b < image_bytes; b += NT)
+        block_out[b] = static_cast<uint8_t>(bits[b >> 2] >> (24 - 8 * (b & 3u)));
       return;
     }
     if (!LONG) {

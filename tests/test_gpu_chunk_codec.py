@@ -222,3 +222,53 @@ def test_encode_chunk_from_threads(F):
     for t in threads:
         t.join()
     assert not bad
+
+
+# The C entries write nothing outside their buffers: each output lies between
+# guard bytes, `rows` on a 16-byte boundary and off it, with last blocks of
+# one to 33 streams whose bytes end inside a 16-byte vector of their rows.
+@pytest.mark.parametrize("shift", [0, 3])
+@pytest.mark.parametrize("L,T,C,cap", [
+    (1, 1, 1, 2), (1, 3, 5, 6), (3, 7, 33, 14), (1, 2, 3, 4), (1, 3, 2, 6), (1, 7, 1, 14), (2, 1, 33, 2), (5, 3, 13, 6),
+    (1, 1, 7, 2), (1, 256, 65, 512), (1, 9, 66, 19), (1, 300, 1, 600), (1, 2, 71, 3),
+])
+def test_encode_rows_keep_to_their_buffers(L, T, C, cap, shift):
+    import ctypes
+
+    from lmcache_amd import _lib, c_ops
+
+    lib, nb, pad = _lib.load(), 16, 256
+    sym = _symbols(L, T, C, nb, T + C, "skewed")
+    blocks = (L * C + 63) // 64
+
+    def guarded(n, at=pad):
+        return torch.full((at + n + pad,), 0xA5, dtype=torch.uint8, device=DEV), at, n
+
+    def part(buf, dtype, shape):
+        return buf[0][buf[1]:buf[1] + buf[2]].view(dtype).view(shape)
+
+    cdf = guarded(L * C * (nb + 1) * 2)
+    rows = guarded(L * C * cap, pad + shift)
+    lens = guarded(L * C * 4)
+    off = guarded((2 * blocks + 1) * 8)
+    dsym = torch.from_numpy(sym).to(DEV)
+    views = [dsym, part(cdf, torch.int16, (L, C, nb + 1)), part(rows, torch.uint8, (L, C, cap)),
+             part(lens, torch.int32, (L, C)), part(off, torch.int64, (2 * blocks + 1,))]
+    d = [c_ops._desc(v) for v in views]
+    total = ctypes.c_int64(-1)
+    stream = c_ops._stream(0)
+    _lib.raise_for(lib.lmc_cachegen_encode_rows(c_ops._ref(d[0]), nb, *map(c_ops._ref, d[1:]), ctypes.byref(total), stream))
+    want_cdf = oc.calculate_cdf(sym, nb)
+    want, want_len = oc.encode(want_cdf, sym, cap)
+    kept = np.minimum(want_len, cap)
+    assert total.value == int(kept.sum())
+    streams = guarded(total.value)
+    s = c_ops._desc(part(streams, torch.uint8, (total.value,)))
+    _lib.raise_for(lib.lmc_cachegen_pack_rows(c_ops._ref(d[2]), c_ops._ref(d[4]), c_ops._ref(s), stream))
+    torch.cuda.synchronize()
+    for name, (buf, at, n) in dict(cdf=cdf, rows=rows, lens=lens, off=off, streams=streams).items():
+        assert bool((buf[:at] == 0xA5).all()) and bool((buf[at + n:] == 0xA5).all()), name
+    assert np.array_equal(views[1].cpu().numpy(), want_cdf)
+    assert np.array_equal(views[3].cpu().numpy(), want_len)
+    got = streams[0][pad:pad + total.value].cpu().numpy()
+    assert np.array_equal(got, np.concatenate([want[l, c, :kept[l, c]] for l in range(L) for c in range(C)]))
