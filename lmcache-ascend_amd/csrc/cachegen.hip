@@ -1708,14 +1708,17 @@ constexpr int kLongRing = cgdec::LongTables::kBytes;
 
 // A lane's stream in 16-byte aligned chunks from a0; `end` is the stream's
 // end from a0 in bytes.  Chunks 0 .. n_ch - 1 each hold a byte of the stream,
-// so no load leaves the buffer's pages.
+// so no load leaves the buffer's pages.  Of a longer stream kMost bytes count,
+// so that positions fit an int; a chunk's codes (calculate_cdf takes fewer
+// than 2^26 tokens) end below 2^27 bytes.
 struct LaneChunks {
+  static constexpr uint32_t kMost = 0x7FFFFFE0u;
   uintptr_t a0;
   uint32_t off, end, n_ch;
 
   __device__ __forceinline__ LaneChunks(const uint8_t *bytes, const DecBlock &bk) {
     const uintptr_t s_lo = reinterpret_cast<uintptr_t>(bytes) + static_cast<uintptr_t>(bk.start);
-    const uint32_t len = static_cast<uint32_t>(bk.end - bk.start);
+    const uint32_t len = min(static_cast<uint32_t>(bk.end - bk.start), kMost);
     a0 = s_lo & ~uintptr_t(15);
     off = static_cast<uint32_t>(s_lo - a0);
     end = off + len;

@@ -130,6 +130,29 @@ def test_decode_chunk_by_lengths(F, L, T, C):
     assert np.array_equal(F.decode_chunk(other).cpu().numpy(), sym)
 
 
+# A stream that reaches almost to 2 GiB.
+@pytest.mark.parametrize("T", [16, 300, 400, 1025])
+def test_decode_stream_of_almost_2gib(F, T):
+    C = 32
+    sym = _symbols(1, T, C, 16, T, "constant")
+    sym[0, :, 0] = np.arange(T) % 16
+    chunk = F.encode_chunk(torch.from_numpy(sym).to(DEV), 16)
+    n0, rest = int(chunk.lengths[0, 0]), int(chunk.lengths[0, 1:].sum())
+    big = torch.zeros(2**31 - 1, dtype=torch.uint8, device=DEV)
+    lens = chunk.lengths.clone()
+    for end in (2**31 - 1 - rest, 2**31 - 1):  # with the other streams behind it, or without
+        if end == 2**31 - 1:
+            lens[0, 1:] = 0
+        else:
+            big[end:] = chunk.streams[n0:]
+        lens[0, 0] = end
+        big[:n0] = chunk.streams[:n0]
+        got = F.decode_chunk(F.CacheGenChunk(chunk.cdf, lens, big, T)).cpu().numpy()
+        assert np.array_equal(got[0, :, 0], sym[0, :, 0])
+        if end < 2**31 - 1:
+            assert np.array_equal(got, sym)
+
+
 # Chunks whose quarters do not follow from where they should lie: streams of
 # one-bit and of long codes at either end (a quarter outgrows its buffer, or
 # starts well off its place), codes of one length (a decoder started between
