@@ -374,8 +374,8 @@ int lmc_decode_fast_prefsum(const lmc_tensor *cdf,
 
 /* No counterpart in the reference: decode_fast_prefsum with the streams'
  * lengths (int32 [L, C], bytes) in place of their inclusive prefix sums.
- * sums: device scratch, int32, one entry per 64 streams and one per 4096
- * (both rounded up). */
+ * sums: device scratch with one entry per 64 streams and one per 4096 (both
+ * rounded up): int64, or int32, which places streams below 2 GiB only. */
 int lmc_cachegen_decode(const lmc_tensor *cdf, const lmc_tensor *bytestreams,
                         const lmc_tensor *lengths, const lmc_tensor *sums,
                         const lmc_tensor *output, void *stream);

@@ -1356,15 +1356,23 @@ __device__ __forceinline__ StreamAt stream_at(int64_t l, int c, uint32_t k, int 
   return {l + up, static_cast<int>(x - up * static_cast<uint32_t>(C))};
 }
 
+// Inclusive prefix sum of 32-bit values over the 64 lanes of a wave, in 64
+// bits (the sums of their halves fit 32).
+__device__ __forceinline__ int64_t wave_incl_scan_wide(uint32_t v) {
+  return (static_cast<int64_t>(wave_incl_scan(v >> 16)) << 16) + wave_incl_scan(v & 0xFFFFu);
+}
+
 // Where the streams lie in the byte buffer: inclusive prefix sums of their
 // lengths, or (prefix null) the lengths with the sums length_sums_kernel
-// makes of them.  Both give a stream's end as the same int32, the sum of the
-// lengths up to it modulo 2^32.
+// makes of them.  Prefix sums and 32-bit sums give a stream's end as the same
+// int32, the sum of the lengths up to it modulo 2^32; buffers of 2 GiB and
+// more take 64-bit sums.
 struct StreamEnds {
   const int32_t *prefix;
   const int32_t *lens;
   const uint32_t *sums;    // [64-stream blocks]: lengths before the block in its group of 64 blocks
   const uint32_t *groups;  // [groups]: lengths of a group
+  const int64_t *wide_sums, *wide_groups;  // the same in 64 bits, in place of the 32-bit ones
 };
 constexpr int kSumThreads = 1024;
 constexpr int kGroupBlocks = 64;  // 64-stream blocks per group
@@ -1391,6 +1399,19 @@ struct DecBlock {
       end = clampb(ends.prefix[stream]);
       B0 = clampb(s0 == 0 ? 0 : ends.prefix[s0 - 1]);
       B1 = clampb(ends.prefix[s0 + cnt - 1]);
+    } else if (ends.wide_sums != nullptr) {
+      const int32_t len = lane < cnt ? max(ends.lens[stream], 0) : 0;
+      int64_t part = 0;
+      for (int64_t g = lane; g < static_cast<int64_t>(blockIdx.x) / kGroupBlocks; g += kDecLanes)
+        part += ends.wide_groups[g];
+#pragma unroll
+      for (int d = 1; d < kDecLanes; d <<= 1) part += __shfl_xor(part, d, kDecLanes);
+      const int64_t base = ends.wide_sums[blockIdx.x] + part;
+      const int64_t incl = wave_incl_scan_wide(static_cast<uint32_t>(len));
+      start = clampb(base + incl - len);
+      end = clampb(base + incl);
+      B0 = clampb(base);
+      B1 = clampb(base + __shfl(incl, kDecLanes - 1, kDecLanes));
     } else {
       const uint32_t len = lane < cnt ? static_cast<uint32_t>(ends.lens[stream]) : 0u;
       uint32_t base = ends.sums[blockIdx.x];
@@ -1554,7 +1575,9 @@ __device__ __forceinline__ bool decode_one_wave_lanes(uint8_t *lds, const int16_
   // Chunks [a0, a0 + 16 n_ch) each hold a byte of the stream, so no load
   // leaves the buffer's pages.
   const uint32_t n_ch = len ? static_cast<uint32_t>(((s_hi - 1) >> 4) - (s_lo >> 4) + 1) : 0u;
-  const uint32_t rbytes = 16u * n_ch + cgdec::LaneRegion::kRoom;  // chunks plus the sealed room
+  // Chunks plus the sealed room; at most one byte more than there is, so that
+  // the sum of the lanes' cannot wrap.
+  const uint32_t rbytes = min(16u * n_ch + cgdec::LaneRegion::kRoom, reg_cap + 1u);
   uint32_t incl = rbytes, n_max = n_ch;
 #pragma unroll
   for (int d = 1; d < kDecLanes; d <<= 1) {
@@ -2309,23 +2332,39 @@ private:
 // 20.7 us, against four launches of about 17 us for prefix sums in 64 bits
 // (widening, scan, narrowing) and 24.4 us for the decode kernel reading them;
 // decode_chunk 35.9 -> 22.4 us.
+// S: uint32_t, or int64_t for buffers of 2 GiB and more (negative lengths
+// count as 0 there).
+template <typename S>
 __global__ void __launch_bounds__(kSumThreads)
     length_sums_kernel(const int32_t *__restrict__ lens, int64_t n_streams, int64_t n_blocks,
-                       uint32_t *__restrict__ sums, uint32_t *__restrict__ groups) {
-  __shared__ uint32_t block_sum[kGroupBlocks];
+                       S *__restrict__ sums, S *__restrict__ groups) {
+  constexpr bool WIDE = sizeof(S) == 8;
+  __shared__ S block_sum[kGroupBlocks];
   const int tid = static_cast<int>(threadIdx.x);
   const int64_t s = (static_cast<int64_t>(blockIdx.x) * kSumThreads + tid) * 4;
-  uint32_t own = 0;
+  S own = 0;
 #pragma unroll
-  for (int k = 0; k < 4; ++k) own += s + k < n_streams ? static_cast<uint32_t>(lens[s + k]) : 0u;
+  for (int k = 0; k < 4; ++k) {
+    const int32_t n = s + k < n_streams ? lens[s + k] : 0;
+    own += static_cast<S>(WIDE ? max(n, 0) : n);
+  }
   // 16 threads hold a block's lengths.
 #pragma unroll
   for (int d = 1; d < 16; d <<= 1) own += __shfl_xor(own, d, 64);
   if ((tid & 15) == 0) block_sum[tid >> 4] = own;
   __syncthreads();
   if (tid < kGroupBlocks) {
-    const uint32_t b = block_sum[tid];
-    const uint32_t incl = wave_incl_scan(b);
+    const S b = block_sum[tid];
+    S incl = b;
+    if constexpr (WIDE) {
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const S v = __shfl_up(incl, d, 64);
+        incl += tid >= d ? v : 0;
+      }
+    } else {
+      incl = wave_incl_scan(b);
+    }
     const int64_t block = static_cast<int64_t>(blockIdx.x) * kGroupBlocks + tid;
     if (block < n_blocks) sums[block] = incl - b;
     if (tid == kGroupBlocks - 1) groups[blockIdx.x] = incl;
@@ -2461,20 +2500,29 @@ void decode_streams(const lmc_tensor &cdf, const lmc_tensor &bs, const lmc_tenso
   const int64_t n_streams = L * C;
   const int64_t blocks = (n_streams + kDecLanes - 1) / kDecLanes;
   check(blocks < (int64_t(1) << 31), "too many streams");
-  StreamEnds ends = {nullptr, nullptr, nullptr, nullptr};
+  StreamEnds ends = {};
   if (sums == nullptr) {
     ends.prefix = static_cast<const int32_t *>(ln.data);
   } else {
     const int64_t groups = (blocks + kGroupBlocks - 1) / kGroupBlocks;
     need_device(*sums, "sums");
-    check(sums->dtype == LMC_I32 && numel(*sums) >= blocks + groups,
-          "sums must be int32 with an entry per block of 64 streams and per 64 blocks");
-    uint32_t *b = static_cast<uint32_t *>(sums->data);
+    check((sums->dtype == LMC_I32 || sums->dtype == LMC_I64) && numel(*sums) >= blocks + groups,
+          "sums must be int32 or int64 with an entry per block of 64 streams and per 64 blocks");
+    const dim3 sum_grid(static_cast<unsigned>(groups));
     ends.lens = static_cast<const int32_t *>(ln.data);
-    ends.sums = b;
-    ends.groups = b + blocks;
-    hipLaunchKernelGGL(length_sums_kernel, dim3(static_cast<unsigned>(groups)), dim3(kSumThreads), 0, stream,
-                       ends.lens, n_streams, blocks, b, b + blocks);
+    if (sums->dtype == LMC_I64) {
+      int64_t *b = static_cast<int64_t *>(sums->data);
+      ends.wide_sums = b;
+      ends.wide_groups = b + blocks;
+      hipLaunchKernelGGL(length_sums_kernel<int64_t>, sum_grid, dim3(kSumThreads), 0, stream, ends.lens, n_streams,
+                         blocks, b, b + blocks);
+    } else {
+      uint32_t *b = static_cast<uint32_t *>(sums->data);
+      ends.sums = b;
+      ends.groups = b + blocks;
+      hipLaunchKernelGGL(length_sums_kernel<uint32_t>, sum_grid, dim3(kSumThreads), 0, stream, ends.lens, n_streams,
+                         blocks, b, b + blocks);
+    }
     hip_check(hipGetLastError(), "length_sums_kernel launch");
   }
   const int16_t *rows = static_cast<const int16_t *>(cdf.data);

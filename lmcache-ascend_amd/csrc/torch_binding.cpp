@@ -273,7 +273,9 @@ at::Tensor cachegen_decode_chunk(const at::Tensor &cdf, const at::Tensor &stream
     throw std::runtime_error("cachegen_decode_chunk: cdf must be a GPU tensor [L, C, nbins + 1]");
   const int64_t L = cdf.size(0), C = cdf.size(1), blocks = (L * C + 63) / 64;
   at::Tensor out = at::empty({L, num_tokens, C}, cdf.options().dtype(at::kByte));
-  at::Tensor sums = at::empty({blocks + (blocks + 63) / 64}, cdf.options().dtype(at::kInt));
+  // (scratch: 32-bit sums hold places below 2 GiB)
+  at::Tensor sums = at::empty({blocks + (blocks + 63) / 64},
+                              cdf.options().dtype(streams.numel() >> 31 ? at::kLong : at::kInt));
   // The op needs an addressable buffer.
   const at::Tensor bytes = streams.numel() ? streams : at::zeros({1}, cdf.options().dtype(at::kByte));
   const lmc_tensor c = desc(cdf), b = desc(bytes), n = desc(lengths), t = desc(sums), o = desc(out);

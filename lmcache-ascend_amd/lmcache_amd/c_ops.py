@@ -444,7 +444,9 @@ def cachegen_decode_chunk(cdf, bytestreams, lengths, num_tokens: int):
         bytestreams = torch.zeros(1, dtype=torch.uint8, device=dev)
     out = torch.empty((L, int(num_tokens), C), dtype=torch.uint8, device=dev)
     blocks = (L * C + 63) // 64
-    sums = torch.empty(blocks + (blocks + 63) // 64, dtype=torch.int32, device=dev)
+    # Scratch: 32-bit sums hold places below 2 GiB.
+    sums = torch.empty(blocks + (blocks + 63) // 64, device=dev,
+                       dtype=torch.int64 if bytestreams.numel() >> 31 else torch.int32)
     c, b, n, t, o = _desc(cdf), _desc(bytestreams), _desc(lengths), _desc(sums), _desc(out)
     _run(_L.lmc_cachegen_decode(_ref(c), _ref(b), _ref(n), _ref(t), _ref(o), _stream(dev.index)))
     return out

@@ -20,8 +20,8 @@ own (upstream's integers are outside the reference tree).
 CacheGen chunks.  Upstream LMCache's CacheGen serde wraps the codec ops in
 `CacheGenGPUEncoderOutput` (call sites tests/v1/test_cachegen_kernels.py:
 299-335): the CDF, the encoded streams concatenated in (layer, channel)
-order, and per-stream lengths, which `decode_fast_prefsum` takes as
-inclusive prefix sums.  `CacheGenChunk` holds the same pieces and
+order, and per-stream lengths (`decode_fast_prefsum` takes their inclusive
+prefix sums).  `CacheGenChunk` holds the same pieces and
 serializes them with an explicit little-endian layout (a magic, a version,
 the dimensions, then the raw arrays), so loading bytes runs no code from
 them.  Byte-level interop with upstream's serialized objects is not claimed:
@@ -209,22 +209,11 @@ def encode_chunk(symbols: torch.Tensor, n_bins: int, max_stream_bytes: int = 0) 
 
 
 def decode_chunk(chunk: CacheGenChunk) -> torch.Tensor:
-    """Decodes a chunk on the GPU into uint8 symbols [L, T, C]: the streams'
-    places come from their lengths on the way (cachegen_decode_chunk), or,
-    for lengths of another type or layout, from their prefix sums
-    (decode_fast_prefsum)."""
+    """Decodes a chunk on the GPU into uint8 symbols [L, T, C]; the streams'
+    places come from their lengths (cachegen_decode_chunk)."""
     L, T, C = chunk.shape
     dev = chunk.cdf.device
     if dev.type != "cuda":
         raise ValueError("decode_chunk takes a chunk on the GPU (CacheGenChunk.to)")
-    n = chunk.lengths
-    if n.dtype == torch.int32 and n.device == dev and n.is_contiguous() and n.numel() == L * C:
-        return c_ops.cachegen_decode_chunk(chunk.cdf, chunk.streams.to(dev), n, T)
-    prefix = torch.cumsum(chunk.lengths.to(torch.int64).view(-1), 0).to(torch.int32).view(L, C)
-    streams = chunk.streams.to(dev)
-    if streams.numel() == 0:  # the op needs an addressable buffer
-        streams = torch.zeros(1, dtype=torch.uint8, device=dev)
-    # decode_fast_prefsum writes all T symbols of every stream.
-    out = torch.empty((L, T, C), dtype=torch.uint8, device=dev)
-    c_ops.decode_fast_prefsum(chunk.cdf, streams, prefix, out)
-    return out
+    lengths = chunk.lengths.to(torch.int32).contiguous()
+    return c_ops.cachegen_decode_chunk(chunk.cdf, chunk.streams.to(dev), lengths, T)

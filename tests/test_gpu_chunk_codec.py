@@ -120,7 +120,7 @@ def test_encode_rows_vs_oracle(L, T, C, nb, chunk, kind):
 
 
 # Streams' places from their lengths (groups of 4096 streams, a last block of
-# 32) and from prefix sums, which lengths of another type take.
+# 32), lengths of another type, and 64-bit sums.
 @pytest.mark.parametrize("L,T,C", [(1, 4, 32), (64, 3, 64), (43, 5, 96), (64, 2, 160), (3, 300, 1056)])
 def test_decode_chunk_by_lengths(F, L, T, C):
     sym = _symbols(L, T, C, 16, L + T + C)
@@ -128,6 +128,38 @@ def test_decode_chunk_by_lengths(F, L, T, C):
     other = F.CacheGenChunk(chunk.cdf, chunk.lengths.to(torch.int64), chunk.streams, T)
     assert np.array_equal(F.decode_chunk(chunk).cpu().numpy(), sym)
     assert np.array_equal(F.decode_chunk(other).cpu().numpy(), sym)
+    from lmcache_amd import _lib, c_ops
+
+    blocks = (L * C + 63) // 64
+    sums = torch.full((blocks + (blocks + 63) // 64,), -1, dtype=torch.int64, device=DEV)
+    out = torch.full((L, T, C), 255, dtype=torch.uint8, device=DEV)
+    d = [c_ops._desc(t) for t in (chunk.cdf, chunk.streams, chunk.lengths, sums, out)]
+    _lib.raise_for(_lib.load().lmc_cachegen_decode(*map(c_ops._ref, d), c_ops._stream(0)))
+    assert np.array_equal(out.cpu().numpy(), sym)
+
+
+# Byte buffers past 2 GiB (64 streams of 40 MB or 64 MiB, their codes in front,
+# the last in another group of 4096 streams than most): every decoder takes
+# places in 64 bits.
+@pytest.mark.parametrize("T", [16, 300, 400, 1025])
+@pytest.mark.parametrize("step", [40_000_000, 1 << 26])
+def test_decode_chunk_past_2gib(F, T, step):
+    L, C = 65, 64
+    sym = _symbols(L, T, C, 16, T)
+    chunk = F.encode_chunk(torch.from_numpy(sym).to(DEV), 16)
+    lens = chunk.lengths.view(-1).tolist()
+    wide = list(range(60)) + list(range(L * C - 4, L * C))  # the streams that are spread out
+    held = chunk.lengths.view(-1).clone()
+    held[wide] = step
+    at = np.concatenate([[0], np.cumsum(held.cpu().numpy().astype(np.int64))])
+    src = np.concatenate([[0], np.cumsum(np.asarray(lens, np.int64))])
+    big = torch.zeros(int(at[-1]), dtype=torch.uint8, device=DEV)
+    for s in wide:
+        big[at[s]:at[s] + lens[s]] = chunk.streams[src[s]:src[s + 1]]
+    big[at[60]:at[L * C - 4]] = chunk.streams[src[60]:src[L * C - 4]]
+    assert big.numel() > 2**31
+    got = F.decode_chunk(F.CacheGenChunk(chunk.cdf, held.view(L, C), big, T))
+    assert np.array_equal(got.cpu().numpy(), sym)
 
 
 # A stream that reaches almost to 2 GiB.
