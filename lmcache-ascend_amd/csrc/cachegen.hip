@@ -1533,6 +1533,58 @@ __device__ __forceinline__ void decode_one_wave(uint8_t *lds, const int16_t *__r
   }
 }
 
+// The streams of a block from their regions, for tables without escapes.
+// Four tokens per group (cgdec::GroupCursor): the four table entries go
+// through the LDS transpose and the symbols of the resulting word are
+// extracted at once, (word >> 3) & 0x1F1F1F1F; each word is stored one
+// group late, so no group waits for its own transpose read.  The
+// transpose writes, that store and the transposing read sit between the
+// group's codes, each under a table read (the cursor's scheduling
+// barriers keep them there).  Measured on MI355X (symbol loop, shader
+// cycles per symbol, s_memtime stamps): 128-133 with the refilled lane
+// cursor (its chain four VALU instructions and the table read, the
+// refill on it every fourth code) -> 112 with this cursor -> 102 with
+// the transpose spread between the codes -> 100 with the window's
+// permutations one code later.  The chain alone, timed in isolation,
+// takes 72 cycles; the rest is issue of the other instructions under
+// it and LDS traffic.
+__device__ __forceinline__ void decode_groups(const cgdec::ByteTables &tb, const uint32_t *region, uint32_t region_at,
+                                              uint32_t off, uint32_t len, uint8_t *obuf, const DecBlock::Quad &quad,
+                                              int T, int C, int lane) {
+  uint32_t *odst = quad.dst;
+  const int64_t step4 = static_cast<int64_t>(C);  // in dwords: 4 tokens of C bytes
+  cgdec::GroupCursor gc;
+  gc.start(tb, region, region_at, off, len);
+  int t = 0;
+  uint32_t word = 0;
+  for (; t + 4 <= T; t += 4) {
+    const uint32_t e0 = gc.step0(tb);
+    const uint32_t e1 = gc.step1(tb);
+    obuf[lane] = static_cast<uint8_t>(e0);
+    if (t > 0) {
+      cg_st(odst, (word >> 3) & 0x1F1F1F1Fu);
+      odst += step4;
+    }
+    const uint32_t e2 = gc.step2(tb);
+    obuf[kDecLanes + lane] = static_cast<uint8_t>(e1);
+    const uint32_t e3 = gc.step3(tb);
+    obuf[2 * kDecLanes + lane] = static_cast<uint8_t>(e2);
+    obuf[3 * kDecLanes + lane] = static_cast<uint8_t>(e3);
+    wave_sync();
+    word = reinterpret_cast<const uint32_t *>(obuf)[quad.at];
+    wave_sync();
+  }
+  if (t > 0) {
+    cg_st(odst, (word >> 3) & 0x1F1F1F1Fu);
+    odst += step4;
+  }
+  if (t < T) {
+    for (int i = 0; t + i < T; ++i) obuf[i * kDecLanes + lane] = static_cast<uint8_t>(gc.single(tb));
+    wave_sync();
+    if ((quad.at >> 4) < T - t) cg_st(odst, reinterpret_cast<const uint32_t *>(obuf)[quad.at]);
+  }
+}
+
 // Byte tables with per-lane stream regions (cgdec::LaneRegion): each lane
 // stages the 16-byte aligned chunks holding its own stream into its own LDS
 // region and zeroes what lies past the stream's end, so the cursors read
@@ -1630,50 +1682,8 @@ __device__ __forceinline__ bool decode_one_wave_lanes(uint8_t *lds, const int16_
   uint32_t *odst = quad.dst;
   const int64_t step4 = static_cast<int64_t>(C);  // in dwords: 4 tokens of C bytes
   if (!__any(tb.escapes)) {
-    // Four tokens per group (cgdec::GroupCursor): the four table entries go
-    // through the LDS transpose and the symbols of the resulting word are
-    // extracted at once, (word >> 3) & 0x1F1F1F1F; each word is stored one
-    // group late, so no group waits for its own transpose read.  The
-    // transpose writes, that store and the transposing read sit between the
-    // group's codes, each under a table read (the cursor's scheduling
-    // barriers keep them there).  Measured on MI355X (symbol loop, shader
-    // cycles per symbol, s_memtime stamps): 128-133 with the refilled lane
-    // cursor (its chain four VALU instructions and the table read, the
-    // refill on it every fourth code) -> 112 with this cursor -> 102 with
-    // the transpose spread between the codes -> 100 with the window's
-    // permutations one code later.  The chain alone, timed in isolation,
-    // takes 72 cycles; the rest is issue of the other instructions under
-    // it and LDS traffic.
-    cgdec::GroupCursor gc;
-    gc.start(tb, reg32, lds_at + static_cast<uint32_t>(region - lds), static_cast<uint32_t>(s_lo - a0), len);
-    int t = 0;
-    uint32_t word = 0;
-    for (; t + 4 <= T; t += 4) {
-      const uint32_t e0 = gc.step0(tb);
-      const uint32_t e1 = gc.step1(tb);
-      obuf[lane] = static_cast<uint8_t>(e0);
-      if (t > 0) {
-        cg_st(odst, (word >> 3) & 0x1F1F1F1Fu);
-        odst += step4;
-      }
-      const uint32_t e2 = gc.step2(tb);
-      obuf[kDecLanes + lane] = static_cast<uint8_t>(e1);
-      const uint32_t e3 = gc.step3(tb);
-      obuf[2 * kDecLanes + lane] = static_cast<uint8_t>(e2);
-      obuf[3 * kDecLanes + lane] = static_cast<uint8_t>(e3);
-      wave_sync();
-      word = reinterpret_cast<const uint32_t *>(obuf)[quad.at];
-      wave_sync();
-    }
-    if (t > 0) {
-      cg_st(odst, (word >> 3) & 0x1F1F1F1Fu);
-      odst += step4;
-    }
-    if (t < T) {
-      for (int i = 0; t + i < T; ++i) obuf[i * kDecLanes + lane] = static_cast<uint8_t>(gc.single(tb));
-      wave_sync();
-      if ((quad.at >> 4) < T - t) cg_st(odst, reinterpret_cast<const uint32_t *>(obuf)[quad.at]);
-    }
+    decode_groups(tb, reg32, lds_at + static_cast<uint32_t>(region - lds), static_cast<uint32_t>(s_lo - a0), len, obuf, quad,
+                  T, C, lane);
   } else {
     tb.finish();
     cgdec::LaneCursor cur;
@@ -1747,6 +1757,7 @@ struct LaneChunks {
     end = off + len;
     n_ch = len ? (end + 15u) >> 4 : 0u;
   }
+  __device__ __forceinline__ uint32_t len() const { return end - off; }
   __device__ __forceinline__ chunk16 load(uint32_t k) const {
     chunk16 v = {0u, 0u, 0u, 0u};
     if (k < n_ch) v = reinterpret_cast<global_chunk16 *>(a0)[k];
@@ -1866,6 +1877,84 @@ __device__ __forceinline__ void decode_serial(cgdec::LongTables &tb, bool irregu
   }
 }
 
+// The lanes' regions (cgdec::LaneRegion), one after the other in `room` bytes
+// of LDS: the lane's chunks and the sealed room behind them.  `at` is where
+// the lane's starts, `most` the largest number of chunks of a lane.
+struct Regions {
+  uint32_t at, total, most, room;
+  __device__ __forceinline__ Regions(const LaneChunks &ch, uint32_t lds_room, int lane) : room(lds_room) {
+    // At most one byte more than there is, so that the sum cannot wrap.
+    const uint32_t own = min(16u * ch.n_ch + cgdec::LaneRegion::kRoom, room + 1u);
+    uint32_t incl = own;
+    most = ch.n_ch;
+#pragma unroll
+    for (int d = 1; d < kDecLanes; d <<= 1) {
+      const uint32_t v = __shfl_up(incl, d, kDecLanes);
+      incl += lane >= d ? v : 0u;
+      const uint32_t m = __shfl_xor(most, d, kDecLanes);
+      most = m > most ? m : most;
+    }
+    total = __shfl(incl, kDecLanes - 1, kDecLanes);
+    at = incl - own;
+  }
+  __device__ __forceinline__ bool fit() const { return total <= room; }
+};
+
+// A lane's chunks into its region: the first N (cv) are in registers, the
+// others are loaded N at a time.  Seals the region.
+template <int N>
+__device__ __forceinline__ void fill_region(const LaneChunks &ch, uint32_t most, chunk16 (&cv)[N], uint8_t *region) {
+#pragma unroll
+  for (int u = 0; u < N; ++u)
+    if (static_cast<uint32_t>(u) < ch.n_ch) reinterpret_cast<chunk16 *>(region)[u] = cv[u];
+  for (uint32_t k0 = N; k0 < most; k0 += N) {
+#pragma unroll
+    for (int u = 0; u < N; ++u)
+      if (k0 + u < ch.n_ch) cv[u] = reinterpret_cast<global_chunk16 *>(ch.a0)[k0 + u];
+#pragma unroll
+    for (int u = 0; u < N; ++u)
+      if (k0 + u < ch.n_ch) reinterpret_cast<chunk16 *>(region)[k0 + u] = cv[u];
+  }
+  cgdec::LaneRegion::seal(reinterpret_cast<uint32_t *>(region), ch.off, ch.len());
+}
+
+// Whether the staged rows (16-byte chunks) may be of short codes only: bases
+// at multiples of 256 and lengths of at most 8.
+__device__ __forceinline__ bool short_rows(const uint8_t *rows, int nrow, int lane) {
+  uint32_t off = 0;
+#pragma unroll
+  for (int k = 0; k < kRowChunks; ++k) {
+    const int j = k * kDecLanes + lane;
+    const chunk16 v = reinterpret_cast<const chunk16 *>(rows)[j < nrow ? j : nrow - 1];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t x = i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w;  // two entries
+      off |= (x & 0x00F000F0u) | (((x & 0x000F000Fu) + 0x00070007u) & 0x00100010u);
+    }
+  }
+  return !__any(off != 0);
+}
+
+// A block of short codes: the byte table holds them all and the streams lie in
+// regions behind it (from kShortRegions on, over the second table and the
+// rings), so that a code takes the group cursor's 100 cycles in place of the
+// two tables' 210.  short_table builds the table (false if it has escapes
+// after all), decode_short decodes; cv holds the lanes' first chunks.
+constexpr int kShortRegions = cgdec::ByteTables::kBytes;
+__device__ __forceinline__ bool short_table(cgdec::ByteTables &tb, uint8_t *obuf, int lane) {
+  tb.build(obuf + lane);
+  return !__any(tb.escapes);
+}
+__device__ __forceinline__ void decode_short(const cgdec::ByteTables &tb, const DecBlock &bk, const LaneChunks &ch,
+                                             chunk16 (&cv)[kFirstChunks], const Regions &regions, uint8_t *lds,
+                                             uint32_t lds_at, uint8_t *obuf, int T, int C, int lane,
+                                             uint8_t *__restrict__ out) {
+  const uint32_t at = kShortRegions + regions.at;
+  fill_region(ch, regions.most, cv, lds + at);
+  decode_groups(tb, reinterpret_cast<const uint32_t *>(lds + at), lds_at + at, ch.off, ch.len(), obuf,
+                bk.quad(out, T, C, lane), T, C, lane);
+}
+
 constexpr int kLongObuf = kLongRing + static_cast<int>(cgdec::RingCursor::kBytes) * kDecLanes;
 constexpr int kLongRows = kLongObuf + kObufBytes;
 // The staged rows, at up to 15 bytes past a 16-byte boundary; a table build
@@ -1904,6 +1993,19 @@ __global__ void __launch_bounds__(kDecLanes)
                  (lane < bk.cnt ? lane : 0) * (nb + 1);
   tb.one.nb = nb;
   uint8_t *obuf = lds + kLongObuf;
+  if (short_rows(lds + kLongRows, nrow, lane)) {
+    const Regions regions(ch, kLongObuf - kShortRegions, lane);
+    chunk16 cv[kFirstChunks];
+#pragma unroll
+    for (uint32_t u = 0; u < kFirstChunks; ++u) cv[u] = ch.load(u);
+    if (regions.fit()) {
+      if (short_table(tb.one, obuf, lane)) {
+        decode_short(tb.one, bk, ch, cv, regions, lds, lds_at, obuf, T, C, lane, out);
+        return;
+      }
+      tb.clear();
+    }
+  }
   tb.build(lds_at + static_cast<uint32_t>(kLongObuf + lane));
   decode_serial(tb, __any(tb.irregular) != 0, bk, ch, lds, lds_at, kLongRing, obuf, T, C, lane, out);
 }
@@ -1944,6 +2046,7 @@ constexpr int kSplitSteps = 16;  // steps per epoch: at most 16 bytes of the rin
 constexpr int kSplitRing = static_cast<int>(cgdec::StepCursor::Ring::kBytes) * kDecLanes;
 constexpr int kSplitBuf = kLongRing + kSplit * kSplitRing;
 constexpr int kSplitFlags = 16;
+constexpr int kSplitShort = 15;
 // Its LDS holds chunks of up to kSplitMaxT tokens, and leaves one block on a
 // CU where decode_long_kernel has three, so it takes launches that leave it a
 // CU per block, and chunks long enough for the codes decoded before each
@@ -1988,7 +2091,7 @@ __global__ void __launch_bounds__(kSplitThreads)
   uint32_t *counts = stops + kSplit * kDecLanes;
   // [0]: an irregular row; [1 + 2 r], [2 + 2 r]: round r left a wave off its
   // boundaries, a wave out of room (each written in its own round, so that
-  // every wave reads the same).
+  // every wave reads the same); [kSplitShort]: decode_short takes the block.
   uint32_t *flags = counts + kSplit * kDecLanes;
   DecBlock bk;
   bk.init(cdf, nbytes, ends, n_streams, C, nb, lane);
@@ -2025,10 +2128,10 @@ __global__ void __launch_bounds__(kSplitThreads)
   // markers put in by wave 0.
   cgdec::LongTables tb;
   tb.bind(lds, lane, lds_at);
+  const int nrow = static_cast<int>((bk.R1 - bk.r_lo + 15) >> 4);
   {
     uint32_t *t32 = reinterpret_cast<uint32_t *>(tb.one.tab);
     for (int d = wave * (128 / kSplit); d < (wave + 1) * (128 / kSplit); ++d) t32[d * kDecLanes] = 0;
-    const int nrow = static_cast<int>((bk.R1 - bk.r_lo + 15) >> 4);
     for (int j = static_cast<int>(threadIdx.x); j < nrow; j += kSplitThreads)
       reinterpret_cast<chunk16 *>(lds + plan.rows_off)[j] = reinterpret_cast<global_chunk16 *>(bk.r_lo)[j];
     if (threadIdx.x < kSplitFlags) flags[threadIdx.x] = 0;
@@ -2038,6 +2141,22 @@ __global__ void __launch_bounds__(kSplitThreads)
                  (live ? lane : 0) * (nb + 1);
   tb.one.nb = nb;
   const uint32_t dummy = lds_at + static_cast<uint32_t>(kSplitBuf + lane);  // scratch for skipped writes
+  // Short codes: one wave takes the block (every wave finds the same).  The
+  // regions reach up to the transpose, at the end of the buffers; wave 0's
+  // first chunks are the streams'.
+  if (short_rows(lds + plan.rows_off, nrow, lane)) {
+    const int obuf_off = plan.meta_off - kObufBytes;
+    const Regions regions(ch, static_cast<uint32_t>(obuf_off - kShortRegions), lane);
+    if (regions.fit()) {
+      if (wave == 0 && short_table(tb.one, lds + obuf_off, lane) && lane == 0) flags[kSplitShort] = 1;
+      __syncthreads();
+      if (flags[kSplitShort] != 0) {
+        if (wave == 0) decode_short(tb.one, bk, ch, cv, regions, lds, lds_at, lds + obuf_off, T, C, lane, out);
+        return;
+      }
+      if (wave == 0) tb.clear();
+    }
+  }
   if (wave == 0) {
     tb.mark(dummy);
     if (__any(tb.irregular) && lane == 0) flags[0] = 1;

@@ -98,6 +98,42 @@ def test_decode_long_foreign_rows(kind, T):
     assert np.array_equal(out.cpu().numpy(), want)
 
 
+# Rows of codes of up to 8 bits, which the group cursor takes from per-lane
+# regions: calculated codes, rows with a symbol 31 of length 8 (its entry reads
+# as an escape) and random rows of that form (zero-length codes, gaps, wraps),
+# streams that fit the regions and that do not, one kernel and the other, and
+# blocks of 32 streams.
+@pytest.mark.parametrize("L,C", [(3, 96), (16, 1056)])
+@pytest.mark.parametrize("T", [257, 384, 385, 1000, 1024, 1025])
+@pytest.mark.parametrize("kind,nb", [("codes", 32), ("codes", 17), ("last", 32), ("random", 32), ("random", 9)])
+def test_decode_long_short_codes(kind, nb, T, L, C):
+    from lmcache_amd import c_ops
+
+    if L * C > 4096 and (T > 400 or kind == "last"):
+        pytest.skip("the small launch covers it")
+    rng = np.random.default_rng(T + nb + L)
+    if kind == "codes":
+        sym = rng.integers(0, min(nb, 12), size=(L, 200, C)).astype(np.uint8)
+        cdf = oc.calculate_cdf(sym, nb)
+    elif kind == "last":
+        row = np.concatenate([[1], (0x8000 + 256 * np.arange(31)) | 8, [0]]).astype(np.uint16)
+        cdf = np.broadcast_to(row.view(np.int16), (L, C, nb + 1)).copy()
+    else:
+        base = rng.integers(0, 256, size=(L, C, nb + 1)) << 8
+        base[:, ::2] = np.sort(base[:, ::2], axis=2)
+        base[:, 1::7] = 0
+        cdf = (base | rng.integers(0, 9, size=base.shape)).astype(np.uint16).view(np.int16)
+    for most in (T // 2, 3000) if L * C < 4096 else (T // 2,):
+        lens = rng.integers(0, most, size=(L, C)).astype(np.int32)
+        prefix = np.cumsum(lens.reshape(-1), dtype=np.int64).astype(np.int32).reshape(L, C)
+        stream = rng.integers(0, 256, size=int(prefix[-1, -1]), dtype=np.uint8)
+        want = oc.decode(cdf, stream, prefix, T)
+        out = torch.full((L, T, C), 255, dtype=torch.uint8, device=DEV)
+        c_ops.decode_fast_prefsum(torch.from_numpy(cdf).to(DEV), torch.from_numpy(stream).to(DEV),
+                                  torch.from_numpy(prefix).to(DEV), out)
+        assert np.array_equal(out.cpu().numpy(), want)
+
+
 # Rows of encode_fast_new: every byte below min(chunk, length) and no other,
 # at row strides off the dword, rows that cut their streams, and one to four
 # 256-token pieces (a stream's last dword carried from one to the next).
