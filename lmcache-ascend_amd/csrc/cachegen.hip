@@ -1777,21 +1777,44 @@ struct LaneChunks {
   }
 };
 
+// The 4 x 64 transpose in registers: each lane holds the low bytes of its
+// stream's four tokens; dword `at` of the transpose (DecBlock::Quad) is byte
+// at / 16 of the lanes 4 * (at % 16) .. + 3.  send() issues the exchanges,
+// take() puts the dword together.
+struct LaneTranspose {
+  int from;            // 4 x the first of the four lanes
+  uint32_t sel;        // byte permutation: a byte of either operand
+  uint32_t r0, r1, r2, r3;
+  __device__ __forceinline__ explicit LaneTranspose(int at)
+      : from(16 * (at & 15)), sel(0x0C0C0400u + 0x0101u * static_cast<uint32_t>(at >> 4)), r0(0), r1(0), r2(0), r3(0) {}
+  __device__ __forceinline__ void send(uint32_t e0, uint32_t e1, uint32_t e2, uint32_t e3) {
+    const uint32_t lo = cgdec::byte_perm(e1, e0, 0x0C0C0400u), hi = cgdec::byte_perm(e3, e2, 0x0C0C0400u);
+    const int four = static_cast<int>(lo | (hi << 16));
+    r0 = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(from, four));
+    r1 = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(from + 4, four));
+    r2 = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(from + 8, four));
+    r3 = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(from + 12, four));
+  }
+  __device__ __forceinline__ uint32_t take() const {
+    return cgdec::byte_perm(r1, r0, sel) | (cgdec::byte_perm(r3, r2, sel) << 16);
+  }
+};
+
 // One wave decodes a block's streams, one lane per stream.  It takes kEpoch
 // tokens at a time: the chunks that refill the ring over an epoch are loaded
 // at its start and stored at its end, so nothing waits for them.  A ring
-// holds 256 bytes; kEpoch codes of at most 16 bits take 64 of them, and an
-// epoch loads as many chunks as there is room for, up to 64 bytes, so at
-// least 100 bytes lie ahead of the cursor at the start of every epoch.
+// holds 128 bytes; kEpoch codes of at most 16 bits take 32 of them, and an
+// epoch loads as many chunks as there is room for, up to 32 bytes, so at
+// least 80 bytes lie ahead of the cursor at the start of every epoch.
 // `irregular`: some row of the block takes the binary search.
 // Bound by the serial chain of each stream, about 210 cycles a code.
-constexpr int kEpoch = 32;
-constexpr int kEpochChunks = 4;  // 16-byte chunks per lane and epoch
+constexpr int kEpoch = 16;
+constexpr int kEpochChunks = 2;  // 16-byte chunks per lane and epoch
 constexpr int kFirstChunks = 8;
 
 __device__ __forceinline__ void decode_serial(cgdec::LongTables &tb, bool irregular, const DecBlock &bk,
                                               const LaneChunks &ch, uint8_t *lds, uint32_t lds_at, int ring_off,
-                                              uint8_t *obuf, int T, int C, int lane, uint8_t *__restrict__ out) {
+                                              int T, int C, int lane, uint8_t *__restrict__ out) {
   uint32_t *ring = reinterpret_cast<uint32_t *>(lds + ring_off) + lane;
   constexpr uint32_t kRingDw = cgdec::RingCursor::kBytes / 4;
   {
@@ -1826,24 +1849,18 @@ __device__ __forceinline__ void decode_serial(cgdec::LongTables &tb, bool irregu
   if (!irregular) {
     cgdec::PairCursor cur;
     cur.start(tb, column, 8u * ch.off);
-    uint32_t word = 0;
+    LaneTranspose tr(quad.at);
     // Four tokens; each transposed word is stored one group late, as in
-    // decode_one_wave_lanes.
+    // decode_groups.
     auto group = [&](bool store_prev) {
       uint32_t e0, e1, e2, e3;
       cur.pair(tb, e0, e1);
-      obuf[lane] = static_cast<uint8_t>(e0);
-      obuf[kDecLanes + lane] = static_cast<uint8_t>(e1);
       if (store_prev) {
-        cg_st(odst, (word >> 3) & 0x1F1F1F1Fu);
+        cg_st(odst, (tr.take() >> 3) & 0x1F1F1F1Fu);
         odst += step4;
       }
       cur.pair(tb, e2, e3);
-      obuf[2 * kDecLanes + lane] = static_cast<uint8_t>(e2);
-      obuf[3 * kDecLanes + lane] = static_cast<uint8_t>(e3);
-      wave_sync();
-      word = reinterpret_cast<const uint32_t *>(obuf)[quad.at];
-      wave_sync();
+      tr.send(e0, e1, e2, e3);
     };
     constexpr int kGroups = kEpoch / 4;
     int g = 0;
@@ -1854,24 +1871,25 @@ __device__ __forceinline__ void decode_serial(cgdec::LongTables &tb, bool irregu
       store_epoch();
     }
     for (; g < groups; ++g) group(g > 0);
-    if ((quad.at >> 4) < T - 4 * (groups - 1)) cg_st(odst, (word >> 3) & 0x1F1F1F1Fu);
+    if ((quad.at >> 4) < T - 4 * (groups - 1)) cg_st(odst, (tr.take() >> 3) & 0x1F1F1F1Fu);
   } else {
     tb.one.finish();
+    LaneTranspose tr(quad.at);
     cgdec::RingCursor cur;
     cur.start(column, 8u * ch.off);
     for (int g = 0; g < groups; ++g) {
       if (g % (kEpoch / 4) == 0) load_epoch(cur.q);
+      uint32_t sym[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        int sym, n;
-        tb.search(cur.hi() >> 16, sym, n);
-        obuf[i * kDecLanes + lane] = static_cast<uint8_t>(sym);
+        int x, n;
+        tb.search(cur.hi() >> 16, x, n);
+        sym[i] = static_cast<uint32_t>(x);
         cur.advance(static_cast<uint32_t>(n));
       }
-      wave_sync();
-      if ((quad.at >> 4) < T - 4 * g) cg_st(odst, reinterpret_cast<const uint32_t *>(obuf)[quad.at]);
+      tr.send(sym[0], sym[1], sym[2], sym[3]);
+      if ((quad.at >> 4) < T - 4 * g) cg_st(odst, tr.take());
       odst += step4;
-      wave_sync();
       if (g % (kEpoch / 4) == kEpoch / 4 - 1) store_epoch();
     }
   }
@@ -1955,11 +1973,17 @@ __device__ __forceinline__ void decode_short(const cgdec::ByteTables &tb, const 
                 bk.quad(out, T, C, lane), T, C, lane);
 }
 
-constexpr int kLongObuf = kLongRing + static_cast<int>(cgdec::RingCursor::kBytes) * kDecLanes;
-constexpr int kLongRows = kLongObuf + kObufBytes;
 // The staged rows, at up to 15 bytes past a 16-byte boundary; a table build
 // reads kMaxBins entries of a row whatever nb is.
 constexpr int rows_lds_bytes(int nb) { return ((nb + 1) * kDecLanes * 2 + 32 + 2 * cgdec::ByteTables::kMaxBins + 15) & ~15; }
+
+// LDS of decode_long_kernel: the two tables and the rings, 40 KiB, so that
+// four blocks fit a CU.  The staged rows lie in the rings' place until the
+// tables are built (an irregular block's then move to the tables' place), and
+// scratch for skipped writes, or the transpose of short codes, at its end.
+constexpr int kLongObuf = kDecLds - kObufBytes;
+static_assert(kLongRing + static_cast<int>(cgdec::RingCursor::kBytes) * kDecLanes == kDecLds, "rings end the LDS");
+static_assert(kLongRing + rows_lds_bytes(cgdec::ByteTables::kMaxBins) <= kLongObuf, "rows lie before the scratch");
 
 // Any length, one wave per block (56 planes x 1000 tokens x 256 channels: 100
 // us, where the shared-window kernel took 1307 us: the streams of a block
@@ -1983,17 +2007,13 @@ __global__ void __launch_bounds__(kDecLanes)
   cgdec::LongTables tb;
   tb.bind(lds, lane, lds_at);
   tb.clear();
-  store_chunks<false>(lds + kLongRows, nrow, 0, lane, rv);
-  for (int j0 = kDecLanes * kRowChunks; j0 < nrow; j0 += kDecLanes * kRowChunks) {
-    load_chunks(bk.r_lo, nrow, j0, lane, rv);
-    store_chunks<false>(lds + kLongRows, nrow, j0, lane, rv);
-  }
+  store_chunks<false>(lds + kLongRing, nrow, 0, lane, rv);  // (all of them: n_bins <= 32)
   wave_sync();
-  tb.one.row.r = reinterpret_cast<const int16_t *>(lds + kLongRows + (bk.R0 - bk.r_lo)) +
-                 (lane < bk.cnt ? lane : 0) * (nb + 1);
+  const int row_at = static_cast<int>(bk.R0 - bk.r_lo) + (lane < bk.cnt ? lane : 0) * (nb + 1) * 2;
+  tb.one.row.r = reinterpret_cast<const int16_t *>(lds + kLongRing + row_at);
   tb.one.nb = nb;
   uint8_t *obuf = lds + kLongObuf;
-  if (short_rows(lds + kLongRows, nrow, lane)) {
+  if (short_rows(lds + kLongRing, nrow, lane)) {
     const Regions regions(ch, kLongObuf - kShortRegions, lane);
     chunk16 cv[kFirstChunks];
 #pragma unroll
@@ -2007,7 +2027,17 @@ __global__ void __launch_bounds__(kDecLanes)
     }
   }
   tb.build(lds_at + static_cast<uint32_t>(kLongObuf + lane));
-  decode_serial(tb, __any(tb.irregular) != 0, bk, ch, lds, lds_at, kLongRing, obuf, T, C, lane, out);
+  const bool irregular = __any(tb.irregular) != 0;
+  if (irregular) {  // the search reads the rows, not the tables
+#pragma unroll
+    for (int k = 0; k < kRowChunks; ++k) {
+      const int j = k * kDecLanes + lane;
+      if (j < nrow) reinterpret_cast<chunk16 *>(lds)[j] = reinterpret_cast<const chunk16 *>(lds + kLongRing)[j];
+    }
+    tb.one.row.r = reinterpret_cast<const int16_t *>(lds + row_at);
+    wave_sync();
+  }
+  decode_serial(tb, irregular, bk, ch, lds, lds_at, kLongRing, T, C, lane, out);
 }
 
 // Split decode: four waves per block of 64 streams, each taking a quarter of
@@ -2048,7 +2078,7 @@ constexpr int kSplitBuf = kLongRing + kSplit * kSplitRing;
 constexpr int kSplitFlags = 16;
 constexpr int kSplitShort = 15;
 // Its LDS holds chunks of up to kSplitMaxT tokens, and leaves one block on a
-// CU where decode_long_kernel has three, so it takes launches that leave it a
+// CU where decode_long_kernel has four, so it takes launches that leave it a
 // CU per block, and chunks long enough for the codes decoded before each
 // quarter's own not to matter (300 tokens, 96 blocks: 42 us against 39 for one
 // wave per block; 512 tokens, 512 blocks: 90 against 60; 1000 tokens, 224
@@ -2237,7 +2267,7 @@ __global__ void __launch_bounds__(kSplitThreads)
   if (one_wave) {
     __syncthreads();
     if (wave == 0)
-      decode_serial(tb, flags[0] != 0, bk, ch, lds, lds_at, kLongRing, lds + kSplitBuf, T, C, lane, out);
+      decode_serial(tb, flags[0] != 0, bk, ch, lds, lds_at, kLongRing, T, C, lane, out);
     return;
   }
   // The tokens, four at a time, a quarter of them per wave; lane = stream.  A
@@ -2657,8 +2687,7 @@ void decode_streams(const lmc_tensor &cdf, const lmc_tensor &bs, const lmc_tenso
       hipLaunchKernelGGL(decode_split_kernel, grid, dim3(kSplitThreads), plan.lds, stream, rows, bytes, numel(bs), ends,
                          (int)T, (int)C, (int)nb, out, n_streams, plan);
     } else {
-      hipLaunchKernelGGL(decode_long_kernel, grid, dim3(kDecLanes),
-                         kLongRows + rows_lds_bytes(static_cast<int>(nb)), stream, rows, bytes, numel(bs), ends,
+      hipLaunchKernelGGL(decode_long_kernel, grid, dim3(kDecLanes), kDecLds, stream, rows, bytes, numel(bs), ends,
                          (int)T, (int)C, (int)nb, out, n_streams);
     }
   } else {

@@ -763,7 +763,7 @@ template <uint32_t BYTES> struct RingCursorT {
     ahead = raw(q);
   }
 };
-using RingCursor = RingCursorT<256>;
+using RingCursor = RingCursorT<128>;
 
 // Two codes per step of LongTables over a ring.  The chain from one code to
 // the next is the two tables' reads (issued together), the select of the

@@ -6,7 +6,7 @@
 //
 // Every row's tables are built as the kernel builds them and its streams are
 // decoded as the kernel decodes them: pairs of codes from the tables, or the
-// binary search where the row is irregular, the ring refilled every 32 codes
+// binary search where the row is irregular, the ring refilled every 16 codes
 // with chunks whose bytes past the stream's end are zero.  LDS is one buffer
 // of the kernel's size (built with AddressSanitizer).
 //
@@ -150,16 +150,16 @@ int main(int argc, char **argv) {
       const uint32_t column = kRingAt + 4u * static_cast<uint32_t>(lane);
       auto refill = [&](uint32_t q_before) {
         uint32_t room = (RingCursor::kBytes - (16 * filled - q_before)) >> 4;
-        room = room < 4 ? room : 4;
+        room = room < 2 ? room : 2;
         for (uint32_t u = 0; u < room; ++u) put(filled + u);
         filled += room;
       };
       if (!tb.irregular) {
         PairCursor cur;
         cur.start(tb, column, 8 * off);
-        for (int t0 = 0; t0 < T; t0 += 32) {
+        for (int t0 = 0; t0 < T; t0 += 16) {
           const uint32_t q0 = cur.ring.q;
-          for (int t = t0; t < t0 + 32 && t < T; t += 2) {
+          for (int t = t0; t < t0 + 16 && t < T; t += 2) {
             uint32_t e0, e1;
             cur.pair(tb, e0, e1);
             got[t] = static_cast<uint8_t>((e0 >> 3) & 31u);
@@ -170,9 +170,9 @@ int main(int argc, char **argv) {
       } else {
         RingCursor cur;
         cur.start(column, 8 * off);
-        for (int t = 0; t < T; t += 32) {
+        for (int t = 0; t < T; t += 16) {
           const uint32_t q0 = cur.q;
-          for (int i = t; i < t + 32 && i < T; ++i) {
+          for (int i = t; i < t + 16 && i < T; ++i) {
             int s, n;
             tb.search(cur.hi() >> 16, s, n);
             got[i] = static_cast<uint8_t>(s);

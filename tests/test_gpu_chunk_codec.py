@@ -103,14 +103,11 @@ def test_decode_long_foreign_rows(kind, T):
 # as an escape) and random rows of that form (zero-length codes, gaps, wraps),
 # streams that fit the regions and that do not, one kernel and the other, and
 # blocks of 32 streams.
-@pytest.mark.parametrize("L,C", [(3, 96), (16, 1056)])
-@pytest.mark.parametrize("T", [257, 384, 385, 1000, 1024, 1025])
+@pytest.mark.parametrize("L,C,T", [(3, 96, T) for T in (257, 384, 385, 1000, 1024, 1025)] + [(16, 1056, 257), (16, 1056, 385)])
 @pytest.mark.parametrize("kind,nb", [("codes", 32), ("codes", 17), ("last", 32), ("random", 32), ("random", 9)])
-def test_decode_long_short_codes(kind, nb, T, L, C):
+def test_decode_long_short_codes(kind, nb, L, C, T):
     from lmcache_amd import c_ops
 
-    if L * C > 4096 and (T > 400 or kind == "last"):
-        pytest.skip("the small launch covers it")
     rng = np.random.default_rng(T + nb + L)
     if kind == "codes":
         sym = rng.integers(0, min(nb, 12), size=(L, 200, C)).astype(np.uint8)
