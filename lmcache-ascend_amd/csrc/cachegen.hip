@@ -211,8 +211,13 @@ __device__ __forceinline__ void gw_lengths(uint32_t *hist, uint32_t *lists, uint
 
 // kBins: register capacity for per-symbol values (nb <= kBins); kExact: nb
 // == kBins, so every per-symbol bound is a constant.
+// The code (55 KB for 32 bins) starts on a 64 KB page, so that where it and
+// the encoder behind it lie does not follow from the size of the code before
+// them: encode_chunk, which runs both back to back, takes 43.4 to 44.9 us at
+// this place and at most others, but 46.5 at some (64 x 256 x 1024 symbols;
+// this kernel by itself takes the same time anywhere).
 template <int kBins, bool kExact>
-__global__ void __launch_bounds__(kCdfThreads)
+__attribute__((aligned(65536))) __global__ void __launch_bounds__(kCdfThreads)
     cdf_tile_kernel(const uint8_t *__restrict__ in, int T, int C, int nb,
                     int16_t *__restrict__ out, int64_t n_streams, int vec_tile,
                     int32_t *__restrict__ lens, int64_t *__restrict__ sums, int64_t cap) {
