@@ -1349,16 +1349,41 @@ __device__ __forceinline__ void decode_stream(const Tab &tb, int T, int C,
   }
 }
 
+// The channels of a layer, and division by them with a multiplication (Granlund
+// and Montgomery, "Division by invariant integers using multiplication",
+// figure 4.1): a decode block finds its first stream's layer before its first
+// load, and the compiler's division is about 40 dependent instructions there
+// (64 planes x 256 tokens x 512 channels 18.2 -> 17.7 us; the encoder and
+// calculate_cdf gain nothing from it).
+struct Channels {
+  int n;
+  uint32_t mul, sh1, sh2;
+  explicit Channels(int64_t c) : n(static_cast<int>(c)) {
+    int l = 0;
+    while ((int64_t(1) << l) < c) ++l;
+    mul = static_cast<uint32_t>(((uint64_t((int64_t(1) << l) - c) << 32) / static_cast<uint64_t>(c)) + 1);
+    sh1 = l < 1 ? l : 1;
+    sh2 = l > 1 ? l - 1 : 0;
+  }
+  __device__ __forceinline__ uint32_t divide(uint32_t x) const {
+    const uint32_t t = __umulhi(x, mul);
+    return (t + ((x - t) >> sh1)) >> sh2;
+  }
+  __device__ __forceinline__ int64_t layer_of(int64_t s) const {
+    return s < (int64_t(1) << 32) ? divide(static_cast<uint32_t>(s)) : s / n;
+  }
+};
+
 // Layer and channel of a stream `k` streams after (l, c); streams are
 // numbered over the layers, channels fastest.
 struct StreamAt {
   int64_t l;
   int c;
 };
-__device__ __forceinline__ StreamAt stream_at(int64_t l, int c, uint32_t k, int C) {
+__device__ __forceinline__ StreamAt stream_at(int64_t l, int c, uint32_t k, const Channels &chans) {
   const uint32_t x = static_cast<uint32_t>(c) + k;
-  const uint32_t up = x / static_cast<uint32_t>(C);
-  return {l + up, static_cast<int>(x - up * static_cast<uint32_t>(C))};
+  const uint32_t up = chans.divide(x);
+  return {l + up, static_cast<int>(x - up * static_cast<uint32_t>(chans.n))};
 }
 
 // Inclusive prefix sum of 32-bit values over the 64 lanes of a wave, in 64
@@ -1392,10 +1417,10 @@ struct DecBlock {
   uintptr_t R0, R1, r_lo;
 
   __device__ __forceinline__ void init(const int16_t *cdf, int64_t nbytes, const StreamEnds &ends,
-                                       int64_t n_streams, int C, int nb, int lane) {
+                                       int64_t n_streams, const Channels &chans, int nb, int lane) {
     s0 = static_cast<int64_t>(blockIdx.x) * kDecLanes;
-    l0 = s0 < (int64_t(1) << 32) ? static_cast<uint32_t>(s0) / static_cast<uint32_t>(C) : s0 / C;
-    c0 = static_cast<int>(s0 - l0 * C);
+    l0 = chans.layer_of(s0);
+    c0 = static_cast<int>(s0 - l0 * chans.n);
     cnt = n_streams - s0 < kDecLanes ? static_cast<int>(n_streams - s0) : kDecLanes;
     const int64_t stream = s0 + (lane < cnt ? lane : 0);
     auto clampb = [&](int64_t x) { return x < 0 ? 0 : (x > nbytes ? nbytes : x); };
@@ -1450,10 +1475,10 @@ struct DecBlock {
     int at;
     uint32_t *dst;
   };
-  __device__ __forceinline__ Quad quad(uint8_t *out, int T, int C, int lane) const {
+  __device__ __forceinline__ Quad quad(uint8_t *out, int T, const Channels &chans, int lane) const {
     const int at = cnt == kDecLanes ? lane : lane & 0x37;
-    const StreamAt a = stream_at(l0, c0, 4u * static_cast<uint32_t>(at & 15), C);
-    return {at, reinterpret_cast<uint32_t *>(out + (a.l * T + (at >> 4)) * C + a.c)};
+    const StreamAt a = stream_at(l0, c0, 4u * static_cast<uint32_t>(at & 15), chans);
+    return {at, reinterpret_cast<uint32_t *>(out + (a.l * T + (at >> 4)) * chans.n + a.c)};
   }
 
   // 16-byte chunks of the window staged from a_lo: the block's bytes from
@@ -1473,15 +1498,16 @@ struct DecBlock {
 template <class Tab>
 __device__ __forceinline__ void decode_one_wave(uint8_t *lds, const int16_t *__restrict__ cdf,
                                                 const uint8_t *__restrict__ bytes, int64_t nbytes,
-                                                const StreamEnds ends, int T, int C,
+                                                const StreamEnds ends, int T, const Channels &chans,
                                                 int nb, uint8_t *__restrict__ out, int64_t n_streams,
                                                 int lane) {
+  const int C = chans.n;
   constexpr int kRowsOff = Tab::kBytes + kObufBytes;
   const int rows_cap = ((nb + 1) * kDecLanes * 2 + 32 + 15) & ~15;
   const int win_off = kRowsOff + rows_cap;
   const int win_cap = (kDecLds - win_off) & ~15;
   DecBlock bk;
-  bk.init(cdf, nbytes, ends, n_streams, C, nb, lane);
+  bk.init(cdf, nbytes, ends, n_streams, chans, nb, lane);
   const int live = lane < bk.cnt;
   const uintptr_t base0 = reinterpret_cast<uintptr_t>(bytes);
   const uintptr_t a_lo = (base0 + bk.B0) & ~uintptr_t(15);
@@ -1523,13 +1549,13 @@ __device__ __forceinline__ void decode_one_wave(uint8_t *lds, const int16_t *__r
   if (!live) return;
   const uint32_t *win = reinterpret_cast<const uint32_t *>(lds + win_off);
   if (fast) {
-    uint32_t *odst = bk.quad(out, T, C, lane).dst;  // a full block
+    uint32_t *odst = bk.quad(out, T, chans, lane).dst;  // a full block
     decode_fast(tb, T, C, win, static_cast<uint32_t>(a_hi - a_lo) - 4,
                 static_cast<uint32_t>(lo - a_lo), static_cast<uint32_t>(hi - a_lo),
                 lds + Tab::kBytes, odst);
   } else {
     tb.finish();
-    const StreamAt at = stream_at(bk.l0, bk.c0, static_cast<uint32_t>(lane), C);
+    const StreamAt at = stream_at(bk.l0, bk.c0, static_cast<uint32_t>(lane), chans);
     uint8_t *o = out + at.l * T * C + at.c;
     if (in_win)
       decode_stream<true>(tb, T, C, bytes, win, a_lo, a_hi, lo, hi, o);
@@ -1602,10 +1628,11 @@ __device__ __forceinline__ void decode_groups(const cgdec::ByteTables &tb, const
 // nothing, for any other block, which then takes decode_one_wave.
 __device__ __forceinline__ bool decode_one_wave_lanes(uint8_t *lds, const int16_t *__restrict__ cdf,
                                                       const uint8_t *__restrict__ bytes, int64_t nbytes,
-                                                      const StreamEnds ends, int T, int C, int nb,
+                                                      const StreamEnds ends, int T, const Channels &chans, int nb,
                                                       uint8_t *__restrict__ out, int64_t n_streams,
                                                       int lane) {
   using Tab = cgdec::ByteTables;
+  const int C = chans.n;
   constexpr int kRowsOff = Tab::kBytes + kObufBytes;
   constexpr int kLaneBatch = 8;  // 16-byte chunks per lane and load batch
   const int rows_cap = ((nb + 1) * kDecLanes * 2 + 32 + 15) & ~15;
@@ -1616,7 +1643,7 @@ __device__ __forceinline__ bool decode_one_wave_lanes(uint8_t *lds, const int16_
   const uint32_t lds_at =
       static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t *)lds));
   DecBlock bk;
-  bk.init(cdf, nbytes, ends, n_streams, C, nb, lane);
+  bk.init(cdf, nbytes, ends, n_streams, chans, nb, lane);
   if ((reinterpret_cast<uintptr_t>(out) & 3) != 0 || (C & 3) != 0 || (lds_at & (Tab::kBytes - 1)) != 0)
     return false;
   // The rows' loads depend on the block alone: issued before the stream
@@ -1683,7 +1710,7 @@ __device__ __forceinline__ bool decode_one_wave_lanes(uint8_t *lds, const int16_
   uint32_t *reg32 = reinterpret_cast<uint32_t *>(region);
   cgdec::LaneRegion::seal(reg32, static_cast<uint32_t>(s_lo - a0), len);
   uint8_t *obuf = lds + Tab::kBytes;
-  const DecBlock::Quad quad = bk.quad(out, T, C, lane);
+  const DecBlock::Quad quad = bk.quad(out, T, chans, lane);
   uint32_t *odst = quad.dst;
   const int64_t step4 = static_cast<int64_t>(C);  // in dwords: 4 tokens of C bytes
   if (!__any(tb.escapes)) {
@@ -1722,16 +1749,16 @@ template <class Tab>
 __global__ void __launch_bounds__(kDecLanes)
     decode_kernel(const int16_t *__restrict__ cdf,
                   const uint8_t *__restrict__ bytes, int64_t nbytes,
-                  const StreamEnds ends, int T, int C, int nb,
+                  const StreamEnds ends, int T, const Channels chans, int nb,
                   uint8_t *__restrict__ out, int64_t n_streams) {
   extern __shared__ uint32_t lds_words[];
   uint8_t *lds = reinterpret_cast<uint8_t *>(lds_words);
   const int lane = static_cast<int>(threadIdx.x);
   if constexpr (std::is_same<Tab, cgdec::ByteTables>::value) {
-    if (LMC_DEC_LANES && decode_one_wave_lanes(lds, cdf, bytes, nbytes, ends, T, C, nb, out, n_streams, lane))
+    if (LMC_DEC_LANES && decode_one_wave_lanes(lds, cdf, bytes, nbytes, ends, T, chans, nb, out, n_streams, lane))
       return;
   }
-  decode_one_wave<Tab>(lds, cdf, bytes, nbytes, ends, T, C, nb, out, n_streams, lane);
+  decode_one_wave<Tab>(lds, cdf, bytes, nbytes, ends, T, chans, nb, out, n_streams, lane);
 }
 
 // Decode of chunks of more than kLaneMaxT tokens (n_bins <= 32).  Codes are
@@ -1819,7 +1846,8 @@ constexpr int kFirstChunks = 8;
 
 __device__ __forceinline__ void decode_serial(cgdec::LongTables &tb, bool irregular, const DecBlock &bk,
                                               const LaneChunks &ch, uint8_t *lds, uint32_t lds_at, int ring_off,
-                                              int T, int C, int lane, uint8_t *__restrict__ out) {
+                                              int T, const Channels &chans, int lane, uint8_t *__restrict__ out) {
+  const int C = chans.n;
   uint32_t *ring = reinterpret_cast<uint32_t *>(lds + ring_off) + lane;
   constexpr uint32_t kRingDw = cgdec::RingCursor::kBytes / 4;
   {
@@ -1831,7 +1859,7 @@ __device__ __forceinline__ void decode_serial(cgdec::LongTables &tb, bool irregu
   }
   uint32_t filled = kFirstChunks;  // chunks in the ring or before it
   wave_sync();
-  const DecBlock::Quad quad = bk.quad(out, T, C, lane);
+  const DecBlock::Quad quad = bk.quad(out, T, chans, lane);
   uint32_t *odst = quad.dst;
   const int64_t step4 = static_cast<int64_t>(C);  // in dwords: 4 tokens of C bytes
   const int groups = (T + 3) / 4;
@@ -1970,12 +1998,12 @@ __device__ __forceinline__ bool short_table(cgdec::ByteTables &tb, uint8_t *obuf
 }
 __device__ __forceinline__ void decode_short(const cgdec::ByteTables &tb, const DecBlock &bk, const LaneChunks &ch,
                                              chunk16 (&cv)[kFirstChunks], const Regions &regions, uint8_t *lds,
-                                             uint32_t lds_at, uint8_t *obuf, int T, int C, int lane,
+                                             uint32_t lds_at, uint8_t *obuf, int T, const Channels &chans, int lane,
                                              uint8_t *__restrict__ out) {
   const uint32_t at = kShortRegions + regions.at;
   fill_region(ch, regions.most, cv, lds + at);
   decode_groups(tb, reinterpret_cast<const uint32_t *>(lds + at), lds_at + at, ch.off, ch.len(), obuf,
-                bk.quad(out, T, C, lane), T, C, lane);
+                bk.quad(out, T, chans, lane), T, chans.n, lane);
 }
 
 // The staged rows, at up to 15 bytes past a 16-byte boundary; a table build
@@ -1996,7 +2024,7 @@ static_assert(kLongRing + rows_lds_bytes(cgdec::ByteTables::kMaxBins) <= kLongOb
 // binary search per symbol after the table's first long code).
 __global__ void __launch_bounds__(kDecLanes)
     decode_long_kernel(const int16_t *__restrict__ cdf, const uint8_t *__restrict__ bytes, int64_t nbytes,
-                       const StreamEnds ends, int T, int C, int nb, uint8_t *__restrict__ out,
+                       const StreamEnds ends, int T, const Channels chans, int nb, uint8_t *__restrict__ out,
                        int64_t n_streams) {
   extern __shared__ uint32_t lds_words[];
   uint8_t *lds = reinterpret_cast<uint8_t *>(lds_words);
@@ -2004,7 +2032,7 @@ __global__ void __launch_bounds__(kDecLanes)
       static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t *)lds));
   const int lane = static_cast<int>(threadIdx.x);
   DecBlock bk;
-  bk.init(cdf, nbytes, ends, n_streams, C, nb, lane);
+  bk.init(cdf, nbytes, ends, n_streams, chans, nb, lane);
   const int nrow = static_cast<int>((bk.R1 - bk.r_lo + 15) >> 4);
   chunk16 rv[kRowChunks];
   load_chunks(bk.r_lo, nrow, 0, lane, rv);
@@ -2025,7 +2053,7 @@ __global__ void __launch_bounds__(kDecLanes)
     for (uint32_t u = 0; u < kFirstChunks; ++u) cv[u] = ch.load(u);
     if (regions.fit()) {
       if (short_table(tb.one, obuf, lane)) {
-        decode_short(tb.one, bk, ch, cv, regions, lds, lds_at, obuf, T, C, lane, out);
+        decode_short(tb.one, bk, ch, cv, regions, lds, lds_at, obuf, T, chans, lane, out);
         return;
       }
       tb.clear();
@@ -2042,7 +2070,7 @@ __global__ void __launch_bounds__(kDecLanes)
     tb.one.row.r = reinterpret_cast<const int16_t *>(lds + row_at);
     wave_sync();
   }
-  decode_serial(tb, irregular, bk, ch, lds, lds_at, kLongRing, T, C, lane, out);
+  decode_serial(tb, irregular, bk, ch, lds, lds_at, kLongRing, T, chans, lane, out);
 }
 
 // Split decode: four waves per block of 64 streams, each taking a quarter of
@@ -2113,8 +2141,10 @@ __device__ __forceinline__ int split_base(const SplitPlan &p, int w) {
 
 __global__ void __launch_bounds__(kSplitThreads)
     decode_split_kernel(const int16_t *__restrict__ cdf, const uint8_t *__restrict__ bytes, int64_t nbytes,
-                        const StreamEnds ends, int T, int C, int nb, uint8_t *__restrict__ out, int64_t n_streams,
+                        const StreamEnds ends, int T, const Channels chans, int nb, uint8_t *__restrict__ out,
+                        int64_t n_streams,
                         const SplitPlan plan) {
+  const int C = chans.n;
   extern __shared__ uint32_t lds_words[];
   uint8_t *lds = reinterpret_cast<uint8_t *>(lds_words);
   const uint32_t lds_at =
@@ -2129,7 +2159,7 @@ __global__ void __launch_bounds__(kSplitThreads)
   // every wave reads the same); [kSplitShort]: decode_short takes the block.
   uint32_t *flags = counts + kSplit * kDecLanes;
   DecBlock bk;
-  bk.init(cdf, nbytes, ends, n_streams, C, nb, lane);
+  bk.init(cdf, nbytes, ends, n_streams, chans, nb, lane);
   const bool live = lane < bk.cnt;
   const LaneChunks ch(bytes, bk);
   // T codes of at most 12 bits end before 2 T bytes: longer streams are of no
@@ -2186,7 +2216,7 @@ __global__ void __launch_bounds__(kSplitThreads)
       if (wave == 0 && short_table(tb.one, lds + obuf_off, lane) && lane == 0) flags[kSplitShort] = 1;
       __syncthreads();
       if (flags[kSplitShort] != 0) {
-        if (wave == 0) decode_short(tb.one, bk, ch, cv, regions, lds, lds_at, lds + obuf_off, T, C, lane, out);
+        if (wave == 0) decode_short(tb.one, bk, ch, cv, regions, lds, lds_at, lds + obuf_off, T, chans, lane, out);
         return;
       }
       if (wave == 0) tb.clear();
@@ -2272,7 +2302,7 @@ __global__ void __launch_bounds__(kSplitThreads)
   if (one_wave) {
     __syncthreads();
     if (wave == 0)
-      decode_serial(tb, flags[0] != 0, bk, ch, lds, lds_at, kLongRing, T, C, lane, out);
+      decode_serial(tb, flags[0] != 0, bk, ch, lds, lds_at, kLongRing, T, chans, lane, out);
     return;
   }
   // The tokens, four at a time, a quarter of them per wave; lane = stream.  A
@@ -2306,7 +2336,7 @@ __global__ void __launch_bounds__(kSplitThreads)
     for (int k = 0; k + 1 < kSplit; ++k) e = t >= until[k] ? until[k + 1] : e;
     return e;
   };
-  const DecBlock::Quad quad = bk.quad(out, T, C, lane);
+  const DecBlock::Quad quad = bk.quad(out, T, chans, lane);
   uint8_t *obuf = lds + kLongRing + wave * kSplitRing;
   const int groups = (T + 3) / 4, share = (groups + kSplit - 1) / kSplit;
   const int g1 = (wave + 1) * share < groups ? (wave + 1) * share : groups;
@@ -2690,14 +2720,14 @@ void decode_streams(const lmc_tensor &cdf, const lmc_tensor &bs, const lmc_tenso
                                     hipFuncAttributeMaxDynamicSharedMemorySize, plan.lds),
                 "decode LDS size");
       hipLaunchKernelGGL(decode_split_kernel, grid, dim3(kSplitThreads), plan.lds, stream, rows, bytes, numel(bs), ends,
-                         (int)T, (int)C, (int)nb, out, n_streams, plan);
+                         (int)T, Channels(C), (int)nb, out, n_streams, plan);
     } else {
       hipLaunchKernelGGL(decode_long_kernel, grid, dim3(kDecLanes), kDecLds, stream, rows, bytes, numel(bs), ends,
-                         (int)T, (int)C, (int)nb, out, n_streams);
+                         (int)T, Channels(C), (int)nb, out, n_streams);
     }
   } else {
     hipLaunchKernelGGL(nb <= cgdec::ByteTables::kMaxBins ? decode_kernel<cgdec::ByteTables> : decode_kernel<DecTables>,
-                       grid, dim3(kDecLanes), kDecLds, stream, rows, bytes, numel(bs), ends, (int)T, (int)C, (int)nb,
+                       grid, dim3(kDecLanes), kDecLds, stream, rows, bytes, numel(bs), ends, (int)T, Channels(C), (int)nb,
                        out, n_streams);
   }
   hip_check(hipGetLastError(), "decode_kernel launch");
