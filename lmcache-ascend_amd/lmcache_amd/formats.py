@@ -215,5 +215,7 @@ def decode_chunk(chunk: CacheGenChunk) -> torch.Tensor:
     dev = chunk.cdf.device
     if dev.type != "cuda":
         raise ValueError("decode_chunk takes a chunk on the GPU (CacheGenChunk.to)")
-    lengths = chunk.lengths.to(torch.int32).contiguous()
+    lengths = chunk.lengths
+    if lengths.dtype != torch.int32 or not lengths.is_contiguous():
+        lengths = lengths.to(torch.int32).contiguous()
     return c_ops.cachegen_decode_chunk(chunk.cdf, chunk.streams.to(dev), lengths, T)
