@@ -221,8 +221,9 @@ def test_decode_stream_of_almost_2gib(F, T):
 # Chunks whose quarters do not follow from where they should lie: streams of
 # one-bit and of long codes at either end (a quarter outgrows its buffer, or
 # starts well off its place), codes of one length (a decoder started between
-# boundaries stays between them), and the kernel's largest chunk and one past.
-@pytest.mark.parametrize("T", [257, 401, 1000, 1024, 1025])
+# boundaries stays between them), the kernel's smallest and largest chunks, and
+# chunks below and above that the one-wave decoder takes.
+@pytest.mark.parametrize("T", [257, 385, 401, 1000, 1024, 1025])
 def test_long_chunk_uneven_streams(F, T):
     L, C, nb = 3, 96, 32
     rng = np.random.default_rng(T)
@@ -236,6 +237,19 @@ def test_long_chunk_uneven_streams(F, T):
     sym[2, :, 5] = 7
     chunk = F.encode_chunk(torch.from_numpy(sym).to(DEV), nb)
     assert np.array_equal(F.decode_chunk(chunk).cpu().numpy(), sym)
+
+
+# The lines between the decoders of long chunks: 384 and 385 tokens, 1024 and
+# 1025, and launches of 256 and 257 blocks of 64 streams, with long codes
+# (skewed symbols) and short ones.
+@pytest.mark.parametrize("kind", ["normal", "skewed"])
+@pytest.mark.parametrize("L,T,C", [
+    (1, 384, 96), (1, 385, 96), (1, 1024, 96), (1, 1025, 96), (1, 400, 256 * 64), (1, 400, 257 * 64), (257, 401, 64),
+])
+def test_long_decoder_lines(F, L, T, C, kind):
+    sym = np.minimum(_symbols(L, T, C, 32, T + L, kind), 31).astype(np.uint8)
+    chunk = F.encode_chunk(torch.from_numpy(sym).to(DEV), 32)
+    assert torch.equal(F.decode_chunk(chunk), torch.from_numpy(sym).to(DEV))
 
 
 # decode_chunk enqueues kernels only, also for the long chunk whose kernel
