@@ -2376,12 +2376,16 @@ __global__ void __launch_bounds__(kSplitThreads)
 // b * stride of `blocks`, to off[b] of `out`.  A thread takes 16-byte aligned
 // pieces of the destination, each from five source dwords shifted together;
 // the bytes of the pieces shared with the blocks before and after are stored
-// one by one.  Every source dword read holds a byte of the block.  Measured
-// on MI355X (64 planes x 256 tokens x 1024 channels, 7.3 MB): 6.0 us.  (A
-// copy stream by stream from rows of their own, each with such edges: 11.5
-// us.  A boolean mask over the rows and a masked select: about 330 us.)
+// one by one.  Every source dword read holds a byte of the block.  A block is
+// shared by kPackParts workgroups: medians of the kernel behind the encoder
+// (MI355X, traced), one workgroup a block -> two -> four: 64 planes x 256
+// tokens x 1024 channels (1024 blocks, 6.9 MB) 6.6 -> 5.4 -> 5.4 us, 128
+// planes 9.4 -> 8.2 -> 8.5, 56 x 256 x 256 (224 blocks, 1.5 MB) 4.8 -> 3.8 ->
+// 3.7, 56 x 1000 x 256 (224 blocks, 5.7 MB) 9.0 -> 6.2 -> 5.0, 64 x 1000 x
+// 1024 (26 MB) 13.2 -> 12.6 -> 10.8.  (A copy stream by stream from rows of
+// their own, each with such edges, took twice as long, and a boolean mask over
+// the rows with a masked select about 330 us.)
 constexpr int kPackThreads = 256;
-constexpr int64_t kPackWhole = 1024;
 constexpr unsigned kPackParts = 4;
 __global__ void __launch_bounds__(kPackThreads)
     pack_blocks_kernel(const uint8_t *__restrict__ blocks, int64_t stride, const int64_t *__restrict__ off,
@@ -2818,10 +2822,7 @@ int lmc_cachegen_pack_rows(const lmc_tensor *rows_t, const lmc_tensor *offsets_t
     if (n_streams == 0 || numel(o) == 0) return;
     check(blocks < (int64_t(1) << 31), "too many streams");
     DeviceGuard guard(rows.device);
-    // Few blocks of long streams are shared by kPackParts workgroups each (224
-    // of 28 KB for 56 x 1000 x 256 symbols: 10 -> 7 us).
-    const unsigned parts = blocks < kPackWhole ? kPackParts : 1;
-    hipLaunchKernelGGL(pack_blocks_kernel, dim3(static_cast<unsigned>(blocks), parts), dim3(kPackThreads), 0,
+    hipLaunchKernelGGL(pack_blocks_kernel, dim3(static_cast<unsigned>(blocks), kPackParts), dim3(kPackThreads), 0,
                        static_cast<hipStream_t>(stream), static_cast<const uint8_t *>(rows.data),
                        kEncLanes * rows.sizes[2], static_cast<const int64_t *>(off.data),
                        static_cast<uint8_t *>(o.data), numel(o));
