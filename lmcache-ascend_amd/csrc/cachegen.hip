@@ -587,7 +587,7 @@ __attribute__((aligned(65536))) __global__ void __launch_bounds__(kCdfThreads)
 //           other forms have four (kRows' work in it: 22.2 us against 16.6).
 //
 // Measured on MI355X, 64 planes x 256 tokens x 1024 channels (32 bins in the
-// first 10 planes, 16 in the others): kRows 16.9 us, kImage 12.3 us; 56
+// first 10 planes, 16 in the others): kRows 16.9 us, kImage 12.3 to 13.0; 56
 // planes x 1000 tokens x 256 channels, kLong 22 us, against 128 us for a lane
 // per stream walking all its tokens.
 enum class EncMode { kRows, kImage, kLong };
@@ -1989,7 +1989,8 @@ __device__ __forceinline__ bool short_rows(const uint8_t *rows, int nrow, int la
 // A block of short codes: the byte table holds them all and the streams lie in
 // regions behind it (from kShortRegions on, over the second table and the
 // rings), so that a code takes the group cursor's 100 cycles in place of the
-// two tables' 210.  short_table builds the table (false if it has escapes
+// two tables' 210 (decode_fast_prefsum of 512 blocks of 300 tokens over four
+// symbols 39 -> 22 us, of 224 blocks of 700 over 16 56 -> 37).  short_table builds the table (false if it has escapes
 // after all), decode_short decodes; cv holds the lanes' first chunks.
 constexpr int kShortRegions = cgdec::ByteTables::kBytes;
 __device__ __forceinline__ bool short_table(cgdec::ByteTables &tb, uint8_t *obuf, int lane) {
@@ -2011,7 +2012,8 @@ __device__ __forceinline__ void decode_short(const cgdec::ByteTables &tb, const 
 constexpr int rows_lds_bytes(int nb) { return ((nb + 1) * kDecLanes * 2 + 32 + 2 * cgdec::ByteTables::kMaxBins + 15) & ~15; }
 
 // LDS of decode_long_kernel: the two tables and the rings, 40 KiB, so that
-// four blocks fit a CU.  The staged rows lie in the rings' place until the
+// four blocks fit a CU (1024 blocks of 300 tokens: 41 us, and 77 with the three
+// that 53 KiB left; fewer than 769 the same).  The staged rows lie in the rings' place until the
 // tables are built (an irregular block's then move to the tables' place), and
 // scratch for skipped writes, or the transpose of short codes, at its end.
 constexpr int kLongObuf = kDecLds - kObufBytes;
@@ -2516,8 +2518,8 @@ private:
 // streams, four lengths per thread.  A decode block adds the groups before
 // its own to its block's sum, which for 65536 streams is one load per lane
 // and one wave sum, so the prefix sums of the streams are never written.
-// Measured on MI355X (65536 streams): 3.0 us and the decode kernel behind it
-// 20.7 us, against four launches of about 17 us for prefix sums in 64 bits
+// Traced on MI355X (65536 streams): 3.9 to 4.7 us and the decode kernel behind
+// it 20.3 us, against four launches of about 17 us for prefix sums in 64 bits
 // (widening, scan, narrowing) and 24.4 us for the decode kernel reading them;
 // decode_chunk 35.9 -> 22.4 us.
 // S: uint32_t, or int64_t for buffers of 2 GiB and more (negative lengths

@@ -66,13 +66,18 @@ typedef __attribute__((address_space(1))) u32x4 GlobalU32x4;
 // (agent) scope, which writes through the XCD's L2 instead of leaving the
 // line dirty there, so the kernel's end-of-launch L2 write-back has nothing
 // left to flush; without it (and for narrower vectors) the store carries the
-// streaming hint.  Which is faster depends on the kernel (MI355X): in
-// back-to-back calls the row and group kernels are 1-8% faster with streaming
-// stores up to 2 GB a call (32 layers x 256 tokens x 1024 columns 12.6 / 13.2
-// us against 13.1 / 13.7, store / retrieve), although a kernel that runs alone
-// is up to 10% faster written through; the tile kernel's stores to memory
-// objects are faster written through (MLA-576 store 0.388 -> 0.402 ms with
-// streaming stores), and the direct kernels measure the same.
+// streaming hint.  Which is faster depends on the kernel (MI355X, store /
+// retrieve).  The row and group kernels are faster with streaming stores where
+// the buffers lie outside the 256 MB last-level cache, up to 2 GB a call: 24
+// buffer sets in turn, streaming against written through, 32 layers x 256
+// tokens x 1024 columns 12.9 / 13.8 against 13.3 / 13.5 us, x 768 10.9 / 11.1
+// against 11.3 / 12.1, x 512 8.4 / 8.6 against 8.9 / 9.1, and batches of 64 x
+// 8192 x 768 566 / 599 against 575 / 614 (kRowsWriteThrough has the row
+// kernel's sizes).  Inside the cache it is the other way round (three sets:
+// 12.2 / 13.1 against 10.7 / 10.8, 7.7 / 8.1 against 7.0 / 7.1); a request's
+// caches are not there.  The tile kernel's stores to memory objects are faster
+// written through (MLA-576 store 0.388 -> 0.402 ms with streaming stores), and
+// the direct kernels measure the same.
 template <typename T, bool NT, bool WT = true> __device__ __forceinline__ void st(T *p, T v) {
   if constexpr (NT && WT && LMC_KV_WT_STORES && sizeof(T) == 16)
     __builtin_amdgcn_global_store_b128((GlobalU32x4 *)(p),

@@ -98,12 +98,15 @@ using ChunkList = ChunkListT<kMaxChunks>;
 // The work of block b of n: blocks are dispatched round-robin over the 8
 // XCDs, and each XCD takes kXcdRun consecutive pieces of the work at a time
 // (512 KiB for the row kernel), so an XCD walks pages of its own instead of
-// every XCD touching every page.  Measured on MI355X, 1024-column rows, store
-// / retrieve: 64 layers x 8192 tokens with 128-token blocks 784 / 913 -> 669
-// / 674 us, 32 layers x 4096 tokens 190 / 222 -> 175 / 173, 32 x 2048 85 / 88
-// -> 84 / 86.  Runs of 16 and 256 pieces, or one run per XCD and object, lie
-// between (32 x 2048: 84 / 86, 84 / 88 and 87 / 89).  The tile kernel is up
-// to 7% slower with it and keeps the dispatch order.
+// every XCD touching every page.  Measured on MI355X, 1024-column rows of
+// 128-token blocks, store / retrieve, streaming stores with the dispatch order
+// -> with runs: 64 layers x 8192 tokens 707 / 880 -> 670 / 687 us, 64 x 5120
+// 430 / 417 -> 415 / 415, 64 x 4096 331 / 338 -> 329 / 334, 32 x 4096 165 / 167
+// -> 165 / 167, 32 x 2048 84.6 / 85.7 -> 83.6 / 84.9.  Runs of 16 and of 256
+// pieces lie within 3% of runs of 64 either way up to 8.6 GB a call, but 256
+// pieces cost small retrieves 5% (32 x 1024 44.4 -> 47.3, 32 x 2048 85.9 ->
+// 90.2).  The tile kernel is up to 7% slower with it and keeps the dispatch
+// order.
 constexpr int kXcdRun = 64;
 __device__ __forceinline__ int xcd_block(int b, int n) {
   const int r = b & (8 * kXcdRun - 1), first = b - r;
@@ -382,7 +385,8 @@ __global__ void __launch_bounds__(kThreads)
 // 4 x 256 x 64 4.9 / 5.6 -> 2.9 / 3.2; batches: 64 x 8192 x 512 360 / 419 ->
 // 354 / 370.  A wave whose lanes take the wave's vectors in address order,
 // with a slot per access, was slower (32 x 256 x 896 17.5 against 11.8), and
-// so were stores written through (32 x 256 x 512 8.9 / 9.1).
+// so were stores written through outside the last-level cache (32 x 256 x 512
+// 8.9 / 9.1).
 template <bool NT, int NC, int U, int R>
 __global__ void __launch_bounds__(kThreads)
     kv_rows_group(const CopyJob job, const ChunkListT<NC> chunks, int g_shift, int linear) {
@@ -642,11 +646,19 @@ ChunkListT<1> first_chunk(const ChunkList &cl) {
   return one;
 }
 
-// The row kernel's stores are written through in copies larger than this
-// and stream in smaller ones (store / retrieve, back-to-back calls over
-// several buffer sets, streaming -> written through): 4.3 GB 675 / 697 -> 668
-// / 673 us, 2.1 GB 328 / 333 -> 328 / 338, 1.1 GB 164 / 167 -> 164 / 171, 157
-// MB 27.7 / 28.4 -> 28.3 / 30.0.
+// The row kernel's stores are written through in copies larger than this and
+// stream in smaller ones.  The line lies where the stores' cost turns (bytes
+// read and written by a call; store / retrieve in us, back-to-back calls over
+// several buffer sets, streaming -> written through):
+//   0.27 GB   44.2 /  44.3 ->   44.5 /   45.1
+//   1.07 GB    165 /   167 ->    165 /    168
+//   2.15 GB    329 /   334 ->    329 /    335
+//   2.68 GB    415 /   415 ->    414 /    413
+//   3.22 GB    500 /   498 ->    490 /    503
+//   4.29 GB    670 /   687 ->    665 /    673
+//   5.37 GB    846 /   843 ->    849 /    819
+//   6.44 GB   1015 /   997 ->    996 /   1016
+//   8.59 GB   1355 /  1376 ->   1312 /   1330
 constexpr int64_t kRowsWriteThrough = int64_t(3) << 30;
 
 template <int VEC, int NC, bool SLOT32, bool TABLE>
@@ -714,9 +726,13 @@ constexpr int64_t kGroupLinear = 2048;
 // columns 2.7 against 3.3 us), and large ones with more in flight per wave
 // (32 x 8192 x 128 stored, 45.7 against 41.1).
 constexpr int64_t kGroupOneRow = 1024;
-// Long stores of rows of nine vector groups (576-column MLA rows in bf16)
-// stay with the tile kernel: 2.3 GB 395 against 420 us, 1.0 GB 180 against
-// 185; 0.58 GB is faster here (112 against 117 us).
+// Long stores of rows of nine vector groups (576-column MLA rows in bf16) stay
+// with the tile kernel, whose stores are written through.  Stores, tile kernel
+// against this one (bytes read and written; us): 0.13 GB 27.1 / 24.9, 0.25 GB
+// 49.4 / 47.3, 0.43 GB 76.3 / 74.3, 0.58 GB 108 / 105, 0.72 GB 126 / 125, 0.86
+// GB 145 / 149, 1.15 GB 190 / 193, 1.73 GB 291 / 305, 2.30 GB 381 / 394.
+// Retrieves are 3-9% faster here at all of these sizes but 0.58 GB (118 / 124)
+// and 1.73 GB (313 / 315).
 constexpr int64_t kGroupNineStore = int64_t(768) << 20;
 
 template <int U, int R>
