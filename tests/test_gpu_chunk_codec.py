@@ -120,14 +120,18 @@ def test_decode_long_short_codes(kind, nb, L, C, T):
         base[:, ::2] = np.sort(base[:, ::2], axis=2)
         base[:, 1::7] = 0
         cdf = (base | rng.integers(0, 9, size=base.shape)).astype(np.uint16).view(np.int16)
+    # Neither the rows nor the streams start on a 16-byte boundary.
+    held_cdf = torch.empty(cdf.size + 8, dtype=torch.int16, device=DEV)[T % 8:][:cdf.size].view(L, C, nb + 1)
+    held_cdf.copy_(torch.from_numpy(cdf))
     for most in (T // 2, 3000) if L * C < 4096 else (T // 2,):
         lens = rng.integers(0, most, size=(L, C)).astype(np.int32)
         prefix = np.cumsum(lens.reshape(-1), dtype=np.int64).astype(np.int32).reshape(L, C)
         stream = rng.integers(0, 256, size=int(prefix[-1, -1]), dtype=np.uint8)
         want = oc.decode(cdf, stream, prefix, T)
+        held = torch.full((stream.size + 16,), 0xFF, dtype=torch.uint8, device=DEV)[T % 13:][:stream.size]
+        held.copy_(torch.from_numpy(stream))
         out = torch.full((L, T, C), 255, dtype=torch.uint8, device=DEV)
-        c_ops.decode_fast_prefsum(torch.from_numpy(cdf).to(DEV), torch.from_numpy(stream).to(DEV),
-                                  torch.from_numpy(prefix).to(DEV), out)
+        c_ops.decode_fast_prefsum(held_cdf, held, torch.from_numpy(prefix).to(DEV), out)
         assert np.array_equal(out.cpu().numpy(), want)
 
 
